@@ -27,8 +27,9 @@ extern "C" {
 
 /* ---------------------------------------------------------------------------------------------
  * GEMV y = W x: W (m, n) row-major, x (n,) BF16, y (m,) FP32.  1 <= threads <= 1024, a power of
- * two (>= 32 for the coalesced kernels).  Vector (16-byte) loads are used when n is a multiple of
- * the vector width and W and x are 16-byte aligned; otherwise element loads with identical bits.
+ * two (>= 32 for the coalesced kernels).  The coalesced kernels use 16-byte loads for every n of
+ * at least one vector, at any address (no byte outside W and x is read); shorter rows, and the
+ * naive kernel's rows that are not whole aligned vectors, use element loads with identical bits.
  * -------------------------------------------------------------------------------------------*/
 
 /* BF16 weights, naive tree (contiguous chunk per lane, then neighbour pairs).
@@ -70,8 +71,8 @@ struct PckCheckBatch;
  * checked outputs must come from launches earlier on `stream` (not from this one).  rho, tau
  * and the verdicts are bit-identical to pck_blocked_check(ride); the checker workgroups are
  * separate wavefronts reading y from memory, so a check never trusts the launch it rides in.
- * At threads = 256 with vector loads the checks share the launch; otherwise they run as their
- * own launch just before the GEMVs.  No reference counterpart: it hides the checker launch's
+ * At threads = 256 with every n a multiple of the vector width and 16-byte aligned W and x the
+ * checks share the launch; otherwise they run as their own launch just before the GEMVs.  No reference counterpart: it hides the checker launch's
  * fixed latency behind the GEMV stream (the reference's check_many is a separate launch). */
 int pck_gemv_group_check(int weight_kind, const PckGemv* gemvs, int count, int threads,
                          const struct PckCheckBatch* ride, void* stream);
@@ -87,7 +88,7 @@ int pck_gemv_group_fp8_scaled(const PckGemv* gemvs, const float* const* scales,
                               float* const* scaled, int count, int threads,
                               const struct PckCheckBatch* ride, void* stream);
 
-/* Launch-shape knob of the coalesced kernels at threads = 256, for tuning sweeps: rows per wave
+/* Launch-shape knob of the coalesced kernels at threads = 256 with aligned rows, for tuning sweeps: rows per wave
  * slot (1, 2 or 4), vector positions loaded ahead per lane (1, 2 or 4) and non-temporal weight
  * loads (0 or 1); rows_per_wave = 0 restores the built-in choice.  Changes only speed: outputs
  * keep the same bits for every shape.  Process-wide and not thread-safe; no reference

@@ -188,23 +188,79 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// T virtual lanes per row, R rows per wave slot, U vector positions loaded ahead, kNt:
-// non-temporal weight loads (streamed once, so they need not displace x in the caches).
-// kPad: some vectors of a chain lie past n (n is not a multiple of T * vec), so loads of those
-// are redirected to column 0 and their data replaced by zeros.  kVector: 16-byte loads (n is a
-// multiple of vec and the pointers are aligned); otherwise element loads.
-template <bool kNt>
-__device__ __forceinline__ uint4 load_w(const unsigned char* p) {
-  if constexpr (kNt) {
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-    return make_uint4(v[0], v[1], v[2], v[3]);
+// How a launch reads W and x.
+//   kAligned    16-byte loads at 16-byte addresses: n is a multiple of the vector width and every
+//               pointer is aligned.
+//   kUnaligned  16-byte loads at any byte address (every n of at least one vector): gfx950's
+//               global loads take them, and a wave still reads contiguous kilobytes.  A row's
+//               last, partial vector is read as the 16 bytes that end the row (nothing past the
+//               row is touched) and moved into place in registers.
+//   kElement    element loads: rows shorter than one vector.
+enum class Load { kElement, kUnaligned, kAligned };
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_any __attribute__((aligned(1)));  // any byte address
+
+template <bool kNt, bool kAny>
+__device__ __forceinline__ uint4 load16(const void* p) {
+  u32x4 v;
+  if constexpr (kAny) {
+    const auto* q = static_cast<const u32x4_any*>(p);
+    v = kNt ? __builtin_nontemporal_load(q) : *q;
   } else {
-    return *reinterpret_cast<const uint4*>(p);
+    const auto* q = static_cast<const u32x4*>(p);
+    v = kNt ? __builtin_nontemporal_load(q) : *q;
+  }
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+typedef unsigned __int128 u128;
+
+__device__ __forceinline__ u128 as_u128(const uint4& v) {
+  return (static_cast<u128>((static_cast<uint64_t>(v.w) << 32) | v.z) << 64) |
+         ((static_cast<uint64_t>(v.y) << 32) | v.x);
+}
+__device__ __forceinline__ uint4 as_uint4(u128 v) {
+  const uint64_t lo = static_cast<uint64_t>(v), hi = static_cast<uint64_t>(v >> 64);
+  return make_uint4(static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32),
+                    static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32));
+}
+
+// Drops the first `skip` (0 .. V) of a vector's V elements, moves the rest to the front and
+// fills with zeros: the partial vector of a row, read as the V elements that end the row.
+template <bool kFp8>
+__device__ __forceinline__ void drop_front(uint4& w, int skip) {
+  const int bits = skip * (kFp8 ? 8 : 16);
+  w = as_uint4(bits < 128 ? as_u128(w) >> bits : 0);
+}
+template <bool kFp8>
+__device__ __forceinline__ void drop_front_x(uint4& xa, uint4& xb, int skip) {
+  if constexpr (!kFp8) {
+    drop_front<false>(xa, skip);
+  } else {  // 16 activations in two registers of eight
+    u128 lo = as_u128(skip >= 8 ? xb : xa), hi = skip >= 8 ? 0 : as_u128(xb);
+    const int bits = (skip & 7) * 16;
+    lo = bits ? (lo >> bits) | (hi << (128 - bits)) : lo;
+    hi = hi >> bits;
+    xa = as_uint4(skip < 16 ? lo : 0);
+    xb = as_uint4(skip < 16 ? hi : 0);
   }
 }
 
-template <int T, int R, int U, bool kFp8, bool kVector, bool kPad, bool kNt, bool kSums = false>
+// T virtual lanes per row, R rows per wave slot, U vector positions loaded ahead, kNt:
+// non-temporal weight loads (streamed once, so they need not displace x in the caches).
+// kPad: some vectors of a chain lie past n (n is not a multiple of T * vec); their loads are
+// redirected to column 0 (kUnaligned: to the row's last vector) and they add +0.  A chain slot
+// whose 64 vectors all lie past n adds +0 once instead of V products of zeros (the same sum,
+// sign of zero included), so a row's short last position costs what its columns cost.
+
+//
+// kLive: chain slots per lane that hold any column, when every row of the launch ends inside the
+// first kLive slots of its first position (n <= 64 kLive vec, one position).  The other slots'
+// chains sum padding only, so they are +0 without being loaded or kept in registers: a tree of
+// 512 or 1024 virtual lanes over a short row then costs what the row's own columns cost.
+template <int T, int R, int U, bool kFp8, Load kLoad, bool kPad, bool kNt, bool kSums = false,
+          int kLive = (T >= kWave ? T / kWave : 1)>
 __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group) {
   constexpr int V = kFp8 ? 16 : 8;
   constexpr int kLanesPerRow = T >= kWave ? kWave : T;
@@ -244,55 +300,73 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
     scale[r] = (kFp8 && it.y_scaled != nullptr) ? it.scale[live[r] ? row : it.m - 1] : 1.0f;
   }
 
-  float acc[R][kChains];
+  float acc[R][kLive];
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int j = 0; j < kChains; ++j) acc[r][j] = -0.0f;
-  RowSums rs[R][kChains];  // per row and chain: the lane's d and s (kSums only)
+    for (int j = 0; j < kLive; ++j) acc[r][j] = -0.0f;
+  RowSums rs[R][kLive];  // per row and chain: the lane's d and s (kSums only)
 
+  constexpr bool kAny = kLoad == Load::kUnaligned;
   for (int64_t v0 = 0; v0 < P; v0 += U) {
-    if constexpr (kVector) {
-      uint4 wb[U][R][kChains];
-      uint4 xa[U][kChains];
-      uint4 xb[U][kChains];
+    if constexpr (kLoad != Load::kElement) {
+      uint4 wb[U][R][kLive];
+      uint4 xa[U][kLive];
+      uint4 xb[U][kLive];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (U > 1 && v0 + u >= P) break;  // uniform: the tail of the last block
 #pragma unroll
-        for (int j = 0; j < kChains; ++j) {
+        for (int j = 0; j < kLive; ++j) {
           const int64_t col = ((v0 + u) * T + chain0 + kLanesPerRow * j) * V;
-          const int64_t at = (!kPad || col < n) ? col : 0;
-          xa[u][j] = *reinterpret_cast<const uint4*>(x + at);
-          if constexpr (kFp8) xb[u][j] = *reinterpret_cast<const uint4*>(x + at + 8);
+          const int64_t at = !kPad ? col : kAny ? (col < n - V ? col : n - V) : (col < n ? col : 0);
+          xa[u][j] = load16<false, kAny>(x + at);
+          if constexpr (kFp8) xb[u][j] = load16<false, kAny>(x + at + 8);
 #pragma unroll
           for (int r = 0; r < R; ++r)
-            wb[u][r][j] = load_w<kNt>(w_rows[r] + at * kElemBytes);
-          if constexpr (kPad) {
-            if (col >= n) {  // a padding vector: +0 products (0 x 0)
-              xa[u][j] = make_uint4(0, 0, 0, 0);
-              xb[u][j] = make_uint4(0, 0, 0, 0);
-#pragma unroll
-              for (int r = 0; r < R; ++r) wb[u][r][j] = make_uint4(0, 0, 0, 0);
-            }
-          }
+            wb[u][r][j] = load16<kNt, kAny>(w_rows[r] + at * kElemBytes);
         }
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (U > 1 && v0 + u >= P) break;
 #pragma unroll
-        for (int r = 0; r < R; ++r)
+        for (int j = 0; j < kLive; ++j) {
+          if constexpr (kPad) {
+            // the slot's first column, the same for every lane of the wave
+            const int64_t first = ((v0 + u) * T + kLanesPerRow * j) * V;
+            if (first >= n) {
 #pragma unroll
-          for (int j = 0; j < kChains; ++j)
+              for (int r = 0; r < R; ++r) acc[r][j] = acc[r][j] + 0.0f;
+              continue;
+            }
+            if (first + kLanesPerRow * V > n) {  // some of the slot's columns lie past n
+              const int64_t col = first + chain0 * V;
+              if constexpr (kAny) {
+                const int64_t over = col - (n - V);  // <= 0: a whole vector
+                const int skip = over <= 0 ? 0 : over < V ? static_cast<int>(over) : V;
+                drop_front_x<kFp8>(xa[u][j], xb[u][j], skip);
+#pragma unroll
+                for (int r = 0; r < R; ++r) drop_front<kFp8>(wb[u][r][j], skip);
+              } else if (col >= n) {
+                xa[u][j] = make_uint4(0, 0, 0, 0);
+                xb[u][j] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < R; ++r) wb[u][r][j] = make_uint4(0, 0, 0, 0);
+              }
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < R; ++r)
             add_products<kFp8, kSums>(acc[r][j], rs[r][j], wb[u][r][j], xa[u][j],
                                       kFp8 ? xb[u][j] : xa[u][j]);
+        }
       }
     } else {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
 #pragma unroll
-        for (int j = 0; j < kChains; ++j) {
+        for (int j = 0; j < kLive; ++j) {
           const int64_t col = (v0 * T + chain0 + kLanesPerRow * j) * V;
           add_products_scalar<kFp8, kSums>(acc[r][j], rs[r][j], w_rows[r], x, col, n);
         }
@@ -307,7 +381,7 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
-      for (int half = kChains / 2; half > 0; half /= 2)
+      for (int half = kLive / 2; half > 0; half /= 2)
 #pragma unroll
         for (int i = 0; i < half; ++i) {
           rs[r][i].d = rs[r][i].d + rs[r][i + half].d;
@@ -331,19 +405,24 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
   for (int r = 0; r < R; ++r) {
     // Halving inside each 32-lane virtual warp.
 #pragma unroll
-    for (int j = 0; j < kChains; ++j) acc[r][j] = halve32(acc[r][j]);
+    for (int j = 0; j < kLive; ++j) acc[r][j] = halve32(acc[r][j]);
     const int64_t row = (wave * kSlots + slot) * R + r;
     if constexpr (kSlots == 2) {
       // T = 32: one virtual warp per row; lanes 0 and 32 hold the two rows' sums.
       if (chain0 == 0 && live[r]) store_row(it, row, acc[r][0], scale[r]);
     } else {
       // Warp w = 2j + h is half h of chain slot j; reduce the T / 32 warp sums by halving.
-      constexpr int kWarps = 2 * kChains;
+      // The sums of slots past kLive are +0: adding them changes at most the sign of a zero.
+      constexpr int kWarps = 2 * kLive;
       float ws[kWarps];
 #pragma unroll
-      for (int j = 0; j < kChains; ++j) {
+      for (int j = 0; j < kLive; ++j) {
         ws[2 * j] = lane_value(acc[r][j], 0);
         ws[2 * j + 1] = lane_value(acc[r][j], kWarp);
+      }
+      if constexpr (kLive < kChains) {
+#pragma unroll
+        for (int i = 0; i < kWarps; ++i) ws[i] = ws[i] + 0.0f;
       }
 #pragma unroll
       for (int half = kWarps / 2; half > 0; half /= 2)
@@ -354,9 +433,9 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
   }
 }
 
-template <int T, int R, int U, bool kFp8, bool kVector, bool kPad, bool kNt>
+template <int T, int R, int U, bool kFp8, Load kLoad, bool kPad, bool kNt, int kLive>
 __global__ void __launch_bounds__(kGroupThreads) gemv_tree_kernel(const GemvBatch batch) {
-  gemv_rows<T, R, U, kFp8, kVector, kPad, kNt>(batch, blockIdx.x);
+  gemv_rows<T, R, U, kFp8, kLoad, kPad, kNt, false, kLive>(batch, blockIdx.x);
 }
 
 // A GEMV launch that also checks outputs of earlier launches: the first workgroups of the grid
@@ -381,14 +460,15 @@ __global__ void __launch_bounds__(kGroupThreads)
       check::check_pair<4>(ride, blockIdx.x, g, lds);
     return;
   }
-  gemv_rows<T, R, U, kFp8, true, kPad, kNt>(batch, static_cast<int64_t>(blockIdx.x) - items);
+  gemv_rows<T, R, U, kFp8, Load::kAligned, kPad, kNt>(batch,
+                                                      static_cast<int64_t>(blockIdx.x) - items);
 }
 
 // The in-pass GEMV: the tree's outputs plus each row's sums (d_i, s_i), and in the first
 // workgroups of the grid the row-sum checks of `ride` (outputs of earlier launches on the stream,
 // read from memory; one wave per (check, block) pair, the code of pck_rowsum_check, so the
 // results are bit-identical to it).  A check never reads anything this launch writes.
-template <int T, int R, int U, bool kFp8, bool kVector, bool kPad, bool kNt>
+template <int T, int R, int U, bool kFp8, Load kLoad, bool kPad, bool kNt, int kLive>
 __global__ void __launch_bounds__(kGroupThreads)
     gemv_rowsum_kernel(const GemvBatch batch, const PckRowSumBatch ride) {
   const int64_t items = rowsum::items(ride);
@@ -399,7 +479,7 @@ __global__ void __launch_bounds__(kGroupThreads)
     if (item < items) rowsum::check_item(ride, item);  // uniform per wave
     return;
   }
-  gemv_rows<T, R, U, kFp8, kVector, kPad, kNt, true>(batch, group - ride_groups);
+  gemv_rows<T, R, U, kFp8, kLoad, kPad, kNt, true, kLive>(batch, group - ride_groups);
 }
 
 // Naive tree (order of the reference model src/pck/gemv.py:14-57): `threads` = T virtual lanes
@@ -488,8 +568,9 @@ __global__ void __launch_bounds__(1024)
 }
 
 // Launch shape of the coalesced kernel: rows per wave slot, vector positions loaded ahead and
-// non-temporal weight loads.  T = 256 (the reference's default tree) has every combination
-// instantiated for tuning; other thread counts use one shape per padding / weight type.
+// non-temporal weight loads.  T = 256 with aligned rows (the reference's default tree) has every
+// combination instantiated for tuning; every other route has the one or two shapes it uses, with
+// non-temporal weight loads.
 struct TreeShape {
   int rows;
   int unroll;
@@ -504,7 +585,7 @@ TreeShape g_shape_override = {0, 0, 0};
 // where one row per wave and two positions ahead give twice the waves (4.9 against 5.4 us).
 // The sweeps replay each launch over weight copies that do not fit the Infinity Cache (with
 // four copies of FP8 down, 235 MB, plain loads won from the cache; streamed from HBM, as in a
-// decode pass, non-temporal loads take 13.1 against 14.6 us).
+// decode pass, non-temporal loads take 12.5 against 14.6 us).
 TreeShape choose_shape(int64_t per_lane, int64_t rows, bool fp8) {
   if (g_shape_override.rows > 0) return g_shape_override;
   if (fp8) return per_lane <= 2 && rows <= 4096 ? TreeShape{1, 2, 1} : TreeShape{2, 1, 1};
@@ -521,8 +602,20 @@ int64_t plan_groups(GemvBatch& batch, int64_t rows_per_group) {
   return batch.first_group[batch.count];
 }
 
+// The launch plan of a group: validated items, how its rows are read, whether any chain has
+// padding vectors, the longest row in vectors and per lane, and the total rows.
+struct GroupPlan {
+  GemvBatch batch{};
+  Load load = Load::kAligned;
+  bool pad = false;
+  int64_t max_vectors = 1;
+  int64_t max_per_lane = 1;
+  int64_t rows = 0;
+};
+
 // kSums: the in-pass kernel, with `rs` the row-sum checks it carries; otherwise the plain tree.
-template <int T, int R, int U, bool kFp8, bool kVector, bool kPad, bool kNt, bool kSums>
+template <int T, int R, int U, bool kFp8, Load kLoad, bool kPad, bool kNt, bool kSums,
+          int kLive = (T >= kWave ? T / kWave : 1)>
 hipError_t launch_tree(GemvBatch& batch, const PckRowSumBatch* rs, hipStream_t stream) {
   constexpr int kLanesPerRow = T >= kWave ? kWave : T;
   const int64_t groups = plan_groups(batch, (kWave / kLanesPerRow) * R * kWavesPerGroup);
@@ -530,13 +623,13 @@ hipError_t launch_tree(GemvBatch& batch, const PckRowSumBatch* rs, hipStream_t s
     const int64_t total = groups + (rowsum::items(*rs) + kWavesPerGroup - 1) / kWavesPerGroup;
     if (total == 0) return hipSuccess;
     if (total * kGroupThreads > 0xFFFFFFFFll) return hipErrorInvalidValue;  // 32-bit dispatch
-    gemv_rowsum_kernel<T, R, U, kFp8, kVector, kPad, kNt>
+    gemv_rowsum_kernel<T, R, U, kFp8, kLoad, kPad, kNt, kLive>
         <<<dim3(static_cast<unsigned>(total)), dim3(kGroupThreads), 0, stream>>>(batch, *rs);
   } else {
     (void)rs;
     if (groups == 0) return hipSuccess;
     if (groups * kGroupThreads > 0xFFFFFFFFll) return hipErrorInvalidValue;  // 32-bit dispatch
-    gemv_tree_kernel<T, R, U, kFp8, kVector, kPad, kNt>
+    gemv_tree_kernel<T, R, U, kFp8, kLoad, kPad, kNt, kLive>
         <<<dim3(static_cast<unsigned>(groups)), dim3(kGroupThreads), 0, stream>>>(batch);
   }
   return hipGetLastError();
@@ -544,40 +637,100 @@ hipError_t launch_tree(GemvBatch& batch, const PckRowSumBatch* rs, hipStream_t s
 
 template <int T, int R, bool kFp8, bool kPad, bool kNt, bool kSums>
 hipError_t launch_unroll(GemvBatch& batch, int unroll, const PckRowSumBatch* rs, hipStream_t s) {
-  if (unroll >= 4) return launch_tree<T, R, 4, kFp8, true, kPad, kNt, kSums>(batch, rs, s);
-  if (unroll == 2) return launch_tree<T, R, 2, kFp8, true, kPad, kNt, kSums>(batch, rs, s);
-  return launch_tree<T, R, 1, kFp8, true, kPad, kNt, kSums>(batch, rs, s);
+  constexpr Load L = Load::kAligned;
+  if (unroll >= 4) return launch_tree<T, R, 4, kFp8, L, kPad, kNt, kSums>(batch, rs, s);
+  if (unroll == 2) return launch_tree<T, R, 2, kFp8, L, kPad, kNt, kSums>(batch, rs, s);
+  return launch_tree<T, R, 1, kFp8, L, kPad, kNt, kSums>(batch, rs, s);
 }
 
-template <int T, bool kFp8, bool kPad, bool kSums>
-hipError_t launch_vector(GemvBatch& batch, TreeShape shape, const PckRowSumBatch* rs,
-                         hipStream_t s) {
-  if constexpr (T == 256) {
-    const bool nt = shape.nt != 0;
-    const int u = shape.unroll;
-    switch (shape.rows) {
-      case 4:
-        return nt ? launch_unroll<T, 4, kFp8, kPad, true, kSums>(batch, u, rs, s)
-                  : launch_unroll<T, 4, kFp8, kPad, false, kSums>(batch, u, rs, s);
-      case 2:
-        return nt ? launch_unroll<T, 2, kFp8, kPad, true, kSums>(batch, u, rs, s)
-                  : launch_unroll<T, 2, kFp8, kPad, false, kSums>(batch, u, rs, s);
-      default:
-        return nt ? launch_unroll<T, 1, kFp8, kPad, true, kSums>(batch, u, rs, s)
-                  : launch_unroll<T, 1, kFp8, kPad, false, kSums>(batch, u, rs, s);
-    }
-  } else {
-    (void)shape;
-    return launch_tree<T, 1, 2, kFp8, true, kPad, false, kSums>(batch, rs, s);
+// T = 256, aligned rows: every shape.
+template <bool kFp8, bool kPad, bool kSums>
+hipError_t launch_default(GemvBatch& batch, TreeShape shape, const PckRowSumBatch* rs,
+                          hipStream_t s) {
+  constexpr int T = 256;
+  const bool nt = shape.nt != 0;
+  const int u = shape.unroll;
+  switch (shape.rows) {
+    case 4:
+      return nt ? launch_unroll<T, 4, kFp8, kPad, true, kSums>(batch, u, rs, s)
+                : launch_unroll<T, 4, kFp8, kPad, false, kSums>(batch, u, rs, s);
+    case 2:
+      return nt ? launch_unroll<T, 2, kFp8, kPad, true, kSums>(batch, u, rs, s)
+                : launch_unroll<T, 2, kFp8, kPad, false, kSums>(batch, u, rs, s);
+    default:
+      return nt ? launch_unroll<T, 1, kFp8, kPad, true, kSums>(batch, u, rs, s)
+                : launch_unroll<T, 1, kFp8, kPad, false, kSums>(batch, u, rs, s);
   }
 }
 
+// Aligned rows in a tree of T != 256 lanes.  The shapes keep 8 to 16 vectors in flight per lane
+// (chains x R x U), fewer chains per lane leaving room for more rows or positions; the best of
+// R in {1, 2, 4}, U in {1 .. 4, 8} streamed from HBM, against R = 1, U = 2 with plain loads
+// (14336 x 4096 BF16: T = 64 / 128 / 512 19.6 / 19.9 / 20.0 against 23.5 / 22.4 / 21.8 us;
+// 4096 x 14336 FP8: T = 64 / 128 / 512 12.0 / 12.1 / 16.1 against 14.0 / 15.2 / 18.2 us).
+template <int T, bool kFp8, bool kPad, bool kSums>
+hipError_t launch_aligned(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
+  constexpr Load L = Load::kAligned;
+  GemvBatch& b = plan.batch;
+  if constexpr (T == 256) {
+    return launch_default<kFp8, kPad, kSums>(
+        b, choose_shape(plan.max_per_lane, plan.rows, kFp8), rs, s);
+  } else if constexpr (T >= 1024) {
+    return launch_tree<T, 1, 1, kFp8, L, kPad, true, kSums>(b, rs, s);
+  } else if constexpr (T >= 512) {
+    return launch_tree<T, kFp8 ? 2 : 1, 1, kFp8, L, kPad, true, kSums>(b, rs, s);
+  } else {
+    constexpr int U = T >= 128 ? 2 : 4;
+    if (!kFp8 && plan.max_vectors <= 512)  // BF16 rows of at most 4096 columns
+      return launch_tree<T, 1, 4, kFp8, L, kPad, true, kSums>(b, rs, s);
+    return launch_tree<T, 2, U, kFp8, L, kPad, true, kSums>(b, rs, s);
+  }
+}
+
+// Rows read at any byte address.  Two rows per wave slot: the best shape of the same sweep for
+// nearly every T and length.  Against element loads, at T = 256: BF16 14336 x 4100 22.3 against
+// 122 us, 14337 x 4099 29.7 against 120; FP8 28672 x 4104 27.1 against 325 us, 28673 x 4099
+// (addresses of any byte) 51 against 326.
+template <int T, bool kFp8, bool kSums>
+hipError_t launch_unaligned(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
+  constexpr int R = T >= 1024 || (T >= 512 && !kFp8) ? 1 : 2;
+  constexpr int U = T <= 64 ? 2 : 1;
+  return launch_tree<T, R, U, kFp8, Load::kUnaligned, true, true, kSums>(plan.batch, rs, s);
+}
+
+// Rows that end inside the first kLive chain slots (at most 64 kLive vectors).
+template <int T, int kLive, bool kFp8, bool kSums>
+hipError_t launch_live(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
+  constexpr Load A = Load::kAligned, X = Load::kUnaligned;
+  constexpr int Ra = kFp8 || kLive == 2 ? 2 : 1;
+  constexpr int Rx = kFp8 || kLive <= 4 ? 2 : 1;
+  GemvBatch& b = plan.batch;
+  return plan.load == A ? launch_tree<T, Ra, 1, kFp8, A, true, true, kSums, kLive>(b, rs, s)
+                        : launch_tree<T, Rx, 1, kFp8, X, true, true, kSums, kLive>(b, rs, s);
+}
+
+// The route of a launch: element loads for rows shorter than a vector; else the fewest live
+// chain slots that hold the longest row (T = 1024, 14336 x 4096: BF16 8 slots of 16 20.3 against
+// 36.6 us with all and 62 before, FP8 4 slots 19.9 against 69.5 and 139 us); else all slots.
+// pck_gemv_set_shape picks the shape of aligned T = 256 launches, which then keep all slots.
 template <int T, bool kFp8, bool kSums = false>
-hipError_t launch_for_threads(GemvBatch& batch, bool vector, bool pad, TreeShape shape,
-                              hipStream_t s, const PckRowSumBatch* rs = nullptr) {
-  if (!vector) return launch_tree<T, 1, 1, kFp8, false, true, false, kSums>(batch, rs, s);
-  return pad ? launch_vector<T, kFp8, true, kSums>(batch, shape, rs, s)
-             : launch_vector<T, kFp8, false, kSums>(batch, shape, rs, s);
+hipError_t launch_for_threads(GroupPlan& plan, hipStream_t s, const PckRowSumBatch* rs = nullptr) {
+  if (plan.load == Load::kElement)
+    return launch_tree<T, 1, 1, kFp8, Load::kElement, true, false, kSums>(plan.batch, rs, s);
+  const bool all =
+      T == 256 && plan.load == Load::kAligned && g_shape_override.rows > 0;  // a chosen shape
+  if constexpr (T >= 256) {
+    if (!all && plan.max_vectors <= 2 * kWave) return launch_live<T, 2, kFp8, kSums>(plan, rs, s);
+  }
+  if constexpr (T >= 512) {
+    if (plan.max_vectors <= 4 * kWave) return launch_live<T, 4, kFp8, kSums>(plan, rs, s);
+  }
+  if constexpr (T >= 1024) {
+    if (plan.max_vectors <= 8 * kWave) return launch_live<T, 8, kFp8, kSums>(plan, rs, s);
+  }
+  if (plan.load == Load::kUnaligned) return launch_unaligned<T, kFp8, kSums>(plan, rs, s);
+  return plan.pad ? launch_aligned<T, kFp8, true, kSums>(plan, rs, s)
+                  : launch_aligned<T, kFp8, false, kSums>(plan, rs, s);
 }
 
 template <int R, int U, bool kFp8, bool kPad, bool kNt = true>
@@ -609,16 +762,6 @@ hipError_t launch_ride(GemvBatch& batch, bool pad, int64_t per_lane, const PckCh
   }
 }
 
-// The launch plan of a group: validated items, whether every row takes 16-byte vectors, whether
-// any chain has padding vectors, the longest chain and the total rows.
-struct GroupPlan {
-  GemvBatch batch{};
-  bool vector = true;
-  bool pad = false;
-  int64_t max_per_lane = 1;
-  int64_t rows = 0;
-};
-
 template <bool kFp8>
 hipError_t plan_group(const PckGemv* gemvs, double* const* sums, int count, int threads,
                       GroupPlan& plan, const float* const* scales = nullptr,
@@ -647,8 +790,12 @@ hipError_t plan_group(const PckGemv* gemvs, double* const* sums, int count, int 
     }
     plan.rows += d.m;
     if (d.m > 0) {
-      plan.vector = plan.vector && n % V == 0 && reinterpret_cast<uintptr_t>(d.W) % 16 == 0 &&
-                    reinterpret_cast<uintptr_t>(d.x) % 16 == 0;
+      const bool aligned = n % V == 0 && reinterpret_cast<uintptr_t>(d.W) % 16 == 0 &&
+                           reinterpret_cast<uintptr_t>(d.x) % 16 == 0;
+      const Load load = n < V ? Load::kElement : aligned ? Load::kAligned : Load::kUnaligned;
+      if (load < plan.load) plan.load = load;  // the narrowest loads any item needs
+      const int64_t vectors = (n + V - 1) / V;
+      plan.max_vectors = vectors > plan.max_vectors ? vectors : plan.max_vectors;
       plan.max_per_lane = per_lane > plan.max_per_lane ? per_lane : plan.max_per_lane;
       plan.pad = plan.pad || n % (static_cast<int64_t>(threads) * V) != 0;
     }
@@ -663,36 +810,24 @@ hipError_t launch_group(const PckGemv* gemvs, int count, int threads, const PckC
   GroupPlan plan;
   if (plan_group<kFp8>(gemvs, nullptr, count, threads, plan, scales, scaled) != hipSuccess)
     return hipErrorInvalidValue;
-  GemvBatch& batch = plan.batch;
-  const bool vector = plan.vector, pad = plan.pad;
-  const int64_t max_per_lane = plan.max_per_lane;
   if (ride != nullptr) {
     if (check::validate(*ride) != hipSuccess) return hipErrorInvalidValue;
-    if (threads == 256 && vector) {
-      bool any_rows = false;
-      for (int g = 0; g < count; ++g) any_rows = any_rows || batch.item[g].m > 0;
-      if (any_rows) return launch_ride<kFp8>(batch, pad, max_per_lane, *ride, stream);
-    }
+    if (threads == 256 && plan.load == Load::kAligned && plan.rows > 0)
+      return launch_ride<kFp8>(plan.batch, plan.pad, plan.max_per_lane, *ride, stream);
     // Other configurations: the same check as its own launch first (identical results).
     const int64_t items = ride->start[ride->count];
     if (items * check::kThreads > 0xFFFFFFFFll) return hipErrorInvalidValue;
     const int err = pck_blocked_check(ride, stream);
     if (err != 0) return static_cast<hipError_t>(err);
   }
-  const TreeShape shape = choose_shape(max_per_lane, plan.rows, kFp8);
   switch (threads) {
-    case 32: return launch_for_threads<32, kFp8>(batch, vector, pad, shape, stream);
-    case 64: return launch_for_threads<64, kFp8>(batch, vector, pad, shape, stream);
-    case 128: return launch_for_threads<128, kFp8>(batch, vector, pad, shape, stream);
-    case 256: return launch_for_threads<256, kFp8>(batch, vector, pad, shape, stream);
-    case 512: return launch_for_threads<512, kFp8>(batch, vector, pad, shape, stream);
-    default: return launch_for_threads<1024, kFp8>(batch, vector, pad, shape, stream);
+    case 32: return launch_for_threads<32, kFp8>(plan, stream);
+    case 64: return launch_for_threads<64, kFp8>(plan, stream);
+    case 128: return launch_for_threads<128, kFp8>(plan, stream);
+    case 256: return launch_for_threads<256, kFp8>(plan, stream);
+    case 512: return launch_for_threads<512, kFp8>(plan, stream);
+    default: return launch_for_threads<1024, kFp8>(plan, stream);
   }
-}
-
-// Launch shape of the in-pass kernel (pck_gemv_set_shape overrides it as for the plain tree).
-TreeShape choose_rowsum_shape(int64_t per_lane, int64_t rows, bool fp8) {
-  return choose_shape(per_lane, rows, fp8);
 }
 
 template <bool kFp8>
@@ -705,17 +840,13 @@ hipError_t launch_group_rowsums(const PckGemv* gemvs, double* const* sums, int c
   PckRowSumBatch none{};
   const PckRowSumBatch* rs = ride != nullptr ? ride : &none;
   if (rowsum::validate(*rs) != hipSuccess) return hipErrorInvalidValue;
-  GemvBatch& b = plan.batch;
-  const TreeShape shape = choose_rowsum_shape(plan.max_per_lane, plan.rows, kFp8);
-  const bool v = plan.vector, p = plan.pad;
-
   switch (threads) {
-    case 32: return launch_for_threads<32, kFp8, true>(b, v, p, shape, stream, rs);
-    case 64: return launch_for_threads<64, kFp8, true>(b, v, p, shape, stream, rs);
-    case 128: return launch_for_threads<128, kFp8, true>(b, v, p, shape, stream, rs);
-    case 256: return launch_for_threads<256, kFp8, true>(b, v, p, shape, stream, rs);
-    case 512: return launch_for_threads<512, kFp8, true>(b, v, p, shape, stream, rs);
-    default: return launch_for_threads<1024, kFp8, true>(b, v, p, shape, stream, rs);
+    case 32: return launch_for_threads<32, kFp8, true>(plan, stream, rs);
+    case 64: return launch_for_threads<64, kFp8, true>(plan, stream, rs);
+    case 128: return launch_for_threads<128, kFp8, true>(plan, stream, rs);
+    case 256: return launch_for_threads<256, kFp8, true>(plan, stream, rs);
+    case 512: return launch_for_threads<512, kFp8, true>(plan, stream, rs);
+    default: return launch_for_threads<1024, kFp8, true>(plan, stream, rs);
   }
 }
 

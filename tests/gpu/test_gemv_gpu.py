@@ -115,6 +115,53 @@ def test_naive_llama_shapes_bit_exact(m: int, n: int) -> None:
     assert_bits(y, gemv_naive_c(W.float().numpy(), x.float().numpy(), 256))
 
 
+# Row lengths around every edge of the vector routes, in vectors v of V columns: shorter than one
+# vector (element loads), one vector, the ends of 2, 4 and 8 live chain slots (64 vectors each)
+# and of a position (threads vectors), each whole and ragged, at every thread count.
+@pytest.mark.parametrize("threads", [32, 64, 128, 256, 512, 1024])
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+def test_every_row_length_route_gives_the_model_bits(fp8: bool, threads: int) -> None:
+    V = 16 if fp8 else 8
+    edges = {1, 128, 256, 512, threads, 2 * threads + 1}
+    lengths = sorted({V - 1, *(v * V + d for v in edges for d in (0, 1, V // 2, V - 1)),
+                      *(v * V - 1 for v in edges)})
+    rng = np.random.default_rng(threads + V)
+    vals = e4m3_values()
+    for n in lengths:
+        print(f"route fp8={fp8} threads={threads} n={n}", flush=True)
+        x = bf16(rng.standard_normal(n))
+        if fp8:
+            codes = rng.integers(0, 256, (9, n), dtype=np.uint8)
+            codes[(codes & 0x7F) == 0x7F] = 0  # no NaN codes
+            W = vals[codes].astype(np.float32)
+            y = gemv_fp8(torch.from_numpy(codes).view(torch.float8_e4m3fn).cuda(), to_gpu(x), threads)
+        else:
+            W = bf16(rng.standard_normal((9, n)) * 0.02)
+            W[0] = 0.0  # signed zeros: every product of row 0 is a zero of x's sign
+            y = gemv_coalesced(to_gpu(W), to_gpu(x), threads)
+        assert_bits(y.cpu().numpy(), emulate_gemv_coalesced(W, x, threads, vec=V))
+
+
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+@pytest.mark.parametrize(("off_w", "off_x"), [(1, 0), (0, 1), (3, 5), (8, 4)])
+def test_rows_at_any_address_and_no_read_past_the_row(fp8: bool, off_w: int, off_x: int) -> None:
+    """W and x start off_w and off_x elements into their buffers and are followed by NaN: a
+    column past the last row or past x that reached a sum would show."""
+    m, n = 5, 2 * 256 * (16 if fp8 else 8) + 37
+    rng = np.random.default_rng(off_w * 10 + off_x)
+    x = bf16(rng.standard_normal(n))
+    xb = torch.full((n + 64,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    xb[off_x : off_x + n] = to_gpu(x)
+    codes = rng.integers(0, 0x7F, (m, n), dtype=np.uint8)
+    W = e4m3_values()[codes].astype(np.float32) if fp8 else bf16(rng.standard_normal((m, n)))
+    raw = torch.from_numpy(codes).cuda() if fp8 else to_gpu(W).view(torch.uint16)
+    wb = torch.full((m * n + 64,), 0x7F if fp8 else 0x7FC0, dtype=raw.dtype, device="cuda")
+    wb[off_w : off_w + m * n] = raw.reshape(-1)
+    Wt = wb.view(torch.float8_e4m3fn if fp8 else torch.bfloat16)[off_w : off_w + m * n].view(m, n)
+    y = (gemv_fp8 if fp8 else gemv_coalesced)(Wt, xb[off_x : off_x + n], 256)
+    assert_bits(y.cpu().numpy(), emulate_gemv_coalesced(W, x, 256, vec=16 if fp8 else 8))
+
+
 @kernels
 @settings(max_examples=30, deadline=None)
 @given(gemv_problems(max_rows=32, max_cols=600), st.sampled_from([32, 64, 128, 256]))
