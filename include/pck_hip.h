@@ -359,6 +359,19 @@ typedef struct PckMemberArgs {
 
 int pck_check_members_ex(const PckMemberArgs* args, void* stream);
 
+/* pck_check_members_ex with every row split over workgroups, in two launches: for logits of a
+ * 16-bit type, rows without a top-k (read once, not twice) and batches of fewer rows than the
+ * GPU has compute units.  logits_kind: 0 = FP32, 1 = BF16, 2 = FP16 (`logits` then points to
+ * that type and is widened exactly).  `workspace` is the caller's, 16-byte aligned, of at least
+ * the bytes pck_check_members_workspace gives; it needs no clearing and is not shared between
+ * calls that overlap.  ok and above are those of pck_check_members_ex, mass_above is within the
+ * same bound (member_eps32).  pck_check_members_workspace gives 0 bytes for a batch that the one
+ * launch serves better or that does not split (a top-k above 128 with a top-p); the split entry
+ * then returns hipErrorInvalidValue.  No reference counterpart. */
+int pck_check_members_workspace(const PckMemberArgs* args, int logits_kind, int64_t* bytes);
+int pck_check_members_split(const PckMemberArgs* args, int logits_kind, void* workspace,
+                            int64_t workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Set-sampling checker (top-k / top-p): is sel[b, 0 .. len[b]) a valid top-k set (top_p = 0,
  * length k) or a valid minimal top-p nucleus (top_p = 1) of row b of logits (rows, vocab) FP32?

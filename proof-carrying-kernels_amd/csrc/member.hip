@@ -341,6 +341,73 @@ __device__ uint32_t radix_select(int64_t rank, V&& visit, Scratch& s) {
   return prefix;
 }
 
+// One row's request, as the checks use it.
+struct RowRequest {
+  int64_t token;
+  bool in_range;    // the token id lies in [0, vocab)
+  int64_t k_row;    // top-k clamped to [1, vocab] (reference src/pck/member.py:153)
+  bool request_ok;  // the request index lies inside the temperature array (or there is none)
+  bool greedy;
+  double p;
+  bool want_mass;  // a top-p below 1
+  bool use_kth;    // the kept set is cut at the k_eff-th largest logit
+  int64_t k_eff;
+};
+
+__device__ __forceinline__ RowRequest row_request(const MemberArgs& A, int64_t r) {
+  RowRequest q;
+  q.token = A.tokens[r];
+  q.in_range = q.token >= 0 && q.token < A.vocab;
+  const int64_t k_req = A.top_k ? A.top_k[r] : A.vocab;
+  q.k_row = k_req < 1 ? 1 : (k_req > A.vocab ? A.vocab : k_req);
+  // Greedy rows: the caller's flags, or temperature 0 of the row's request (vLLM's sampling
+  // state, read through the row's request index).  A request index outside the temperature
+  // array rejects the row without reading it.
+  const int64_t request = A.temperature ? A.temperature_index[r] : 0;
+  q.request_ok = !A.temperature || (request >= 0 && request < A.temperature_count);
+  q.greedy = A.temperature ? q.request_ok && A.temperature[q.request_ok ? request : 0] == 0.0f
+                           : (A.greedy ? A.greedy[r] != 0 : false);
+  const bool has_p = A.top_p != nullptr;
+  q.p = !has_p ? 1.0
+        : A.top_p_fp32 ? static_cast<double>(static_cast<const float*>(A.top_p)[r])
+                       : static_cast<const double*>(A.top_p)[r];
+  q.want_mass = has_p && q.p < 1.0;
+  q.use_kth = A.all_k || (A.k_lim > 0 && q.k_row < A.vocab);
+  q.k_eff = q.k_row < A.k_lim ? q.k_row : A.k_lim;
+  return q;
+}
+
+// The row's verdict from its exact count above the token and its two masses (z kept, a kept and
+// above the token; used when the row wants a mass), written by one lane.
+__device__ __forceinline__ void write_verdict(const MemberArgs& A, int64_t r, const RowRequest& q,
+                                              int64_t above, bool any_nan, double z, double a) {
+  bool ok = q.request_ok && !any_nan && q.in_range && above < (q.greedy ? 1 : q.k_row);
+  double mass = 0.0;
+  if (q.want_mass) {
+    const double ratio = a / z;
+    mass = ratio;
+    const double high = next_up(q.p + A.slack);  // the bound rounded outward
+    ok = ok && (q.greedy || ratio < high);
+  }
+  if (A.ok) A.ok[r] = ok;
+  if (A.above) A.above[r] = above;
+  if (A.mass_above) A.mass_above[r] = mass;
+  if (A.totals) {
+    // Running totals (integer atomics, so the sums do not depend on the order of rows):
+    // rows, rejected, injected, caught (rejected and injected), false alarms (rejected, not
+    // injected), and the maximum of r - p over accepted top-p rows not greedy (the key of
+    // -1 is the host's initial value: no such row yet).
+    unsigned long long* tot = A.totals;
+    const bool injected = A.injected ? A.injected[r] != 0 : false;
+    atomicAdd(&tot[0], 1ull);
+    if (!ok) atomicAdd(&tot[1], 1ull);
+    if (injected) atomicAdd(&tot[2], 1ull);
+    if (!ok && injected) atomicAdd(&tot[3], 1ull);
+    if (!ok && !injected) atomicAdd(&tot[4], 1ull);
+    if (ok && q.want_mass && !q.greedy) atomicMax(&tot[5], order_key64(mass - q.p));
+  }
+}
+
 __global__ void __launch_bounds__(kThreads) member_kernel(const MemberArgs A) {
   __shared__ Scratch s;
   const int64_t r = blockIdx.x;
@@ -348,27 +415,10 @@ __global__ void __launch_bounds__(kThreads) member_kernel(const MemberArgs A) {
   const int64_t vocab = A.vocab;
   const float* __restrict__ row = A.logits + r * vocab;
 
-  const int64_t token = A.tokens[r];
-  const bool in_range = token >= 0 && token < vocab;
-  const float lt = row[in_range ? token : (token < 0 ? 0 : vocab - 1)];
-  // a requested top-k is clamped to [1, vocab] (reference src/pck/member.py:153)
-  const int64_t k_req = A.top_k ? A.top_k[r] : vocab;
-  const int64_t k_row = k_req < 1 ? 1 : (k_req > vocab ? vocab : k_req);
-  // Greedy rows: the caller's flags, or temperature 0 of the row's request (vLLM's sampling
-  // state, read through the row's request index).  A request index outside the temperature
-  // array rejects the row without reading it.
-  const int64_t request = A.temperature ? A.temperature_index[r] : 0;
-  const bool request_ok = !A.temperature || (request >= 0 && request < A.temperature_count);
-  const bool greedy = A.temperature ? request_ok && A.temperature[request_ok ? request : 0] == 0.0f
-                                    : (A.greedy ? A.greedy[r] != 0 : false);
-  const bool has_p = A.top_p != nullptr;
-  const double p = !has_p ? 1.0
-                   : A.top_p_fp32 ? static_cast<double>(static_cast<const float*>(A.top_p)[r])
-                                  : static_cast<const double*>(A.top_p)[r];
-
-  const bool want_mass = has_p && p < 1.0;
-  const bool use_kth = A.all_k || (A.k_lim > 0 && k_row < vocab);
-  const int64_t k_eff = k_row < A.k_lim ? k_row : A.k_lim;
+  const RowRequest q = row_request(A, r);
+  const float lt = row[q.in_range ? q.token : (q.token < 0 ? 0 : vocab - 1)];
+  const bool want_mass = q.want_mass, use_kth = q.use_kth;
+  const int64_t k_eff = q.k_eff;
   const bool fused = want_mass && use_kth && k_eff <= kThreads;
   const int64_t prefix = vocab < kPrefix ? vocab : kPrefix;
 
@@ -466,11 +516,9 @@ __global__ void __launch_bounds__(kThreads) member_kernel(const MemberArgs A) {
   const bool any_nan = flags & 1;
   const bool overflow = flags & 2;
 
-  bool ok = request_ok && !any_nan && in_range && above < (greedy ? 1 : k_row);
-  double mass = 0.0;
+  double z = 0.0;
+  double a = 0.0;
   if (want_mass) {
-    double z = 0.0;
-    double a = 0.0;
     if (!use_kth) {
       for_each<false>(row, 0, vocab, [&](float l) {
         const float e = split_term(l, m);
@@ -517,46 +565,608 @@ __global__ void __launch_bounds__(kThreads) member_kernel(const MemberArgs A) {
       });
     }
     group_sum2(z, a, s);
-    const double ratio = a / z;
-    mass = ratio;
-    const double high = next_up(p + A.slack);  // the bound rounded outward
-    ok = ok && (greedy || ratio < high);
   }
-  if (t == 0) {
-    if (A.ok) A.ok[r] = ok;
-    if (A.above) A.above[r] = above;
-    if (A.mass_above) A.mass_above[r] = mass;
-    if (A.totals) {
-      // Running totals (integer atomics, so the sums do not depend on the order of rows):
-      // rows, rejected, injected, caught (rejected and injected), false alarms (rejected, not
-      // injected), and the maximum of r - p over accepted top-p rows not greedy (the key of
-      // -1 is the host's initial value: no such row yet).
-      unsigned long long* tot = A.totals;
-      const bool injected = A.injected ? A.injected[r] != 0 : false;
-      atomicAdd(&tot[0], 1ull);
-      if (!ok) atomicAdd(&tot[1], 1ull);
-      if (injected) atomicAdd(&tot[2], 1ull);
-      if (!ok && injected) atomicAdd(&tot[3], 1ull);
-      if (!ok && !injected) atomicAdd(&tot[4], 1ull);
-      if (ok && want_mass && !greedy) atomicMax(&tot[5], order_key64(mass - p));
+  if (t == 0) write_verdict(A, r, q, above, any_nan, z, a);
+}
+
+// ---- rows split over workgroups ----------------------------------------------------------------
+//
+// One workgroup per row leaves most of the GPU idle for a small batch, reads a row without a
+// top-k twice, and needs FP32 logits.  The split check gives every (row, segment of L logits) a
+// 256-lane workgroup that reads its segment once, in the logits' own type, and keeps it in
+// registers:
+//   segment  count above the token, NaN flag, maximum; then, for a row cut at its k_eff-th
+//            largest logit, `low`: each wave finds the ceil(k_eff / 4)-th largest of its 64 lane
+//            maxima (its top 16 key bits, by ballots), and low is the smallest of the four, so at
+//            least k_eff of the segment's logits are >= low and the row's kth is >= low.  Every
+//            logit > low goes into the segment's slots, those equal to it are counted.  For a
+//            row that keeps everything: the FP64 sums of its terms relative to the segment's own
+//            maximum.
+//   finish   a workgroup per row.  Lower bounds of kth are every segment's low and, in the same
+//            way as low, the smallest over the four waves of the ceil(k_eff / 4)-th largest of
+//            the wave's lane maxima over the slots; G is the largest of them.  Only slots > G
+//            matter, one or two hundred values: kth is the k_eff-th largest of them, or G itself
+//            when fewer than k_eff exceed it (the logits equal to G then enter as one term times
+//            their count, so ties, such as the -inf of masked logits, take no slots).  A row
+//            without a top-k adds the segments' sums scaled by exp(m_s - max) in FP64.
+// Orders are fixed (lane, wave, segment), nothing depends on scheduling.  A segment with more
+// than kSegSlots logits above its low, or more than kCap of them above G, sends the row to an
+// exact radix select over the row by the finish workgroup, as in the one-workgroup kernel.
+constexpr int kSegThreads = 256;
+constexpr int kSegWaves = kSegThreads / kWave;
+constexpr int kSegSlots = 1024;
+constexpr int kFinishThreads = 256;
+constexpr int kFinishWaves = kFinishThreads / kWave;
+constexpr int64_t kSplitMaxK = 128;  // top-k values the lane maxima of a segment can bound
+
+// The largest float of 16 key bits that at least `want` of the wave's lanes hold a value >= of
+// (-inf if fewer do): the key's top 16 bits, from the highest down, each kept if enough lanes
+// still reach it.
+__device__ __forceinline__ float wave_bound(float v, int want) {
+  const uint32_t key = order_key(v);
+  uint32_t bound = 0;
+#pragma unroll
+  for (int bit = 31; bit >= 16; --bit) {
+    const uint32_t trial = bound | (1u << bit);
+    if (__builtin_popcountll(__ballot(key >= trial)) >= want) bound = trial;
+  }
+  const float low = key_value(bound);
+  return low == low ? low : -__builtin_inff();  // below the finite values
+}
+
+enum class Logits { kF32, kBf16, kF16 };
+
+template <Logits kType>
+struct LogitType;
+template <>
+struct LogitType<Logits::kF32> {
+  typedef float type;
+  static __device__ __forceinline__ float widen(float v) { return v; }
+};
+template <>
+struct LogitType<Logits::kBf16> {
+  typedef uint16_t type;
+  static __device__ __forceinline__ float widen(uint16_t v) {
+    return __uint_as_float(static_cast<uint32_t>(v) << 16);
+  }
+};
+template <>
+struct LogitType<Logits::kF16> {
+  typedef _Float16 type;
+  static __device__ __forceinline__ float widen(_Float16 v) { return static_cast<float>(v); }
+};
+
+struct alignas(16) SegmentHeader {
+  float max, low;
+  uint32_t above, ties;  // logits above the token's; logits equal to low
+  uint32_t count;        // logits above low (the first kSegSlots are in the slots)
+  int flags;             // bit 0: a NaN
+  double z, a;           // kept mass and mass above the token, relative to max (no top-k)
+  uint64_t unused;
+};
+static_assert(sizeof(SegmentHeader) == 48, "three 16-byte words");
+
+struct SplitArgs {
+  MemberArgs m;
+  SegmentHeader* headers;  // (rows, segments)
+  float* slots;            // (rows, segments, kSegSlots), when any row has a top-k
+  int64_t segments;
+  int64_t length;  // logits per segment
+};
+
+struct SegmentScratch {
+  uint32_t above[kSegWaves], ties[kSegWaves], count[kSegWaves];
+  int flags[kSegWaves];
+  float max[kSegWaves], low[kSegWaves];
+  double z[kSegWaves], a[kSegWaves];
+};
+
+template <Logits kType, int kLoads>
+__global__ void __launch_bounds__(kSegThreads) member_segment_kernel(const SplitArgs S) {
+  using L = LogitType<kType>;
+  using T = typename L::type;
+  constexpr int kVec = 16 / static_cast<int>(sizeof(T));
+  constexpr int kElems = kLoads * kVec;
+  typedef T vec __attribute__((ext_vector_type(kVec)));
+  typedef vec vec_any __attribute__((aligned(sizeof(T))));  // a row may start at any logit
+  __shared__ SegmentScratch s;
+
+  const MemberArgs& A = S.m;
+  const int t = static_cast<int>(threadIdx.x);
+  const uint32_t item = blockIdx.x;  // row * segments + segment
+  const uint32_t segments = static_cast<uint32_t>(S.segments);
+  const int64_t r = item / segments;
+  const int64_t j0 = static_cast<int64_t>(item % segments) * S.length;
+  const int64_t vocab = A.vocab;
+  const T* __restrict__ row = reinterpret_cast<const T*>(A.logits) + r * vocab;
+  const float inf = __builtin_inff();
+
+  // The segment in registers; slots past the row hold -inf, which no count, sum or candidate
+  // sees.
+  float x[kElems];
+  if (j0 + S.length <= vocab) {
+    vec v[kLoads];
+#pragma unroll
+    for (int q = 0; q < kLoads; ++q)
+      v[q] = __builtin_nontemporal_load(
+          reinterpret_cast<const vec_any*>(row + j0 + (q * kSegThreads + t) * kVec));
+#pragma unroll
+    for (int i = 0; i < kElems; ++i) x[i] = L::widen(v[i / kVec][i % kVec]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < kElems; ++i) {
+      const int64_t j = j0 + (i / kVec * kSegThreads + t) * kVec + i % kVec;
+      const float v = L::widen(row[j < vocab ? j : vocab - 1]);
+      x[i] = j < vocab ? v : -inf;
     }
   }
+  const RowRequest q = row_request(A, r);
+  const float lt = L::widen(row[q.in_range ? q.token : (q.token < 0 ? 0 : vocab - 1)]);
+
+  uint32_t above = 0;
+  int nan = 0;
+  float top = -inf;
+#pragma unroll
+  for (int i = 0; i < kElems; ++i) {
+    above += x[i] > lt;
+    nan |= x[i] != x[i];
+    top = fmaxf(top, x[i]);
+  }
+  const uint32_t wave_above = wave_reduce(above, [](uint32_t a, uint32_t b) { return a + b; });
+  const uint32_t wave_nan =
+      wave_reduce(static_cast<uint32_t>(nan), [](uint32_t a, uint32_t b) { return a | b; });
+  const float wave_max = wave_reduce(top, [](float a, float b) { return fmaxf(a, b); });
+  const int wave = t / kWave;
+  const bool cut = q.want_mass && q.use_kth;  // uniform over the workgroup
+  float wave_low = -inf;
+  if (cut) wave_low = wave_bound(top, static_cast<int>((q.k_eff + kSegWaves - 1) / kSegWaves));
+  if (lane_id() == 0) {
+    s.above[wave] = wave_above;
+    s.flags[wave] = static_cast<int>(wave_nan);
+    s.max[wave] = wave_max;
+    s.low[wave] = wave_low;
+  }
+  __syncthreads();
+  SegmentHeader h{};
+  h.above = (s.above[0] + s.above[1]) + (s.above[2] + s.above[3]);
+  h.flags = (s.flags[0] | s.flags[1]) | (s.flags[2] | s.flags[3]);
+  h.max = fmaxf(fmaxf(s.max[0], s.max[1]), fmaxf(s.max[2], s.max[3]));
+  h.low = -inf;
+
+  if (cut) {
+    const float low = fminf(fminf(s.low[0], s.low[1]), fminf(s.low[2], s.low[3]));
+    uint32_t mine = 0, ties = 0;
+#pragma unroll
+    for (int i = 0; i < kElems; ++i) {
+      mine += x[i] > low;
+      ties += x[i] == low;
+    }
+    const uint32_t incl = wave_inclusive_sum(mine);
+    const uint32_t wave_ties = wave_reduce(ties, [](uint32_t a, uint32_t b) { return a + b; });
+    if (lane_id() == kWave - 1) s.count[wave] = incl;
+    if (lane_id() == 0) s.ties[wave] = wave_ties;
+    __syncthreads();
+    uint32_t at = incl - mine;
+    for (int w = 0; w < wave; ++w) at += s.count[w];
+    float* slots = S.slots + static_cast<int64_t>(item) * kSegSlots;
+    if (mine != 0) {
+#pragma unroll
+      for (int i = 0; i < kElems; ++i) {
+        if (x[i] > low) {
+          if (at < kSegSlots) slots[at] = x[i];
+          ++at;
+        }
+      }
+    }
+    h.low = low;
+    h.count = (s.count[0] + s.count[1]) + (s.count[2] + s.count[3]);
+    h.ties = (s.ties[0] + s.ties[1]) + (s.ties[2] + s.ties[3]);
+  } else if (q.want_mass) {
+    double z = 0.0, a = 0.0;
+#pragma unroll
+    for (int i = 0; i < kElems; ++i) {
+      const float e = split_term(x[i], h.max);
+      z += e;
+      a += x[i] > lt ? e : 0.0;
+    }
+    const auto add = [](double u, double v) { return u + v; };
+    z = wave_reduce(z, add);
+    a = wave_reduce(a, add);
+    if (lane_id() == 0) {
+      s.z[wave] = z;
+      s.a[wave] = a;
+    }
+    __syncthreads();
+    h.z = (s.z[0] + s.z[1]) + (s.z[2] + s.z[3]);
+    h.a = (s.a[0] + s.a[1]) + (s.a[2] + s.a[3]);
+  }
+  if (t == 0) S.headers[item] = h;
+}
+
+struct FinishScratch : Scratch {
+  float low[kFinishWaves], kth[kFinishWaves], max[kFinishWaves];
+  uint32_t above[kFinishWaves], count[kFinishWaves], ties[kFinishWaves];
+  int flags[kFinishWaves];
+  double z[kFinishWaves], a[kFinishWaves];
+};
+
+// 256 lanes: the exchanges between waves are short chains of LDS reads, and a row of 152 K logits
+// has 19 segments, one round of early slots.  Against 1024 lanes and a radix select for every
+// row: see the figures at split_plan.
+template <Logits kType>
+__global__ void __launch_bounds__(kFinishThreads) member_finish_kernel(const SplitArgs S) {
+  using L = LogitType<kType>;
+  using T = typename L::type;
+  constexpr int kEarly = 5;  // segments per wave whose first slots are read ahead,
+  constexpr int kDeep = 2;   // this many 64-slot rows of each
+  constexpr int kHeld = 4;   // candidates per lane when one wave selects
+  __shared__ FinishScratch s;
+
+  const MemberArgs& A = S.m;
+  const int64_t r = blockIdx.x;
+  const int t = static_cast<int>(threadIdx.x);
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(wave_id());
+  const int64_t n = S.segments;
+  const SegmentHeader* hs = S.headers + r * n;
+  const float* slots = S.slots + r * n * kSegSlots;
+  const float inf = __builtin_inff();
+  // Lane i of wave w holds the header of segment w + 4 i; the first slots of the wave's first
+  // segments are requested with the headers (what they hold past a segment's count is not used).
+  const int64_t own = wave + static_cast<int64_t>(lane) * kFinishWaves;
+  SegmentHeader mine_h{};
+  mine_h.max = mine_h.low = -inf;
+  if (own < n) mine_h = hs[own];
+  float early[kEarly][kDeep];
+  const bool any_cut = A.top_p != nullptr && A.k_lim > 0;  // there are slots
+  if (any_cut) {
+#pragma unroll
+    for (int i = 0; i < kEarly; ++i) {
+      const int64_t seg = wave + static_cast<int64_t>(i) * kFinishWaves;
+#pragma unroll
+      for (int d = 0; d < kDeep; ++d)
+        early[i][d] = slots[(seg < n ? seg : 0) * kSegSlots + d * kWave + lane];
+    }
+  }
+  const RowRequest q = row_request(A, r);
+  const int64_t vocab = A.vocab;
+  const T* __restrict__ row = reinterpret_cast<const T*>(A.logits) + r * vocab;
+  const float lt = L::widen(row[q.in_range ? q.token : (q.token < 0 ? 0 : vocab - 1)]);
+  const bool cut = q.want_mass && q.use_kth;  // uniform
+
+  // f(header) for each of this lane's segments
+  auto headers = [&](auto&& f) {
+    if (own < n) f(mine_h);
+    for (int64_t i = own + kFinishThreads; i < n; i += kFinishThreads) f(hs[i]);
+  };
+  uint32_t above32 = 0;  // at most vocab in all, below 2^31
+  int flags = 0;
+  float m = -inf, low = -inf;
+  headers([&](const SegmentHeader& h) {
+    above32 += h.above;
+    flags |= h.flags | (h.count > kSegSlots ? 2 : 0) | (h.count > kDeep * kWave ? 4 : 0);
+    m = fmaxf(m, h.max);
+    low = fmaxf(low, h.low);
+  });
+  const auto add = [](uint32_t u, uint32_t v) { return u + v; };
+  const auto larger = [](float u, float v) { return fmaxf(u, v); };
+  float wave_kth = -inf;
+  if (cut) {
+    float top = -inf;
+#pragma unroll
+    for (int i = 0; i < kEarly; ++i) {
+      const int count = static_cast<int>(read_lane(mine_h.count, i));  // 0 past the row
+#pragma unroll
+      for (int d = 0; d < kDeep; ++d) {
+        if (d * kWave + lane >= count) early[i][d] = -inf;
+        top = fmaxf(top, early[i][d]);
+      }
+    }
+    wave_kth = wave_bound(top, static_cast<int>((q.k_eff + kFinishWaves - 1) / kFinishWaves));
+  }
+  {
+    const uint32_t wave_above = wave_reduce(above32, add);
+    const uint32_t wave_flags =
+        wave_reduce(static_cast<uint32_t>(flags), [](uint32_t u, uint32_t v) { return u | v; });
+    const float wave_max = wave_reduce(m, larger);
+    const float wave_low = wave_reduce(low, larger);
+    if (lane == 0) {
+      s.above[wave] = wave_above;
+      s.flags[wave] = static_cast<int>(wave_flags);
+      s.max[wave] = wave_max;
+      s.low[wave] = wave_low;
+      s.kth[wave] = wave_kth;
+    }
+  }
+  s.hist[0][t] = 0;  // for a radix select below, behind the barriers between
+  __syncthreads();
+  int64_t above = 0;
+  flags = 0;
+  m = -inf;
+  float floor_value = -inf, every_wave = inf;
+#pragma unroll
+  for (int w = 0; w < kFinishWaves; ++w) {
+    above += s.above[w];
+    flags |= s.flags[w];
+    m = fmaxf(m, s.max[w]);
+    floor_value = fmaxf(floor_value, s.low[w]);
+    every_wave = fminf(every_wave, s.kth[w]);
+  }
+  floor_value = fmaxf(floor_value, every_wave);  // G
+
+  double z = 0.0, a = 0.0;
+  auto term = [&](float l, float kth) {
+    if (l >= kth) {
+      const float e = split_term(l, m);
+      z += e;
+      a += l > lt ? e : 0.0;
+    }
+  };
+  bool one_wave = !q.want_mass;  // wave 0 holds the row's sums
+  if (cut) {
+    bool whole_row = flags & 2;
+    if (!whole_row) {
+      // This wave's slots above G and its logits equal to G (ties): counted, then compacted at
+      // the wave's offset, in segment and slot order.  A segment whose low is G has its ties in
+      // its header (its slots are all above G); one whose low is below G has them in its slots.
+      const bool more = (flags & 4) || n > static_cast<int64_t>(kEarly) * kFinishWaves;
+      auto each = [&](auto&& f) {  // f(value) by whole waves, -inf where there is no slot
+#pragma unroll
+        for (int i = 0; i < kEarly; ++i)
+#pragma unroll
+          for (int d = 0; d < kDeep; ++d) f(early[i][d]);
+        if (more) {
+          for (int64_t seg = wave, i = 0; seg < n; seg += kFinishWaves, ++i) {
+            const int count = static_cast<int>(
+                i < kWave ? read_lane(mine_h.count, static_cast<int>(i)) : hs[seg].count);
+            for (int j = i < kEarly ? kDeep * kWave : 0; j < count; j += kWave) {
+              const float v = slots[seg * kSegSlots + (j + lane < count ? j + lane : count - 1)];
+              f(j + lane < count ? v : -inf);
+            }
+          }
+        }
+      };
+      uint32_t mine = 0, ties = 0;
+      each([&](float v) {
+        mine += v > floor_value;
+        ties += v == floor_value;
+      });
+      headers([&](const SegmentHeader& h) { ties += h.low == floor_value ? h.ties : 0u; });
+      const uint32_t wave_n = wave_reduce(mine, add);
+      const uint32_t wave_ties = wave_reduce(ties, add);
+      if (lane == 0) {
+        s.count[wave] = wave_n;
+        s.ties[wave] = wave_ties;
+      }
+      __syncthreads();
+      uint32_t total = 0, tied = 0, at = 0;
+#pragma unroll
+      for (int w = 0; w < kFinishWaves; ++w) {
+        at = w == wave ? total : at;
+        total += s.count[w];
+        tied += s.ties[w];
+      }
+      whole_row = total > static_cast<uint32_t>(kCap);
+      if (!whole_row) {
+        each([&](float v) {
+          const bool take = v > floor_value;
+          const uint64_t want = __ballot(take);
+          if (take) {
+            const uint64_t below = lane ? want & (~0ull >> (kWave - lane)) : 0ull;
+            s.cand[at + __builtin_popcountll(below)] = v;
+          }
+          at += __builtin_popcountll(want);
+        });
+        __syncthreads();
+        const bool select = static_cast<int64_t>(total) >= q.k_eff;  // kth exceeds G
+        if (!select && t == 0) {
+          z = static_cast<double>(split_term(floor_value, m)) * tied;
+          a = floor_value > lt ? z : 0.0;
+        }
+        if (total <= kHeld * kWave) {
+          // Wave 0 alone, with no further barrier: the candidates in its registers, kth bit by
+          // bit from the first bit in which G and the maximum differ, until exactly k_eff of
+          // them reach the bound (kth is then the smallest of those) or no bit is left.
+          if (wave != 0) return;
+          one_wave = true;
+          float c[kHeld];
+          uint32_t key[kHeld];
+#pragma unroll
+          for (int i = 0; i < kHeld; ++i) {
+            const uint32_t j = lane + i * kWave;
+            const float v = s.cand[j < total ? j : 0];
+            c[i] = j < total ? v : -inf;
+            key[i] = j < total ? order_key(v) : 0u;
+          }
+          float kth = floor_value;
+          if (select) {
+            const uint32_t hi = order_key(m), lo = order_key(floor_value);
+            const uint32_t diff = hi ^ lo;  // hi > lo: some logit exceeds G
+            int bit = 31 - __builtin_clz(diff | 1u);
+            uint32_t bound = bit == 31 ? 0u : (hi >> (bit + 1)) << (bit + 1);
+            for (; bit >= 0; --bit) {
+              const uint32_t trial = bound | (1u << bit);
+              int count = 0;
+#pragma unroll
+              for (int i = 0; i < kHeld; ++i)
+                count += __builtin_popcountll(__ballot(key[i] >= trial));
+              if (count >= q.k_eff) bound = trial;
+              if (count == q.k_eff) break;
+            }
+            uint32_t least = 0xFFFFFFFFu;
+#pragma unroll
+            for (int i = 0; i < kHeld; ++i)
+              if (key[i] >= bound && key[i] < least) least = key[i];
+            kth = key_value(wave_reduce(least, [](uint32_t u, uint32_t v) { return u < v ? u : v; }));
+          }
+#pragma unroll
+          for (int i = 0; i < kHeld; ++i)
+            if (c[i] > floor_value) term(c[i], kth);
+        } else {
+          float kth = floor_value;
+          if (select) {
+            kth = key_value(radix_select(q.k_eff, [&](auto&& f) {
+              for (uint32_t i = t; i < total; i += kFinishThreads) f(order_key(s.cand[i]));
+            }, s));
+          }
+          for (uint32_t i = t; i < total; i += kFinishThreads) term(s.cand[i], kth);
+        }
+      }
+    }
+    if (whole_row) {
+      // f(logit) for the row's logits, kAhead in flight per lane
+      constexpr int kAhead = 8;
+      auto logits = [&](auto&& f) {
+        for (int64_t i = t; i < vocab; i += kAhead * kFinishThreads) {
+          float v[kAhead];
+#pragma unroll
+          for (int e = 0; e < kAhead; ++e) {
+            const int64_t j = i + e * kFinishThreads;
+            v[e] = L::widen(row[j < vocab ? j : vocab - 1]);
+          }
+#pragma unroll
+          for (int e = 0; e < kAhead; ++e)
+            if (i + e * kFinishThreads < vocab) f(v[e]);
+        }
+      };
+      const float kth = key_value(radix_select(
+          q.k_eff, [&](auto&& f) { logits([&](float l) { f(order_key(l)); }); }, s));
+      logits([&](float l) { term(l, kth); });
+    }
+  } else if (q.want_mass) {
+    headers([&](const SegmentHeader& h) {
+      if (h.max > -inf) {
+        const double scale = exp(static_cast<double>(h.max) - static_cast<double>(m));
+        z += h.z * scale;
+        a += h.a * scale;
+      }
+    });
+  }
+  if (q.want_mass) {
+    const auto sum = [](double u, double v) { return u + v; };
+    z = wave_reduce(z, sum);
+    a = wave_reduce(a, sum);
+    if (!one_wave) {
+      if (lane == 0) {
+        s.z[wave] = z;
+        s.a[wave] = a;
+      }
+      __syncthreads();
+      z = (s.z[0] + s.z[1]) + (s.z[2] + s.z[3]);
+      a = (s.a[0] + s.a[1]) + (s.a[2] + s.a[3]);
+    }
+  }
+  if (t == 0) write_verdict(A, r, q, above, flags & 1, z, a);
 }
 
 }  // namespace
 }  // namespace pck
 
-extern "C" int pck_check_members_ex(const PckMemberArgs* args, void* stream) {
+namespace pck {
+namespace {
+
+hipError_t validate(const PckMemberArgs* args) {
   if (args == nullptr) return hipErrorInvalidValue;
   const PckMemberArgs& a = *args;
-  if (a.rows < 0 || a.rows * pck::kThreads > 0xFFFFFFFFll || a.vocab < 1 ||
-      a.vocab > 0x7FFFFFFF || a.k_lim < 0 || a.k_lim > a.vocab)
+  if (a.rows < 0 || a.rows * kThreads > 0xFFFFFFFFll || a.vocab < 1 || a.vocab > 0x7FFFFFFF ||
+      a.k_lim < 0 || a.k_lim > a.vocab)
     return hipErrorInvalidValue;
   if (a.rows == 0) return hipSuccess;
   if (!a.logits || !a.tokens ||
-      (a.temperature && (!a.temperature_index || a.temperature_count < 1)))
+      (a.temperature && (!a.temperature_index || a.temperature_count < 1)) ||
+      (a.all_k && a.k_lim < 1))
     return hipErrorInvalidValue;
-  if (a.all_k && a.k_lim < 1) return hipErrorInvalidValue;
+  return hipSuccess;
+}
+
+// The split of a batch: logits per segment, segments per row and the workspace (0 bytes: the
+// one-workgroup kernel).  FP32 rows split where that is faster; 16-bit logits always do, since
+// the one-workgroup kernel would need them converted first.  Measured on 151,936 logits a row,
+// one workgroup against split (us; top-k 50 + top-p / top-p only / top-k only):
+//   1 row     21.5 / 10.7    38.8 / 6.2     11.2 / 5.0
+//   64 rows   25.8 / 17.3    44.4 / 17.6    15.7 / 11.6
+//   128 rows  29.3 / 23.9    48.0 / 25.8    18.5 / 17.2
+//   256 rows  34.0 / 36.4    62.2 / 46.1    28.4 / 28.8
+// A row that keeps everything is read once instead of twice at any batch size; the others gain
+// while the rows leave compute units idle.  Short rows (16,384 logits: 9.8 / 10.6, 7.7 / 6.7 us)
+// lose to the second launch first where a k-th logit is selected.
+// Segments are 8,192 logits (their candidates are what the finish reads), shorter ones only
+// where no row is cut and the batch would not fill the GPU.
+struct SplitPlan {
+  int64_t length = 0, segments = 0, header_bytes = 0, bytes = 0;
+};
+
+SplitPlan split_plan(const PckMemberArgs& a, int kind) {
+  SplitPlan p;
+  if (a.rows < 1) return p;
+  const bool cut = a.top_p != nullptr && a.k_lim > 0;     // a row may be cut at its k-th logit
+  const bool keeps_all = a.top_p != nullptr && !a.all_k;  // a row may keep every logit
+  if (kind == 0 && !(keeps_all ? a.vocab >= 16384 : a.vocab >= 24576 && a.rows < 192)) return p;
+  int64_t length = 8192;
+  while (!cut && length > 2048 && a.rows * ((a.vocab + length - 1) / length) < 1024) length /= 2;
+  const int64_t segments = (a.vocab + length - 1) / length;
+  // about 1.4 k candidates of each segment reach the finish workgroup, which holds kCap
+  if (cut && (a.k_lim > kSplitMaxK || segments * a.k_lim > kCap * 5 / 8)) return p;
+  if (a.rows * segments > 0x7FFFFFFF / kSegThreads) return p;
+  p.length = length;
+  p.segments = segments;
+  p.header_bytes = a.rows * segments * static_cast<int64_t>(sizeof(SegmentHeader));
+  p.bytes = p.header_bytes +
+            (cut ? a.rows * segments * kSegSlots * static_cast<int64_t>(sizeof(float)) : 0);
+  return p;
+}
+
+template <Logits kType>
+hipError_t launch_split(const SplitArgs& s, hipStream_t stream) {
+  constexpr int kVec = kType == Logits::kF32 ? 4 : 8;
+  constexpr int kUnit = kSegThreads * kVec;  // logits per load of the workgroup
+  const dim3 grid(static_cast<unsigned>(s.m.rows * s.segments)), group(kSegThreads);
+  if (s.length == 8192)
+    member_segment_kernel<kType, 8192 / kUnit><<<grid, group, 0, stream>>>(s);
+  else if (s.length == 4096)
+    member_segment_kernel<kType, 4096 / kUnit><<<grid, group, 0, stream>>>(s);
+  else
+    member_segment_kernel<kType, 2048 / kUnit><<<grid, group, 0, stream>>>(s);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  member_finish_kernel<kType>
+      <<<dim3(static_cast<unsigned>(s.m.rows)), dim3(kFinishThreads), 0, stream>>>(s);
+  return hipGetLastError();
+}
+
+}  // namespace
+}  // namespace pck
+
+extern "C" int pck_check_members_workspace(const PckMemberArgs* args, int logits_kind,
+                                           int64_t* bytes) {
+  if (pck::validate(args) != hipSuccess || logits_kind < 0 || logits_kind > 2 || bytes == nullptr)
+    return hipErrorInvalidValue;
+  *bytes = pck::split_plan(*args, logits_kind).bytes;
+  return hipSuccess;
+}
+
+extern "C" int pck_check_members_split(const PckMemberArgs* args, int logits_kind, void* workspace,
+                                       int64_t workspace_bytes, void* stream) {
+  using namespace pck;
+  if (validate(args) != hipSuccess || logits_kind < 0 || logits_kind > 2)
+    return hipErrorInvalidValue;
+  if (args->rows == 0) return hipSuccess;
+  const SplitPlan p = split_plan(*args, logits_kind);
+  if (p.bytes == 0 || workspace == nullptr || workspace_bytes < p.bytes ||
+      reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+    return hipErrorInvalidValue;
+  const SplitArgs s{*args, static_cast<SegmentHeader*>(workspace),
+                    reinterpret_cast<float*>(static_cast<char*>(workspace) + p.header_bytes),
+                    p.segments, p.length};
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (logits_kind == 0) return launch_split<Logits::kF32>(s, st);
+  if (logits_kind == 1) return launch_split<Logits::kBf16>(s, st);
+  return launch_split<Logits::kF16>(s, st);
+}
+
+extern "C" int pck_check_members_ex(const PckMemberArgs* args, void* stream) {
+  if (pck::validate(args) != hipSuccess) return hipErrorInvalidValue;
+  const PckMemberArgs& a = *args;
+  if (a.rows == 0) return hipSuccess;
   pck::member_kernel<<<dim3(static_cast<unsigned>(a.rows)), dim3(pck::kThreads), 0,
                        static_cast<hipStream_t>(stream)>>>(a);
   return hipGetLastError();

@@ -163,6 +163,8 @@ SIGNATURES: dict[str, list[Any]] = {
         _p, _i64, _i64, _p, _p, _p, _p, _f64, _i64, _int, _p, _p, _p, _p,
     ],  # fmt: skip
     "pck_check_members_ex": [ctypes.POINTER(PckMemberArgs), _p],
+    "pck_check_members_workspace": [ctypes.POINTER(PckMemberArgs), _int, ctypes.POINTER(_i64)],
+    "pck_check_members_split": [ctypes.POINTER(PckMemberArgs), _int, _p, _i64, _p],
     "pck_sampling_check": [
         _p, _p, _p, _i64, _i64, _i64, _i64, _int, _f64, _f64, _f64, _i64,
         _p, _p, _p, _p, _p, _p, _p, _p,

@@ -9,8 +9,8 @@ For a row of logits ``l``, the sampled token ``t`` and the request's ``top_k`` /
   greedy  accept iff no logit is strictly larger than ``l[t]``;
   NaN logits or an id outside [0, V) reject.
 
-`check_members` runs the whole batch in one launch of the HIP kernel (`pck_check_members_ex`:
-exact FP32 comparisons, FP32 softmax terms on an exact split argument, FP64 sums); it needs the
+`check_members` runs the whole batch in one or two launches (`pck_check_members_ex`,
+`pck_check_members_split`: exact FP32 comparisons, FP32 softmax terms on an exact split argument, FP64 sums); it needs the
 logits on the GPU, and `launch_check` also keeps running totals on the device.  `check_member`
 is the reference's FP64 check of one row on the CPU.  `member_eps` / `member_eps32` are the
 error bounds the slack is built from (reference `src/pck/member.py:37-41,84-102`).
@@ -18,6 +18,7 @@ error bounds the slack is built from (reference `src/pck/member.py:37-41,84-102`
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 from typing import Any
@@ -144,7 +145,9 @@ def launch_check(
     totals: Any = None,
     outputs: bool = True,
 ) -> dict[str, Any] | None:
-    """One launch of the membership kernel (`pck_check_members_ex`) over a batch.
+    """The membership kernel over a batch: one launch (`pck_check_members_ex`), or two with the
+    rows split over workgroups where that is faster or the logits are of a 16-bit type
+    (`pck_check_members_split`).
 
     Beside `check_members`'s arguments: ``temperature`` (requests,) FP32 with
     ``temperature_index`` (B,) makes row r greedy iff temperature[index[r]] == 0 (instead of
@@ -156,13 +159,15 @@ def launch_check(
 
     from pck.cuda._lib import PckMemberArgs, check, lib, stream_handle
 
+    kinds = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
     if not logits.is_cuda:
         raise RuntimeError(
             "check_members runs the HIP membership kernel and needs logits on the GPU, "
             f"got {logits.device}"
         )
     device = logits.device
-    lv = logits.float().contiguous()
+    kind = kinds.get(logits.dtype, 0)
+    lv = (logits if logits.dtype in kinds else logits.float()).contiguous()
     if lv.dim() != 2:
         raise RuntimeError(f"expected logits of shape (B, V), got {list(lv.shape)}")
     rows, vocab = lv.shape
@@ -219,8 +224,19 @@ def launch_check(
     if rows == 0:
         return out
     a.slack = next_up(tol + member_eps32(vocab))
+    handle = lib()
+    need = ctypes.c_int64(0)
+    check(handle.pck_check_members_workspace(a, kind, ctypes.byref(need)), "membership check plan")
     with torch.cuda.device(device):
-        err = lib().pck_check_members_ex(a, stream_handle(device))
+        if need.value:  # rows split over workgroups, read in the logits' own type
+            work = torch.empty(need.value, dtype=torch.uint8, device=device)
+            err = handle.pck_check_members_split(
+                a, kind, work.data_ptr(), need.value, stream_handle(device)
+            )
+        else:  # one workgroup per row of FP32 logits
+            lv = lv.float()
+            a.logits = lv.data_ptr()
+            err = handle.pck_check_members_ex(a, stream_handle(device))
     check(err, "membership check launch")
     return out
 

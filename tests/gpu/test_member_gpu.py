@@ -259,3 +259,51 @@ def test_request_index_outside_the_temperature_array_rejects_the_row() -> None:
     out = launch_check(logits, tokens, temperature=temperature, temperature_index=bad, totals=totals)
     assert out["ok"].tolist() == [True, True, False, True, True, False, True, True]
     assert int(totals[0]) == rows and int(totals[1]) == 2
+
+
+SPLIT_CASES = ["plain", "ties", "masked", "all_masked", "nan", "sorted", "overflow", "mixed"]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("vocab", [24576, 24577, 32003, 151_937])
+@pytest.mark.parametrize("case", SPLIT_CASES)
+def test_rows_split_over_workgroups_match_the_oracle(case: str, vocab: int, dtype: torch.dtype) -> None:
+    """Whole and partial last segments, rows at any 2- or 4-byte address, 16-bit logits read as
+    they are; ties at the k-th logit, masked (-inf) rows, NaN, a row sorted within its segments,
+    and segments with more logits above their bound than slots (one wave's logits all low), which
+    takes the whole-row select.  Top-k 1, 50, 128 and none, with top-p; then top-k alone."""
+    rng = np.random.default_rng(vocab + len(case))
+    rows = 6
+    logits = rng.standard_normal((rows, vocab)) * 3
+    logits[np.arange(rows)[:, None], rng.integers(0, vocab, (rows, 6))] += 9.0
+    if case == "ties":
+        logits[:, 100:400] = np.sort(logits, axis=1)[:, -20:-19]
+    elif case in ("masked", "all_masked"):
+        keep = rng.random((rows, vocab)) < (0.001 if case == "masked" else 0.0)
+        keep[:, rng.integers(0, vocab, 3)] |= case == "masked"
+        logits[~keep] = -np.inf
+        if case == "all_masked":
+            logits[:, 7] = 1.0
+    elif case == "nan":
+        logits[::2, vocab - 1] = np.nan
+    elif case == "sorted":
+        logits[:] = 5.0 - (np.arange(vocab) % 8192) * 2.0**-9 + np.arange(rows)[:, None]
+    elif case == "overflow":
+        logits[:, np.arange(vocab) % 1024 >= 768] = -50.0
+    t = torch.from_numpy(logits).to(dtype)
+    host = t.float().numpy()
+    order = np.argsort(-np.nan_to_num(host, nan=-1e30), axis=1, kind="stable")
+    top_k = np.array([1, 50, 128, 50, 7, vocab] if case == "mixed" else [1, 50, 128, 50, 7, 20])
+    tokens = order[np.arange(rows), [0, 3, 90, 60, 2, 5]]
+    top_p = np.array([0.9, 0.5, 0.999, 0.9, 1.0, 0.9])
+    dev = lambda a: None if a is None else torch.as_tensor(a).cuda()  # noqa: E731
+    for k, p in ((top_k, top_p), (None, top_p), (top_k, None)):
+        out = check_members(t.cuda(), dev(tokens), dev(k), dev(p), top_k_host=k)
+        got = {name: v.cpu().numpy() for name, v in out.items()}
+        want = check_members_ref(host, tokens, k, p, None, top_k_host=k)
+        np.testing.assert_array_equal(got["ok"], want["ok"])
+        np.testing.assert_array_equal(got["above"], want["above"])
+        if p is not None:
+            finite = np.isfinite(want["mass_above"]) & ~np.isnan(host).any(axis=1)
+            err = np.abs(got["mass_above"] - want["mass_above"])[finite]
+            assert np.all(err <= 2 * member_eps32(vocab))
