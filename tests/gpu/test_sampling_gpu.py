@@ -233,3 +233,35 @@ def test_native_entry_takes_the_pybind_sampling_arguments() -> None:
     assert len(out) == 5 and bool(out[0].all())
     assert torch.equal(out[0], ref.passed) and torch.equal(out[1], ref.min_selected)
     assert torch.equal(out[2], ref.max_rejected)
+
+
+@pytest.mark.parametrize("vocab", [2, 4, 5, 5119, 5121, 10_243, 25_601])
+@pytest.mark.parametrize("segments", [1, 2, 3])
+@pytest.mark.parametrize("temp", [1.0, 0.7, 1e-42, 1e30])
+def test_chunks_of_a_segment_match_cpu(vocab: int, segments: int, temp: float) -> None:
+    """Segments around the 5,120 logits of one chunk, with a partial last quad, one to five
+    chunks, rows at any 4-byte address, maxima that rise from chunk to chunk, and temperatures
+    of each way the quotient is formed (T = 1, two floats, FP64)."""
+    segments = min(segments, vocab)
+    lg = logits(3, vocab, seed=vocab, scale=2.0) + torch.arange(vocab, device="cuda") / vocab
+    if temp == 1e-42:
+        lg = torch.round(lg)  # ties carry the mass: e^0 for the maximum, 0 for the rest
+    p = 0.8
+    # the smallest sets of the FP64 softmax, in descending order
+    selected = torch.sort(lg.double(), dim=1, descending=True, stable=True).indices.contiguous()
+    probs = [softmax64(row.cpu().numpy(), temp) for row in lg]
+    cum = [np.cumsum(pr[s.cpu().numpy()]) for pr, s in zip(probs, selected)]
+    lengths = torch.tensor([int(np.searchsorted(c, p)) + 1 for c in cum], device="cuda")
+    res = check_topp_gpu(lg, selected, lengths, p, temp, tol=1e-5, segments=segments)
+    for b in range(3):
+        sel = selected[b, : lengths[b]].cpu().numpy()
+        mass = float(probs[b][sel].sum())
+        zmax = float(np.abs(lg[b].cpu().numpy() / temp).max()) if temp > 1e-3 else 0.0
+        bound = 2 * topp_slack(vocab, segments, 0.0) + softmax_eps(vocab, zmax)
+        assert abs(float(res.mass[b]) - mass) <= bound
+    assert res.passed.all()
+    topk = check_topk_gpu(lg, selected[:, : vocab // 2].contiguous(), vocab // 2, segments=segments)
+    assert topk.passed.all()
+    bad = selected[:, 1 : vocab // 2 + 1].contiguous()  # the maximum left out
+    want = [bool(lg[b][bad[b]].min() >= lg[b].max()) for b in range(3)]  # all tied only
+    assert check_topk_gpu(lg, bad, vocab // 2, segments=segments).passed.tolist() == want
