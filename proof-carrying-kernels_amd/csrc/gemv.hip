@@ -198,6 +198,8 @@ __device__ __forceinline__ float lane_value(float v, int lane) {
 //   kElement    element loads: rows shorter than one vector.
 enum class Load { kElement, kUnaligned, kAligned };
 
+enum class Pad { kNone, kZeroed, kSkipped };
+
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4_any __attribute__((aligned(1)));  // any byte address
 
@@ -249,17 +251,21 @@ __device__ __forceinline__ void drop_front_x(uint4& xa, uint4& xb, int skip) {
 
 // T virtual lanes per row, R rows per wave slot, U vector positions loaded ahead, kNt:
 // non-temporal weight loads (streamed once, so they need not displace x in the caches).
-// kPad: some vectors of a chain lie past n (n is not a multiple of T * vec); their loads are
-// redirected to column 0 (kUnaligned: to the row's last vector) and they add +0.  A chain slot
-// whose 64 vectors all lie past n adds +0 once instead of V products of zeros (the same sum,
-// sign of zero included), so a row's short last position costs what its columns cost.
-
+// kPad: what a launch does about vectors of a chain that lie past n (n is not a multiple of
+// T * vec); their loads are redirected to column 0 (kUnaligned: to the row's last vector) and
+// they add +0.
+//   kNone     there are none.
+//   kZeroed   they are zeroed in the registers they were loaded to.
+//   kSkipped  a chain slot whose 64 vectors all lie past n adds +0 once instead of V products of
+//             zeros (the same sum, sign of zero included), so a row's short last position costs
+//             what its columns cost (FP8 4096 x 14336: 12.4 against 14.2 us).  Its branches cost
+//             rows without such a slot 3 to 10%, so a launch takes this form only if it has one.
 //
 // kLive: chain slots per lane that hold any column, when every row of the launch ends inside the
 // first kLive slots of its first position (n <= 64 kLive vec, one position).  The other slots'
 // chains sum padding only, so they are +0 without being loaded or kept in registers: a tree of
 // 512 or 1024 virtual lanes over a short row then costs what the row's own columns cost.
-template <int T, int R, int U, bool kFp8, Load kLoad, bool kPad, bool kNt, bool kSums = false,
+template <int T, int R, int U, bool kFp8, Load kLoad, Pad kPad, bool kNt, bool kSums = false,
           int kLive = (T >= kWave ? T / kWave : 1)>
 __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group) {
   constexpr int V = kFp8 ? 16 : 8;
@@ -308,6 +314,7 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
   RowSums rs[R][kLive];  // per row and chain: the lane's d and s (kSums only)
 
   constexpr bool kAny = kLoad == Load::kUnaligned;
+  constexpr bool kZeroed = kPad == Pad::kZeroed && !kAny;
   for (int64_t v0 = 0; v0 < P; v0 += U) {
     if constexpr (kLoad != Load::kElement) {
       uint4 wb[U][R][kLive];
@@ -319,47 +326,61 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
 #pragma unroll
         for (int j = 0; j < kLive; ++j) {
           const int64_t col = ((v0 + u) * T + chain0 + kLanesPerRow * j) * V;
-          const int64_t at = !kPad ? col : kAny ? (col < n - V ? col : n - V) : (col < n ? col : 0);
+          const int64_t at = kPad == Pad::kNone ? col : kAny ? (col < n - V ? col : n - V) : (col < n ? col : 0);
           xa[u][j] = load16<false, kAny>(x + at);
           if constexpr (kFp8) xb[u][j] = load16<false, kAny>(x + at + 8);
 #pragma unroll
           for (int r = 0; r < R; ++r)
             wb[u][r][j] = load16<kNt, kAny>(w_rows[r] + at * kElemBytes);
+          if constexpr (kZeroed) {
+            if (col >= n) {
+              xa[u][j] = make_uint4(0, 0, 0, 0);
+              xb[u][j] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+              for (int r = 0; r < R; ++r) wb[u][r][j] = make_uint4(0, 0, 0, 0);
+            }
+          }
         }
       }
+      auto products = [&](int u, int j) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          add_products<kFp8, kSums>(acc[r][j], rs[r][j], wb[u][r][j], xa[u][j],
+                                    kFp8 ? xb[u][j] : xa[u][j]);
+      };
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (U > 1 && v0 + u >= P) break;
+        if (kPad == Pad::kNone || kZeroed || (v0 + u + 1) * T * V <= n) {  // nothing to drop
+#pragma unroll
+          for (int j = 0; j < kLive; ++j) products(u, j);
+          continue;
+        }
 #pragma unroll
         for (int j = 0; j < kLive; ++j) {
-          if constexpr (kPad) {
-            // the slot's first column, the same for every lane of the wave
-            const int64_t first = ((v0 + u) * T + kLanesPerRow * j) * V;
-            if (first >= n) {
+          // the slot's first column, the same for every lane of the wave
+          const int64_t first = ((v0 + u) * T + kLanesPerRow * j) * V;
+          if (first >= n) {
 #pragma unroll
-              for (int r = 0; r < R; ++r) acc[r][j] = acc[r][j] + 0.0f;
-              continue;
-            }
-            if (first + kLanesPerRow * V > n) {  // some of the slot's columns lie past n
-              const int64_t col = first + chain0 * V;
-              if constexpr (kAny) {
-                const int64_t over = col - (n - V);  // <= 0: a whole vector
-                const int skip = over <= 0 ? 0 : over < V ? static_cast<int>(over) : V;
-                drop_front_x<kFp8>(xa[u][j], xb[u][j], skip);
+            for (int r = 0; r < R; ++r) acc[r][j] = acc[r][j] + 0.0f;
+            continue;
+          }
+          if (first + kLanesPerRow * V > n) {  // some of the slot's columns lie past n
+            const int64_t col = first + chain0 * V;
+            if constexpr (kAny) {
+              const int64_t over = col - (n - V);  // <= 0: a whole vector
+              const int skip = over <= 0 ? 0 : over < V ? static_cast<int>(over) : V;
+              drop_front_x<kFp8>(xa[u][j], xb[u][j], skip);
 #pragma unroll
-                for (int r = 0; r < R; ++r) drop_front<kFp8>(wb[u][r][j], skip);
-              } else if (col >= n) {
-                xa[u][j] = make_uint4(0, 0, 0, 0);
-                xb[u][j] = make_uint4(0, 0, 0, 0);
+              for (int r = 0; r < R; ++r) drop_front<kFp8>(wb[u][r][j], skip);
+            } else if (col >= n) {
+              xa[u][j] = make_uint4(0, 0, 0, 0);
+              xb[u][j] = make_uint4(0, 0, 0, 0);
 #pragma unroll
-                for (int r = 0; r < R; ++r) wb[u][r][j] = make_uint4(0, 0, 0, 0);
-              }
+              for (int r = 0; r < R; ++r) wb[u][r][j] = make_uint4(0, 0, 0, 0);
             }
           }
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-            add_products<kFp8, kSums>(acc[r][j], rs[r][j], wb[u][r][j], xa[u][j],
-                                      kFp8 ? xb[u][j] : xa[u][j]);
+          products(u, j);
         }
       }
     } else {
@@ -433,7 +454,7 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
   }
 }
 
-template <int T, int R, int U, bool kFp8, Load kLoad, bool kPad, bool kNt, int kLive>
+template <int T, int R, int U, bool kFp8, Load kLoad, Pad kPad, bool kNt, int kLive>
 __global__ void __launch_bounds__(kGroupThreads) gemv_tree_kernel(const GemvBatch batch) {
   gemv_rows<T, R, U, kFp8, kLoad, kPad, kNt, false, kLive>(batch, blockIdx.x);
 }
@@ -447,7 +468,7 @@ __global__ void __launch_bounds__(kGroupThreads) gemv_tree_kernel(const GemvBatc
 // Rows longer than 4,096 columns keep 8 quads per lane in flight (a 14,336-column row in two
 // round trips instead of four); more would push the kernel past 128 VGPRs and halve the GEMV
 // waves a SIMD holds.
-template <int T, int R, int U, bool kFp8, bool kPad, bool kNt>
+template <int T, int R, int U, bool kFp8, Pad kPad, bool kNt>
 __global__ void __launch_bounds__(kGroupThreads)
     gemv_ride_kernel(const GemvBatch batch, const PckCheckBatch ride) {
   __shared__ check::Quad lds[check::kWaves];
@@ -468,7 +489,7 @@ __global__ void __launch_bounds__(kGroupThreads)
 // workgroups of the grid the row-sum checks of `ride` (outputs of earlier launches on the stream,
 // read from memory; one wave per (check, block) pair, the code of pck_rowsum_check, so the
 // results are bit-identical to it).  A check never reads anything this launch writes.
-template <int T, int R, int U, bool kFp8, Load kLoad, bool kPad, bool kNt, int kLive>
+template <int T, int R, int U, bool kFp8, Load kLoad, Pad kPad, bool kNt, int kLive>
 __global__ void __launch_bounds__(kGroupThreads)
     gemv_rowsum_kernel(const GemvBatch batch, const PckRowSumBatch ride) {
   const int64_t items = rowsum::items(ride);
@@ -579,18 +600,35 @@ struct TreeShape {
 
 TreeShape g_shape_override = {0, 0, 0};
 
-// Defaults from sweeps of every shape over each Llama-3-8B decode launch on MI355X.  BF16:
-// non-temporal weight loads won everywhere.  FP8 rows are half as long, so two rows per wave
-// keep as many bytes in flight as one BF16 row, except for a launch of at most 4096 rows (o),
-// where one row per wave and two positions ahead give twice the waves (4.9 against 5.4 us).
-// The sweeps replay each launch over weight copies that do not fit the Infinity Cache (with
-// four copies of FP8 down, 235 MB, plain loads won from the cache; streamed from HBM, as in a
-// decode pass, non-temporal loads take 12.5 against 14.6 us).
+// Defaults from sweeps of every shape over Llama-3-8B decode launches and over 1024 .. 4096 rows of
+// 4096 .. 14336 columns on MI355X.  Non-temporal weight loads won everywhere; the sweeps replay
+// each launch over weight copies that do not fit the Infinity Cache (with four copies of FP8
+// down, 235 MB, plain loads won from the cache; streamed from HBM, as in a decode pass,
+// non-temporal loads take 12.4 against 14.6 us).  per_lane is the positions of the longest row.
+//   BF16, one or two positions (n <= 4096): one row per wave, both positions ahead.
+//   BF16, longer rows: two rows per wave above 3072 rows; fewer rows leave too few waves, so one
+//     row, and below 1536 rows two positions ahead as well (2304 x 13824: 13.7 against 16.9 us
+//     with two rows, 3573 x 13824: 20.2 against 19.2; 1024 x 14336: 8.5 against 11.4).
+//   FP8 rows are half as long, so two rows per wave keep as many bytes in flight as one BF16 row;
+//     one row per wave below 2048 rows (1024 x 14336: 6.8 against 8.6 us), for rows of one
+//     position up to 4096 rows (o: 4.9 against 5.4 us) and of two up to 3072.
 TreeShape choose_shape(int64_t per_lane, int64_t rows, bool fp8) {
   if (g_shape_override.rows > 0) return g_shape_override;
-  if (fp8) return per_lane <= 2 && rows <= 4096 ? TreeShape{1, 2, 1} : TreeShape{2, 1, 1};
-  return per_lane > 2 ? TreeShape{2, 2, 1} : TreeShape{1, 2, 1};
+  if (!fp8) {
+    if (per_lane <= 2 || rows < 1536) return TreeShape{1, 2, 1};
+    return rows <= 3072 ? TreeShape{1, 1, 1} : TreeShape{2, 1, 1};
+  }
+  if (per_lane == 1 && rows <= 4096) return TreeShape{1, 2, 1};
+  if (rows < 2048 || (per_lane == 2 && rows <= 3072)) return TreeShape{1, 1, 1};
+  return TreeShape{2, 1, 1};
 }
+
+// Trees of T != 256 lanes read aligned weights with plain loads where a launch's weights may
+// still be in the 256 MB Infinity Cache at the next call on them (below a third of it, as when one matrix
+// is evaluated again and again: 2653 x 11376, T = 512, three copies in turn, 14.0 against 15.8
+// us), and with non-temporal ones above (14336 x 4096, T = 512, from HBM: 20.0 against 21.8).
+// T = 256 is the decode path, which streams its weights: non-temporal.
+constexpr int64_t kCachedBytes = int64_t{85} << 20;
 
 // Fills the workgroup prefix sums for rows_per_group rows per workgroup; returns the total.
 int64_t plan_groups(GemvBatch& batch, int64_t rows_per_group) {
@@ -603,18 +641,20 @@ int64_t plan_groups(GemvBatch& batch, int64_t rows_per_group) {
 }
 
 // The launch plan of a group: validated items, how its rows are read, whether any chain has
-// padding vectors, the longest row in vectors and per lane, and the total rows.
+// padding vectors, the longest row in vectors and per lane, the total rows and weight bytes.
 struct GroupPlan {
   GemvBatch batch{};
   Load load = Load::kAligned;
   bool pad = false;
+  bool dead_slot = false;  // some chain slot of a last position lies wholly past its row
   int64_t max_vectors = 1;
   int64_t max_per_lane = 1;
   int64_t rows = 0;
+  int64_t bytes = 0;  // of weights
 };
 
 // kSums: the in-pass kernel, with `rs` the row-sum checks it carries; otherwise the plain tree.
-template <int T, int R, int U, bool kFp8, Load kLoad, bool kPad, bool kNt, bool kSums,
+template <int T, int R, int U, bool kFp8, Load kLoad, Pad kPad, bool kNt, bool kSums,
           int kLive = (T >= kWave ? T / kWave : 1)>
 hipError_t launch_tree(GemvBatch& batch, const PckRowSumBatch* rs, hipStream_t stream) {
   constexpr int kLanesPerRow = T >= kWave ? kWave : T;
@@ -635,7 +675,7 @@ hipError_t launch_tree(GemvBatch& batch, const PckRowSumBatch* rs, hipStream_t s
   return hipGetLastError();
 }
 
-template <int T, int R, bool kFp8, bool kPad, bool kNt, bool kSums>
+template <int T, int R, bool kFp8, Pad kPad, bool kNt, bool kSums>
 hipError_t launch_unroll(GemvBatch& batch, int unroll, const PckRowSumBatch* rs, hipStream_t s) {
   constexpr Load L = Load::kAligned;
   if (unroll >= 4) return launch_tree<T, R, 4, kFp8, L, kPad, kNt, kSums>(batch, rs, s);
@@ -643,23 +683,30 @@ hipError_t launch_unroll(GemvBatch& batch, int unroll, const PckRowSumBatch* rs,
   return launch_tree<T, R, 1, kFp8, L, kPad, kNt, kSums>(batch, rs, s);
 }
 
-// T = 256, aligned rows: every shape.
-template <bool kFp8, bool kPad, bool kSums>
+// T = 256, aligned rows: every shape, and the default shapes with padding slots skipped.
+template <bool kFp8, Pad kPad, bool kSums>
 hipError_t launch_default(GemvBatch& batch, TreeShape shape, const PckRowSumBatch* rs,
                           hipStream_t s) {
   constexpr int T = 256;
   const bool nt = shape.nt != 0;
   const int u = shape.unroll;
-  switch (shape.rows) {
-    case 4:
-      return nt ? launch_unroll<T, 4, kFp8, kPad, true, kSums>(batch, u, rs, s)
-                : launch_unroll<T, 4, kFp8, kPad, false, kSums>(batch, u, rs, s);
-    case 2:
-      return nt ? launch_unroll<T, 2, kFp8, kPad, true, kSums>(batch, u, rs, s)
-                : launch_unroll<T, 2, kFp8, kPad, false, kSums>(batch, u, rs, s);
-    default:
-      return nt ? launch_unroll<T, 1, kFp8, kPad, true, kSums>(batch, u, rs, s)
-                : launch_unroll<T, 1, kFp8, kPad, false, kSums>(batch, u, rs, s);
+  if constexpr (kPad == Pad::kSkipped) {
+    constexpr Load L = Load::kAligned;
+    if (shape.rows == 2) return launch_tree<T, 2, 1, kFp8, L, kPad, true, kSums>(batch, rs, s);
+    return u == 2 ? launch_tree<T, 1, 2, kFp8, L, kPad, true, kSums>(batch, rs, s)
+                  : launch_tree<T, 1, 1, kFp8, L, kPad, true, kSums>(batch, rs, s);
+  } else {
+    switch (shape.rows) {
+      case 4:
+        return nt ? launch_unroll<T, 4, kFp8, kPad, true, kSums>(batch, u, rs, s)
+                  : launch_unroll<T, 4, kFp8, kPad, false, kSums>(batch, u, rs, s);
+      case 2:
+        return nt ? launch_unroll<T, 2, kFp8, kPad, true, kSums>(batch, u, rs, s)
+                  : launch_unroll<T, 2, kFp8, kPad, false, kSums>(batch, u, rs, s);
+      default:
+        return nt ? launch_unroll<T, 1, kFp8, kPad, true, kSums>(batch, u, rs, s)
+                  : launch_unroll<T, 1, kFp8, kPad, false, kSums>(batch, u, rs, s);
+    }
   }
 }
 
@@ -668,22 +715,36 @@ hipError_t launch_default(GemvBatch& batch, TreeShape shape, const PckRowSumBatc
 // R in {1, 2, 4}, U in {1 .. 4, 8} streamed from HBM, against R = 1, U = 2 with plain loads
 // (14336 x 4096 BF16: T = 64 / 128 / 512 19.6 / 19.9 / 20.0 against 23.5 / 22.4 / 21.8 us;
 // 4096 x 14336 FP8: T = 64 / 128 / 512 12.0 / 12.1 / 16.1 against 14.0 / 15.2 / 18.2 us).
-template <int T, bool kFp8, bool kPad, bool kSums>
-hipError_t launch_aligned(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
+template <int T, bool kFp8, Pad kPad, bool kNt, bool kSums>
+hipError_t launch_other(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
   constexpr Load L = Load::kAligned;
   GemvBatch& b = plan.batch;
+  if constexpr (T >= 1024) {
+    return launch_tree<T, 1, 1, kFp8, L, kPad, kNt, kSums>(b, rs, s);
+  } else if constexpr (T >= 512) {
+    if (kFp8 && plan.rows >= 2048)
+      return launch_tree<T, 2, 1, kFp8, L, kPad, kNt, kSums>(b, rs, s);
+    return launch_tree<T, 1, 1, kFp8, L, kPad, kNt, kSums>(b, rs, s);
+  } else {
+    if constexpr (!kNt) {  // served from a cache, one row and two positions is the best shape
+      return launch_tree<T, 1, 2, kFp8, L, kPad, kNt, kSums>(b, rs, s);
+    } else {
+      // one row per wave for BF16 rows of at most 4096 columns and for few rows
+      if ((!kFp8 && plan.max_vectors <= 512) || plan.rows < 4096)
+        return launch_tree<T, 1, 4, kFp8, L, kPad, kNt, kSums>(b, rs, s);
+      return launch_tree<T, 2, T >= 128 ? 2 : 4, kFp8, L, kPad, kNt, kSums>(b, rs, s);
+    }
+  }
+}
+
+template <int T, bool kFp8, Pad kPad, bool kSums>
+hipError_t launch_aligned(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
   if constexpr (T == 256) {
     return launch_default<kFp8, kPad, kSums>(
-        b, choose_shape(plan.max_per_lane, plan.rows, kFp8), rs, s);
-  } else if constexpr (T >= 1024) {
-    return launch_tree<T, 1, 1, kFp8, L, kPad, true, kSums>(b, rs, s);
-  } else if constexpr (T >= 512) {
-    return launch_tree<T, kFp8 ? 2 : 1, 1, kFp8, L, kPad, true, kSums>(b, rs, s);
+        plan.batch, choose_shape(plan.max_per_lane, plan.rows, kFp8), rs, s);
   } else {
-    constexpr int U = T >= 128 ? 2 : 4;
-    if (!kFp8 && plan.max_vectors <= 512)  // BF16 rows of at most 4096 columns
-      return launch_tree<T, 1, 4, kFp8, L, kPad, true, kSums>(b, rs, s);
-    return launch_tree<T, 2, U, kFp8, L, kPad, true, kSums>(b, rs, s);
+    return plan.bytes < kCachedBytes ? launch_other<T, kFp8, kPad, false, kSums>(plan, rs, s)
+                                     : launch_other<T, kFp8, kPad, true, kSums>(plan, rs, s);
   }
 }
 
@@ -695,7 +756,7 @@ template <int T, bool kFp8, bool kSums>
 hipError_t launch_unaligned(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
   constexpr int R = T >= 1024 || (T >= 512 && !kFp8) ? 1 : 2;
   constexpr int U = T <= 64 ? 2 : 1;
-  return launch_tree<T, R, U, kFp8, Load::kUnaligned, true, true, kSums>(plan.batch, rs, s);
+  return launch_tree<T, R, U, kFp8, Load::kUnaligned, Pad::kSkipped, true, kSums>(plan.batch, rs, s);
 }
 
 // Rows that end inside the first kLive chain slots (at most 64 kLive vectors).
@@ -705,8 +766,9 @@ hipError_t launch_live(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s)
   constexpr int Ra = kFp8 || kLive == 2 ? 2 : 1;
   constexpr int Rx = kFp8 || kLive <= 4 ? 2 : 1;
   GemvBatch& b = plan.batch;
-  return plan.load == A ? launch_tree<T, Ra, 1, kFp8, A, true, true, kSums, kLive>(b, rs, s)
-                        : launch_tree<T, Rx, 1, kFp8, X, true, true, kSums, kLive>(b, rs, s);
+  return plan.load == A
+             ? launch_tree<T, Ra, 1, kFp8, A, Pad::kZeroed, true, kSums, kLive>(b, rs, s)
+             : launch_tree<T, Rx, 1, kFp8, X, Pad::kSkipped, true, kSums, kLive>(b, rs, s);
 }
 
 // The route of a launch: element loads for rows shorter than a vector; else the fewest live
@@ -716,7 +778,7 @@ hipError_t launch_live(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s)
 template <int T, bool kFp8, bool kSums = false>
 hipError_t launch_for_threads(GroupPlan& plan, hipStream_t s, const PckRowSumBatch* rs = nullptr) {
   if (plan.load == Load::kElement)
-    return launch_tree<T, 1, 1, kFp8, Load::kElement, true, false, kSums>(plan.batch, rs, s);
+    return launch_tree<T, 1, 1, kFp8, Load::kElement, Pad::kZeroed, false, kSums>(plan.batch, rs, s);
   const bool all =
       T == 256 && plan.load == Load::kAligned && g_shape_override.rows > 0;  // a chosen shape
   if constexpr (T >= 256) {
@@ -729,11 +791,14 @@ hipError_t launch_for_threads(GroupPlan& plan, hipStream_t s, const PckRowSumBat
     if (plan.max_vectors <= 8 * kWave) return launch_live<T, 8, kFp8, kSums>(plan, rs, s);
   }
   if (plan.load == Load::kUnaligned) return launch_unaligned<T, kFp8, kSums>(plan, rs, s);
-  return plan.pad ? launch_aligned<T, kFp8, true, kSums>(plan, rs, s)
-                  : launch_aligned<T, kFp8, false, kSums>(plan, rs, s);
+  if (!plan.pad) return launch_aligned<T, kFp8, Pad::kNone, kSums>(plan, rs, s);
+  if constexpr (T >= 256) {
+    if (plan.dead_slot && !all) return launch_aligned<T, kFp8, Pad::kSkipped, kSums>(plan, rs, s);
+  }
+  return launch_aligned<T, kFp8, Pad::kZeroed, kSums>(plan, rs, s);
 }
 
-template <int R, int U, bool kFp8, bool kPad, bool kNt = true>
+template <int R, int U, bool kFp8, Pad kPad, bool kNt = true>
 hipError_t launch_ride_shape(GemvBatch& batch, const PckCheckBatch& ride, hipStream_t stream) {
   const int64_t groups = plan_groups(batch, static_cast<int64_t>(R) * kWavesPerGroup);
   const int64_t total = groups + ride.start[ride.count];
@@ -743,23 +808,23 @@ hipError_t launch_ride_shape(GemvBatch& batch, const PckCheckBatch& ride, hipStr
   return hipGetLastError();
 }
 
-// The carried-check launch uses the built-in shape of the T = 256 vector path for long rows
-// (choose_shape's), the launches a layer's checks ride in.
-template <bool kFp8>
-hipError_t launch_ride(GemvBatch& batch, bool pad, int64_t per_lane, const PckCheckBatch& ride,
-                       hipStream_t stream) {
+// The carried-check launch uses one shape per weight type and row length of the T = 256 aligned
+// path, the launches a layer's checks ride in.
+template <bool kFp8, Pad kPad>
+hipError_t launch_ride_pad(GroupPlan& plan, const PckCheckBatch& ride, hipStream_t stream) {
   if constexpr (kFp8) {
-    (void)per_lane;
-    return pad ? launch_ride_shape<2, 1, true, true>(batch, ride, stream)
-               : launch_ride_shape<2, 1, true, false>(batch, ride, stream);
+    return launch_ride_shape<2, 1, true, kPad>(plan.batch, ride, stream);
   } else {
-    if (per_lane > 2) {
-      return pad ? launch_ride_shape<2, 2, false, true>(batch, ride, stream)
-                 : launch_ride_shape<2, 2, false, false>(batch, ride, stream);
-    }
-    return pad ? launch_ride_shape<1, 2, false, true>(batch, ride, stream)
-               : launch_ride_shape<1, 2, false, false>(batch, ride, stream);
+    return plan.max_per_lane > 2 ? launch_ride_shape<2, 2, false, kPad>(plan.batch, ride, stream)
+                                 : launch_ride_shape<1, 2, false, kPad>(plan.batch, ride, stream);
   }
+}
+
+template <bool kFp8>
+hipError_t launch_ride(GroupPlan& plan, const PckCheckBatch& ride, hipStream_t stream) {
+  if (!plan.pad) return launch_ride_pad<kFp8, Pad::kNone>(plan, ride, stream);
+  return plan.dead_slot ? launch_ride_pad<kFp8, Pad::kSkipped>(plan, ride, stream)
+                        : launch_ride_pad<kFp8, Pad::kZeroed>(plan, ride, stream);
 }
 
 template <bool kFp8>
@@ -789,6 +854,7 @@ hipError_t plan_group(const PckGemv* gemvs, double* const* sums, int count, int 
       plan.batch.item[g].y_scaled = scaled[g];
     }
     plan.rows += d.m;
+    plan.bytes += d.m * n * (kFp8 ? 1 : 2);
     if (d.m > 0) {
       const bool aligned = n % V == 0 && reinterpret_cast<uintptr_t>(d.W) % 16 == 0 &&
                            reinterpret_cast<uintptr_t>(d.x) % 16 == 0;
@@ -798,6 +864,8 @@ hipError_t plan_group(const PckGemv* gemvs, double* const* sums, int count, int 
       plan.max_vectors = vectors > plan.max_vectors ? vectors : plan.max_vectors;
       plan.max_per_lane = per_lane > plan.max_per_lane ? per_lane : plan.max_per_lane;
       plan.pad = plan.pad || n % (static_cast<int64_t>(threads) * V) != 0;
+      plan.dead_slot =
+          plan.dead_slot || (threads > kWave && (vectors + kWave - 1) / kWave % (threads / kWave) != 0);
     }
   }
   return hipSuccess;
@@ -813,7 +881,7 @@ hipError_t launch_group(const PckGemv* gemvs, int count, int threads, const PckC
   if (ride != nullptr) {
     if (check::validate(*ride) != hipSuccess) return hipErrorInvalidValue;
     if (threads == 256 && plan.load == Load::kAligned && plan.rows > 0)
-      return launch_ride<kFp8>(plan.batch, plan.pad, plan.max_per_lane, *ride, stream);
+      return launch_ride<kFp8>(plan, *ride, stream);
     // Other configurations: the same check as its own launch first (identical results).
     const int64_t items = ride->start[ride->count];
     if (items * check::kThreads > 0xFFFFFFFFll) return hipErrorInvalidValue;
