@@ -508,83 +508,131 @@ __global__ void __launch_bounds__(kGroupThreads)
 // column order from its first product (columns past n add +0), then the T chain sums combined
 // by neighbour pairs, stride 1, 2, 4, ...: a[t] += a[t + s] for t a multiple of 2s.
 //
-// One workgroup of max(T, 64) lanes per row, lane t of the workgroup being virtual lane t (lanes
-// t >= T, present only when T < 64, own chunks wholly past n and feed no level below T).  The
-// levels of stride 1 .. 32 run inside each wave: every lane adds the value of its partner lane
+// One workgroup of max(T, 64) lanes takes R rows, lane t of the workgroup being virtual lane t
+// (lanes t >= T, present only when T < 64, own chunks wholly past n and feed no level below T).
+// The levels of stride 1 .. 32 run inside each wave: every lane adds the value of its partner lane
 // t + s, moved by DPP (quad permutes for 1 and 2, row rotations for 4 and 8), permlane16_swap
 // (16) or a read of lane 32 (32); the lanes that matter at a level read only lanes that
 // mattered at the level before, so lane 0 ends with the wave's subtree.  The levels of stride 64
 // and up combine the T / 64 wave sums, which meet in LDS behind one barrier, in the same pair
-// order.  kVector: 16-byte loads of W and x (c and n multiples of 8, aligned pointers), every
-// vector wholly before or wholly past n.
-template <bool kVector>
+// order.  kLoad: kAligned, 16-byte loads of chunks that are whole aligned vectors; kUnaligned, the
+// same at any 2-byte address (n >= 8), where a chunk's columns past its last whole vector, and
+// vectors that cross n, are read as 16 bytes inside the row and moved into place, so no lane takes
+// element loads; kElement, element loads, for chunks of fewer than four columns (a wave's lanes
+// then read one contiguous piece) and rows shorter than a vector.
+template <Load kLoad, int R>
 __global__ void __launch_bounds__(1024)
     gemv_naive_kernel(const uint16_t* __restrict__ W, const uint16_t* __restrict__ x,
-                      float* __restrict__ y, int64_t n, int64_t chunk, int threads) {
-  __shared__ float wave_sum[1024 / kWave];
+                      float* __restrict__ y, int64_t m, int64_t n, int64_t chunk, int threads) {
+  __shared__ float wave_sum[R][1024 / kWave];
   const int t = static_cast<int>(threadIdx.x);
   const int lane = t & (kWave - 1);
-  const uint16_t* row = W + static_cast<int64_t>(blockIdx.x) * n;
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * R;
   const int64_t first = static_cast<int64_t>(t) * chunk;
-
-  float acc = 0.0f;
-  if constexpr (kVector) {
-    for (int64_t v = 0; v < chunk; v += 8) {
-      const int64_t col = first + v;
-      uint4 wv = make_uint4(0, 0, 0, 0), xv = make_uint4(0, 0, 0, 0);  // past n: +0 products
-      if (col < n) {
-        wv = *reinterpret_cast<const uint4*>(row + col);
-        xv = *reinterpret_cast<const uint4*>(x + col);
-      }
-      const uint32_t wd[4] = {wv.x, wv.y, wv.z, wv.w};
-      const uint32_t xd[4] = {xv.x, xv.y, xv.z, xv.w};
+  const uint16_t* rows[R];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float p0 = bf16_lo(wd[k]) * bf16_lo(xd[k]);
-        const float p1 = bf16_hi(wd[k]) * bf16_hi(xd[k]);
-        acc = (v == 0 && k == 0) ? p0 : acc + p0;
-        acc = acc + p1;
+  for (int r = 0; r < R; ++r)  // rows past m compute on row m - 1 and are not stored
+    rows[r] = W + (row0 + r < m ? row0 + r : m - 1) * n;
+
+  float acc[R];  // -0.0 + p0 is p0: the chain starts from its first product
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = -0.0f;
+  if constexpr (kLoad != Load::kElement) {
+    constexpr bool kAny = kLoad == Load::kUnaligned;
+    // columns col .. col + 7 of x and of the rows (+0 past n)
+    struct Vectors {
+      uint4 x, w[R];
+    };
+    auto load = [&](int64_t col) {
+      const int64_t at = col < n - 8 ? col : n - 8;
+      Vectors v;
+      v.x = load16<false, kAny>(x + at);
+#pragma unroll
+      for (int r = 0; r < R; ++r) v.w[r] = load16<false, kAny>(rows[r] + at);
+      return v;
+    };
+    auto add = [&](Vectors& v, int64_t col, int count) {  // the first `count` columns
+      if (col > n - 8) {
+        const int skip = col < n ? static_cast<int>(col - (n - 8)) : 8;
+        drop_front<false>(v.x, skip);
+#pragma unroll
+        for (int r = 0; r < R; ++r) drop_front<false>(v.w[r], skip);
       }
+      const uint32_t xd[4] = {v.x.x, v.x.y, v.x.z, v.x.w};
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const uint32_t wd[4] = {v.w[r].x, v.w[r].y, v.w[r].z, v.w[r].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (2 * k < count) acc[r] = acc[r] + bf16_lo(wd[k]) * bf16_lo(xd[k]);
+          if (2 * k + 1 < count) acc[r] = acc[r] + bf16_hi(wd[k]) * bf16_hi(xd[k]);
+        }
+      }
+    };
+    int64_t c = 0;
+    for (; c + 16 <= chunk; c += 16) {
+      Vectors a = load(first + c), b = load(first + c + 8);
+      add(a, first + c, 8);
+      add(b, first + c + 8, 8);
+    }
+    for (; c < chunk; c += 8) {  // the last one or two vectors, the last perhaps partial
+      Vectors a = load(first + c);
+      if (c + 8 <= chunk) add(a, first + c, 8);
+      else add(a, first + c, static_cast<int>(chunk - c));
     }
   } else {
     for (int64_t j = first; j < first + chunk; ++j) {
-      float p = 0.0f;
-      if (j < n) p = __uint_as_float(static_cast<uint32_t>(row[j]) << 16) *
-                     __uint_as_float(static_cast<uint32_t>(x[j]) << 16);
-      acc = j == first ? p : acc + p;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float p = 0.0f;
+        if (j < n) p = __uint_as_float(static_cast<uint32_t>(rows[r][j]) << 16) *
+                       __uint_as_float(static_cast<uint32_t>(x[j]) << 16);
+        acc[r] = acc[r] + p;
+      }
     }
   }
 
-  // Levels inside the wave (uniform bounds: `threads` is the same for every lane).
-  if (threads > 1) acc = acc + dpp_move<0xB1>(acc);   // stride 1: quad_perm [1,0,3,2]
-  if (threads > 2) acc = acc + dpp_move<0x4E>(acc);   // stride 2: quad_perm [2,3,0,1]
-  if (threads > 4) acc = acc + dpp_move<0x12C>(acc);  // stride 4: row_ror:12, lane i <- i + 4
-  if (threads > 8) acc = acc + dpp_move<0x128>(acc);  // stride 8: row_ror:8, lane i <- i + 8
-  if (threads > 16) {                                  // stride 16: lanes 0-15 <- 16-31
-    const auto swapped =
-        __builtin_amdgcn_permlane16_swap(__float_as_int(acc), __float_as_int(acc), false, false);
-    acc = acc + __int_as_float(swapped[1]);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    float v = acc[r];
+    // Levels inside the wave (uniform bounds: `threads` is the same for every lane).
+    if (threads > 1) v = v + dpp_move<0xB1>(v);   // stride 1: quad_perm [1,0,3,2]
+    if (threads > 2) v = v + dpp_move<0x4E>(v);   // stride 2: quad_perm [2,3,0,1]
+    if (threads > 4) v = v + dpp_move<0x12C>(v);  // stride 4: row_ror:12, lane i <- i + 4
+    if (threads > 8) v = v + dpp_move<0x128>(v);  // stride 8: row_ror:8, lane i <- i + 8
+    if (threads > 16) {                            // stride 16: lanes 0-15 <- 16-31
+      const auto swapped =
+          __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+      v = v + __int_as_float(swapped[1]);
+    }
+    if (threads > 32) v = lane_value(v, 0) + lane_value(v, 32);  // stride 32
+    acc[r] = v;
   }
-  if (threads > 32) acc = lane_value(acc, 0) + lane_value(acc, 32);  // stride 32
 
   if (threads <= kWave) {
-    if (t == 0) y[blockIdx.x] = acc;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (t == 0 && row0 + r < m) y[row0 + r] = acc[r];
     return;
   }
-  // Levels across waves: wave w's subtree is a[64 w]; pairs of stride 64, 128, ...
-  if (lane == 0) wave_sum[t / kWave] = acc;
+  // Levels across waves: wave w's subtree is a[64 w]; pairs of stride 64, 128, ...  Lane r of the
+  // workgroup finishes row r.
+  if (lane == 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) wave_sum[r][t / kWave] = acc[r];
+  }
   __syncthreads();
-  if (t == 0) {
+  if (t < R && row0 + t < m) {
     const int waves = threads / kWave;
     float a[1024 / kWave];
 #pragma unroll
-    for (int w = 0; w < 1024 / kWave; ++w) a[w] = w < waves ? wave_sum[w] : 0.0f;
+    for (int w = 0; w < 1024 / kWave; ++w) a[w] = w < waves ? wave_sum[t][w] : 0.0f;
 #pragma unroll
     for (int s = 1; s < 1024 / kWave; s *= 2)
 #pragma unroll
       for (int w = 0; w + s < 1024 / kWave; w += 2 * s)
         if (s < waves) a[w] = a[w] + a[w + s];
-    y[blockIdx.x] = a[0];
+    y[row0 + t] = a[0];
   }
 }
 
@@ -971,17 +1019,32 @@ int pck_gemv_bf16_naive(const void* W, const void* x, float* y, int64_t m, int64
   if (m == 0) return hipSuccess;
   if (n < 1 || !W || !x || !y) return hipErrorInvalidValue;
   const int64_t chunk = (n + threads - 1) / threads;
-  const bool vector = chunk % 8 == 0 && n % 8 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  const dim3 grid(static_cast<unsigned>(m)), group(static_cast<unsigned>(lanes));
+  using pck::Load;
+  const bool aligned = chunk % 8 == 0 && n % 8 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  const Load load = n < 8 || chunk < 4 ? Load::kElement : aligned ? Load::kAligned : Load::kUnaligned;
+  // Four rows per workgroup for many short aligned chunks (14336 x 4096 at T = 256: 24.3 against
+  // 25.7 us with one; longer chunks of several rows push each other out of the L1: 4096 x 14336
+  // 84 against 58) and for ragged ones (14536 x 3647 at T = 512: 23 against 100 us with element
+  // loads; 7182 x 8960, T = 256: 55 against 212).
+  const bool four = load == Load::kUnaligned ? m >= 2048
+                                             : load == Load::kAligned && chunk <= 16 && m >= 8192 &&
+                                                   threads >= 256;
+  const int rows = four ? 4 : 1;
+  const dim3 grid(static_cast<unsigned>((m + rows - 1) / rows)), group(static_cast<unsigned>(lanes));
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const auto* w16 = static_cast<const uint16_t*>(W);
   const auto* x16 = static_cast<const uint16_t*>(x);
-  if (vector)
-    pck::gemv_naive_kernel<true><<<grid, group, 0, s>>>(w16, x16, y, n, chunk, threads);
-  else
-    pck::gemv_naive_kernel<false><<<grid, group, 0, s>>>(w16, x16, y, n, chunk, threads);
-  return hipGetLastError();
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, group, 0, s>>>(w16, x16, y, m, n, chunk, threads);
+    return hipGetLastError();
+  };
+  if (load == Load::kElement) return launch(pck::gemv_naive_kernel<Load::kElement, 1>);
+  if (load == Load::kAligned)
+    return four ? launch(pck::gemv_naive_kernel<Load::kAligned, 4>)
+                : launch(pck::gemv_naive_kernel<Load::kAligned, 1>);
+  return four ? launch(pck::gemv_naive_kernel<Load::kUnaligned, 4>)
+              : launch(pck::gemv_naive_kernel<Load::kUnaligned, 1>);
 }
 
 int pck_gemv_set_shape(int rows_per_wave, int unroll, int nontemporal) {

@@ -104,6 +104,26 @@ def test_naive_vector_and_element_paths(m: int, n: int, threads: int) -> None:
     assert_bits(run(KERNELS[0], W, x, threads), emulate_gemv(W, x, threads))
 
 
+# (m, n, threads): four rows per workgroup with a last partial one (ragged and aligned chunks),
+# chunks of 3 (element loads), 4, 17 and 8 k + 1 columns, lanes wholly past n, one vector per row.
+@pytest.mark.parametrize(("m", "n", "threads"), [(2051, 1003, 64), (2050, 4100, 256), (8195, 4096, 256),
+                                                 (7, 3072, 1024), (7, 4099, 1024), (5, 9, 1), (6, 8, 2),
+                                                 (5, 2049, 32)])  # fmt: skip
+def test_naive_rows_of_any_length_and_address(m: int, n: int, threads: int) -> None:
+    """Against the C model; W and x start one and three elements into NaN-filled buffers, so a
+    column read from outside its row would show."""
+    g = torch.Generator().manual_seed(n + threads)
+    W = (torch.randn(m, n, generator=g) * 0.02).to(torch.bfloat16)
+    x = torch.randn(n, generator=g).to(torch.bfloat16)
+    want = gemv_naive_c(W.float().numpy(), x.float().numpy(), threads)
+    assert_bits(gemv_naive(W.cuda(), x.cuda(), threads).cpu().numpy(), want)
+    wb = torch.full((m * n + 64,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    xb = torch.full((n + 64,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wb[1 : 1 + m * n], xb[3 : 3 + n] = W.cuda().reshape(-1), x.cuda()
+    y = gemv_naive(wb[1 : 1 + m * n].view(m, n), xb[3 : 3 + n], threads)
+    assert_bits(y.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize(("m", "n"), [(1024, 4096), (4096, 14336)])
 def test_naive_llama_shapes_bit_exact(m: int, n: int) -> None:
     """The naive tree at T = 256 on decode shapes (chunks of 16 and 56 columns) against the
