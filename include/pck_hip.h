@@ -129,6 +129,25 @@ int pck_bgemm_pack(int kind, const void* src, void* dst, int64_t rows, int64_t n
 int pck_bgemm_packed(int weight_kind, const void* Wp, const void* Xp, float* Y, int64_t m,
                      int64_t n, int64_t batch, void* stream);
 
+/* The packed product for any m, n and addresses: the same tiles, with each of the 8 K segments
+ * (P = ceil(ceil(n / 8) / 8) chunks) on step pairs of its own: pair j of segment w is step pair
+ * w ceil(P / 2) + j and holds chunks w P + 2 j and w P + 2 j + 1, zero past the segment and past
+ * n.  A tile row then has pck_bgemm_any_columns(n) = 128 ceil(P / 2) elements (n itself when
+ * n % 128 == 0, where the layout is pck_bgemm_pack's); dst holds ceil(rows / 32) * 32 times that,
+ * 16-byte aligned.  pck_bgemm_packed_any takes operands packed by pck_bgemm_pack_any and gives
+ * the bits of pck_bgemm.  pck_bgemm_any_columns returns -1 for n < 1 or n > 2^30.  No reference
+ * counterpart. */
+int64_t pck_bgemm_any_columns(int64_t n);
+int pck_bgemm_pack_any(int kind, const void* src, void* dst, int64_t rows, int64_t n, void* stream);
+int pck_bgemm_packed_any(int weight_kind, const void* Wp, const void* Xp, float* Y, int64_t m,
+                         int64_t n, int64_t batch, void* stream);
+
+/* Both launches of a batched product from row-major X in one call: packs X (batch, n) into the
+ * caller's Xp (as pck_bgemm_pack's dst, or pck_bgemm_pack_any's), then the product.  Wp is packed
+ * by pck_bgemm_pack when n % 128 == 0 and m % 4 == 0, else by pck_bgemm_pack_any. */
+int pck_bgemm_product(int weight_kind, const void* Wp, const void* X, void* Xp, float* Y, int64_t m,
+                      int64_t n, int64_t batch, void* stream);
+
 /* Tuning knob of pck_bgemm_packed: 32-row weight tiles and 32-row batch tiles per workgroup,
  * (1, 1), (1, 2), (1, 4) or (2, 2); (0, 0) restores the built-in choice.
  * Changes only speed: outputs keep the same bits.  Process-wide and not thread-safe; no

@@ -279,10 +279,13 @@ __device__ __forceinline__ s16x4 x_step(const u32x4& v, int j) {
 struct PackedArgs {
   const char* Wp;  // packed weights, ceil(m / 32) tiles
   const char* Xp;  // packed activations, ceil(batch / 32) tiles
-  float* Y;        // (batch, ldy) FP32, row-major, columns 0 .. m - 1 written, 16-byte aligned
-  int64_t ldy;     // Y's row stride (a multiple of 4)
+  float* Y;        // (batch, ldy) FP32, row-major, columns 0 .. m - 1 written
+  int64_t ldy;     // Y's row stride
   int64_t m;
-  int64_t n;
+  int64_t chunks;  // ceil(n / 8)
+  int64_t seg_pairs;  // step pairs a K segment takes in the layout
+  bool any;        // the kernel for any n, m and Y
+  bool quads;      // m and ldy are multiples of 4 and Y is 16-byte aligned: 16-byte stores
   int64_t batch;
   int64_t row_tiles;
   int64_t batch_tiles;
@@ -306,7 +309,9 @@ constexpr int ring_pairs() {
 // (row group, pass): with the groups a multiple of 8, the passes of a row group are items 8
 // apart, which run at about the same time on one XCD (workgroup w runs on XCD w % 8 when G is
 // a multiple of 8), so their repeated weight reads hit that XCD's L2.
-template <int R, int T, bool kFp8>
+// kAny: segments of an odd number of chunks, empty segments and rows that do not take 16-byte
+// stores (pck_bgemm_packed_any); the others compile to code without them.
+template <int R, int T, bool kFp8, bool kAny>
 __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
   constexpr uint32_t kQ = kFp8 ? 8 : 16;  // weight bytes per lane and step pair
   // Step pairs in flight per lane, the same for both operands: the vector-memory counter
@@ -322,18 +327,22 @@ __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
 
   const int64_t groups = (a.row_tiles + R - 1) / R;
   const int64_t items = groups * a.passes;
-  // Segments of whole step pairs (the host requires n % 128 == 0, so per is even).
-  const int64_t chunks = a.n / kStep;
+  // Each segment starts a step pair of the layout of its own; a segment of an odd number of
+  // chunks (never when n % 128 == 0) ends with half a pair, and one past the row has none.
+  const int64_t chunks = a.chunks;
   const int64_t per = (chunks + kWaves - 1) / kWaves;
   const int64_t c_lo = wave * per < chunks ? wave * per : chunks;
   const int64_t c_hi = c_lo + per < chunks ? c_lo + per : chunks;
-  const int pairs = static_cast<int>(c_hi - c_lo) / 2;
-  const int last = pairs - 1;
+  const int pairs = static_cast<int>(c_hi - c_lo + (kAny ? 1 : 0)) / 2;
+  const bool odd = kAny && (c_hi - c_lo) % 2 != 0;
+  const int last = !kAny || pairs > 0 ? pairs - 1 : 0;
 
   // One buffer per operand and item: the item's row group of the weights and its pass's batch
   // tiles.  Tiles past the end (a partial last group or pass) lie past the buffer and read 0.
-  const uint32_t w_tile_bytes = static_cast<uint32_t>(chunks / 2 * 64 * kQ);
-  const uint32_t x_tile_bytes = static_cast<uint32_t>(chunks / 2 * 64 * 16);
+  const uint32_t tile_pairs = static_cast<uint32_t>(kWaves * a.seg_pairs);
+  const uint32_t first_pair = static_cast<uint32_t>(wave * a.seg_pairs);
+  const uint32_t w_tile_bytes = tile_pairs * 64 * kQ;
+  const uint32_t x_tile_bytes = tile_pairs * 64 * 16;
   struct Item {
     const char* w_base;  // the row group's first tile
     const char* x_base;  // the pass's first batch tile
@@ -367,10 +376,10 @@ __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
   };
   uint32_t w_voff[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r) w_voff[r] = static_cast<uint32_t>(r * w_tile_bytes + (c_lo / 2 * 64 + lane) * kQ);
+  for (int r = 0; r < R; ++r) w_voff[r] = static_cast<uint32_t>(r * w_tile_bytes + (first_pair * 64 + lane) * kQ);
   uint32_t x_voff[T];
 #pragma unroll
-  for (int t = 0; t < T; ++t) x_voff[t] = static_cast<uint32_t>(t * x_tile_bytes + (c_lo / 2 * 64 + lane) * 16);
+  for (int t = 0; t < T; ++t) x_voff[t] = static_cast<uint32_t>(t * x_tile_bytes + (first_pair * 64 + lane) * 16);
   constexpr uint32_t kWs = 64 * kQ;  // weight bytes per step pair
   constexpr uint32_t kXs = 64 * 16;  // batch bytes per step pair and tile
 
@@ -417,8 +426,6 @@ __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
     }
   };
 
-  // n % 128 == 0 (checked on the host) gives every wave per = n / 64 chunks, so pairs >= 1
-  // and is the same in every wave.
   int64_t g = blockIdx.x;
   if (g >= items) return;  // uniform
 
@@ -461,11 +468,13 @@ __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
     // Pair q with ring slot k: two steps of one MFMA per (row tile, batch tile), each step's
     // products added to its group sum (kFirst: the group's first step, assigned), then the
     // slot's refill.
-    auto pair_step = [&](int q, auto k_const, auto first_const, const Refill& rf) {
+    auto pair_step = [&](int q, auto k_const, auto first_const, const Refill& rf, auto tail_const) {
       constexpr int k = decltype(k_const)::value;
       constexpr bool kFirst = decltype(first_const)::value;
+      constexpr bool kTail = decltype(tail_const)::value;  // may be the segment's half pair
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
+        if (kTail && j == 1 && odd && q == last) break;  // uniform
 #pragma unroll
         for (int r = 0; r < R; ++r) {
           const s16x4 wv = w_step<kFp8>(w[k][r], j);
@@ -499,14 +508,14 @@ __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
         for (int v = 0; v < 16; ++v) acc[r][t][v] = -0.0f;
     // Whole groups: ring passes with no exit inside, so the loads in flight are the same on
     // every entry to the loop head and no step waits for more than its own operands.
-    const int whole = pairs / kGroupPairs * kGroupPairs;
+    const int whole = (pairs - (odd ? 1 : 0)) / kGroupPairs * kGroupPairs;
     for (int base = 0; base < whole; base += kGroupPairs) {
       auto ring_pass = [&](auto p_const) {
         constexpr int P = decltype(p_const)::value;
         const Refill rf = refill_for(base + P * kRing);
         [&]<int... K>(std::integer_sequence<int, K...>) {
           (pair_step(base + P * kRing + K, std::integral_constant<int, K>{},
-                     std::integral_constant<bool, P == 0 && K == 0>{}, rf), ...);
+                     std::integral_constant<bool, P == 0 && K == 0>{}, rf, No{}), ...);
         }(std::make_integer_sequence<int, kRing>{});
       };
       [&]<int... P>(std::integer_sequence<int, P...>) {
@@ -526,12 +535,15 @@ __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
       for (int base = whole; base < full; base += kRing) {
         const Refill rf = refill_for(base);
         [&]<int... K>(std::integer_sequence<int, K...>) {
-          (pair_step(base + K, std::integral_constant<int, K>{}, No{}, rf), ...);
+          (pair_step(base + K, std::integral_constant<int, K>{}, No{}, rf, std::true_type{}), ...);
         }(std::make_integer_sequence<int, kRing>{});
       }
       const Refill rf = refill_for(full);  // chaining implies full == pairs: no pair runs here
       [&]<int... K>(std::integer_sequence<int, K...>) {
-        ((full + K < pairs ? (pair_step(full + K, std::integral_constant<int, K>{}, No{}, rf), 0) : 0), ...);
+        ((full + K < pairs
+              ? (pair_step(full + K, std::integral_constant<int, K>{}, No{}, rf, std::true_type{}), 0)
+              : 0),
+         ...);
       }(std::make_integer_sequence<int, kRing>{});
       flush();
     }
@@ -573,8 +585,14 @@ __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
                             ((slots[4][k][lane] + slots[5][k][lane]) +
                              (slots[6][k][lane] + slots[7][k][lane]));
             const int64_t i = rt * kRows + 8 * q + 4 * h;
-            if (b < a.batch && i < a.m)
-              *reinterpret_cast<float4*>(yrow + 8 * q) = make_float4(y[0], y[1], y[2], y[3]);
+            if (!kAny || a.quads) {
+              if (b < a.batch && i < a.m)
+                *reinterpret_cast<float4*>(yrow + 8 * q) = make_float4(y[0], y[1], y[2], y[3]);
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if (b < a.batch && i + e < a.m) yrow[8 * q + e] = y[e];
+            }
           }
         }
       }
@@ -654,6 +672,55 @@ __global__ void __launch_bounds__(256) pack_bf16_kernel(const char* __restrict__
       make_uint4(lo.x, lo.y, hi.x, hi.y);
 }
 
+// Packs (rows, n) of any n and address into the step-pair layout with each K segment on a step
+// pair of its own: pair j of segment w holds chunks w per + 2 j and the next one, zero past the
+// segment and past n.  One 16-byte piece (8 for E4M3) per lane; a lane's four columns of a chunk
+// are one load where they lie inside the row.
+template <bool kFp8>
+__global__ void __launch_bounds__(256) pack_any_kernel(const char* __restrict__ src,
+                                                       char* __restrict__ dst, int64_t rows,
+                                                       int64_t n, int64_t chunks, int64_t per,
+                                                       int64_t seg_pairs, int64_t pieces) {
+  constexpr int kBytes = kFp8 ? 1 : 2;
+  typedef u32x2 u32x2_any __attribute__((aligned(2)));
+  typedef uint32_t u32_any __attribute__((aligned(1)));
+  const int64_t p = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (p >= pieces) return;
+  const int64_t pairs = kWaves * seg_pairs;
+  const int64_t L = p % 64;
+  const int64_t q = (p / 64) % pairs;
+  const int64_t row = p / (64 * pairs) * 32 + (L & 31);
+  const int64_t seg = q / seg_pairs;
+  const int64_t seg_end = (seg + 1) * per < chunks ? (seg + 1) * per : chunks;
+  uint32_t v[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int64_t c = seg * per + 2 * (q - seg * seg_pairs) + j;
+    const int64_t col = c * kStep + 4 * (L >> 5);
+    if (row >= rows || c >= seg_end) continue;
+    const char* at = src + (row * n + col) * kBytes;
+    if (col + 4 <= n) {
+      if constexpr (kFp8) {
+        v[j] = *reinterpret_cast<const u32_any*>(at);
+      } else {
+        const u32x2 w = *reinterpret_cast<const u32x2_any*>(at);
+        v[2 * j] = w[0];
+        v[2 * j + 1] = w[1];
+      }
+    } else {
+      for (int e = 0; e < 4 && col + e < n; ++e) {
+        if constexpr (kFp8)
+          v[j] |= static_cast<uint32_t>(static_cast<uint8_t>(at[e])) << (8 * e);
+        else
+          v[2 * j + e / 2] |=
+              static_cast<uint32_t>(*reinterpret_cast<const uint16_t*>(at + 2 * e)) << (16 * (e % 2));
+      }
+    }
+  }
+  if constexpr (kFp8) reinterpret_cast<uint2*>(dst)[p] = make_uint2(v[0], v[1]);
+  else reinterpret_cast<uint4*>(dst)[p] = make_uint4(v[0], v[1], v[2], v[3]);
+}
+
 template <bool kFp8, bool kVector>
 hipError_t launch_tiles(const BgemmArgs& a, int tiles, dim3 grid, hipStream_t stream) {
   switch (tiles) {
@@ -699,9 +766,9 @@ PackedShape choose_shape(int64_t row_tiles, int64_t batch, bool fp8) {
   return PackedShape{1, 1};
 }
 
-// Workgroups of bgemm_packed_kernel<R, T, kFp8> to launch at most: one per CU where a CU holds
+// Workgroups of bgemm_packed_kernel<R, T, kFp8, kAny> to launch at most: one per CU where a CU holds
 // one, else no limit (one item per workgroup); computed once per instantiation and device.
-template <int R, int T, bool kFp8>
+template <int R, int T, bool kFp8, bool kAny>
 hipError_t resident_groups(int64_t* out) {
   constexpr int kMaxDevices = 64;
   static std::atomic<int64_t> cache[kMaxDevices];  // one array per instantiation
@@ -718,7 +785,7 @@ hipError_t resident_groups(int64_t* out) {
   int cus = 0, per_cu = 0;
   err = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (err != hipSuccess) return err;
-  err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bgemm_packed_kernel<R, T, kFp8>,
+  err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bgemm_packed_kernel<R, T, kFp8, kAny>,
                                                      kThreads, 0);
   if (err != hipSuccess) return err;
   // With two or more workgroups per CU the others already cover one's start-up latency, and
@@ -729,24 +796,26 @@ hipError_t resident_groups(int64_t* out) {
   return hipSuccess;
 }
 
-template <int R, int T, bool kFp8>
+template <int R, int T, bool kFp8, bool kAny>
 hipError_t launch_rtf(PackedArgs a, hipStream_t stream) {
   a.passes = (a.batch_tiles + T - 1) / T;
   const int64_t items = (a.row_tiles + R - 1) / R * a.passes;
   if (items > 0x7FFFFFFF) return hipErrorInvalidValue;
   int64_t resident = 0;
-  const hipError_t err = resident_groups<R, T, kFp8>(&resident);
+  const hipError_t err = resident_groups<R, T, kFp8, kAny>(&resident);
   if (err != hipSuccess) return err;
   const int64_t groups = items < resident ? items : resident;
   if (groups > 0x7FFFFFFF / kThreads) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((bgemm_packed_kernel<R, T, kFp8>), dim3(static_cast<unsigned>(groups)),
+  hipLaunchKernelGGL((bgemm_packed_kernel<R, T, kFp8, kAny>), dim3(static_cast<unsigned>(groups)),
                      dim3(kThreads), 0, stream, a);
   return hipGetLastError();
 }
 
 template <int R, int T>
 hipError_t launch_rt(const PackedArgs& a, bool fp8, hipStream_t stream) {
-  return fp8 ? launch_rtf<R, T, true>(a, stream) : launch_rtf<R, T, false>(a, stream);
+  if (a.any)
+    return fp8 ? launch_rtf<R, T, true, true>(a, stream) : launch_rtf<R, T, false, true>(a, stream);
+  return fp8 ? launch_rtf<R, T, true, false>(a, stream) : launch_rtf<R, T, false, false>(a, stream);
 }
 
 hipError_t launch_one(const PackedArgs& a, PackedShape shape, bool fp8, hipStream_t stream) {
@@ -759,16 +828,17 @@ hipError_t launch_one(const PackedArgs& a, PackedShape shape, bool fp8, hipStrea
 }
 
 template <int R, int T>
-hipError_t resident_rt(bool fp8, int64_t* out) {
-  return fp8 ? resident_groups<R, T, true>(out) : resident_groups<R, T, false>(out);
+hipError_t resident_rt(bool fp8, bool any, int64_t* out) {
+  if (any) return fp8 ? resident_groups<R, T, true, true>(out) : resident_groups<R, T, false, true>(out);
+  return fp8 ? resident_groups<R, T, true, false>(out) : resident_groups<R, T, false, false>(out);
 }
 
-hipError_t resident_for(PackedShape shape, bool fp8, int64_t* out) {
-  if (shape.rows == 2) return resident_rt<2, 2>(fp8, out);
-  if (shape.rows == 3) return resident_rt<3, 1>(fp8, out);
-  if (shape.tiles == 4) return resident_rt<1, 4>(fp8, out);
-  if (shape.tiles == 2) return resident_rt<1, 2>(fp8, out);
-  return resident_rt<1, 1>(fp8, out);
+hipError_t resident_for(PackedShape shape, bool fp8, bool any, int64_t* out) {
+  if (shape.rows == 2) return resident_rt<2, 2>(fp8, any, out);
+  if (shape.rows == 3) return resident_rt<3, 1>(fp8, any, out);
+  if (shape.tiles == 4) return resident_rt<1, 4>(fp8, any, out);
+  if (shape.tiles == 2) return resident_rt<1, 2>(fp8, any, out);
+  return resident_rt<1, 1>(fp8, any, out);
 }
 
 // A looping shape (one resident workgroup per CU) whose item count is not a multiple of the
@@ -779,7 +849,7 @@ hipError_t resident_for(PackedShape shape, bool fp8, int64_t* out) {
 // output keeps its bits: an output's sum does not depend on the item that computes it.
 hipError_t launch_packed(const PackedArgs& a, PackedShape shape, bool fp8, hipStream_t stream) {
   int64_t resident = 0;
-  hipError_t err = resident_for(shape, fp8, &resident);
+  hipError_t err = resident_for(shape, fp8, a.any, &resident);
   if (err != hipSuccess) return err;
   const int64_t passes = (a.batch_tiles + shape.tiles - 1) / shape.tiles;
   const int64_t items = (a.row_tiles + shape.rows - 1) / shape.rows * passes;
@@ -793,7 +863,7 @@ hipError_t launch_packed(const PackedArgs& a, PackedShape shape, bool fp8, hipSt
   err = launch_one(lead, shape, fp8, stream);
   if (err != hipSuccess) return err;
   PackedArgs rest = a;
-  const int64_t w_tile_bytes = (a.n / kStep) / 2 * 64 * (fp8 ? 8 : 16);
+  const int64_t w_tile_bytes = kWaves * a.seg_pairs * 64 * (fp8 ? 8 : 16);
   rest.Wp = a.Wp + lead_tiles * w_tile_bytes;
   rest.Y = a.Y + lead.m;
   rest.row_tiles = a.row_tiles - lead_tiles;
@@ -874,8 +944,79 @@ extern "C" int pck_bgemm_packed(int weight_kind, const void* Wp, const void* Xp,
   const int64_t batch_tiles = (batch + 31) / 32;
   // One buffer resource covers one weight tile and one pass's batch tiles (32-bit offsets).
   if ((n / kStep) * 32 * 16 * 4 > 0x7FFFFFFFll) return hipErrorInvalidValue;
-  const PackedArgs a{static_cast<const char*>(Wp), static_cast<const char*>(Xp), Y, m, m, n,
-                     batch, row_tiles, batch_tiles, 1};
+  const PackedArgs a{static_cast<const char*>(Wp), static_cast<const char*>(Xp), Y, m, m,
+                     n / kStep, n / (2 * kStep * kWaves), false, true, batch, row_tiles, batch_tiles, 1};
   return launch_packed(a, choose_shape(row_tiles, batch, weight_kind == 1), weight_kind == 1,
                        static_cast<hipStream_t>(stream));
+}
+
+namespace pck {
+namespace {
+
+// Chunks per K segment and step pairs a segment takes in the layout, for any n.
+struct AnyLayout {
+  int64_t chunks, per, seg_pairs;
+};
+
+AnyLayout any_layout(int64_t n) {
+  const int64_t chunks = (n + kStep - 1) / kStep;
+  const int64_t per = (chunks + kWaves - 1) / kWaves;
+  return AnyLayout{chunks, per, (per + 1) / 2};
+}
+
+}  // namespace
+}  // namespace pck
+
+extern "C" int64_t pck_bgemm_any_columns(int64_t n) {
+  if (n < 1 || n > (int64_t{1} << 30)) return -1;
+  return pck::any_layout(n).seg_pairs * pck::kWaves * 2 * pck::kStep;
+}
+
+extern "C" int pck_bgemm_pack_any(int kind, const void* src, void* dst, int64_t rows, int64_t n,
+                                  void* stream) {
+  using namespace pck;
+  if ((kind != 0 && kind != 1) || !src || !dst || rows < 1 || n < 1 || n > (int64_t{1} << 30) ||
+      reinterpret_cast<uintptr_t>(dst) % 16 != 0 || (kind == 0 && reinterpret_cast<uintptr_t>(src) % 2 != 0))
+    return hipErrorInvalidValue;
+  const AnyLayout l = any_layout(n);
+  const int64_t tiles = (rows + 31) / 32;
+  const int64_t pieces = tiles * 64 * kWaves * l.seg_pairs;
+  if (pieces * (kind == 1 ? 8 : 16) > 0xFFFFFFFFll / 2) return hipErrorInvalidValue;
+  const dim3 grid(static_cast<unsigned>((pieces + 255) / 256));
+  auto s = static_cast<hipStream_t>(stream);
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, dim3(256), 0, s>>>(static_cast<const char*>(src), static_cast<char*>(dst), rows,
+                                      n, l.chunks, l.per, l.seg_pairs, pieces);
+    return hipGetLastError();
+  };
+  return kind == 1 ? launch(pack_any_kernel<true>) : launch(pack_any_kernel<false>);
+}
+
+extern "C" int pck_bgemm_packed_any(int weight_kind, const void* Wp, const void* Xp, float* Y,
+                                    int64_t m, int64_t n, int64_t batch, void* stream) {
+  using namespace pck;
+  if ((weight_kind != 0 && weight_kind != 1) || !Wp || !Xp || !Y || m < 1 || batch < 1 || n < 1 ||
+      n > (int64_t{1} << 30) || reinterpret_cast<uintptr_t>(Y) % 4 != 0 ||
+      reinterpret_cast<uintptr_t>(Wp) % 16 != 0 || reinterpret_cast<uintptr_t>(Xp) % 16 != 0)
+    return hipErrorInvalidValue;
+  const AnyLayout l = any_layout(n);
+  const int64_t row_tiles = (m + 31) / 32;
+  const int64_t batch_tiles = (batch + 31) / 32;
+  // One buffer resource covers one weight tile and one pass's batch tiles (32-bit offsets).
+  if (l.seg_pairs * kWaves * 2 * 32 * 16 * 4 > 0x7FFFFFFFll) return hipErrorInvalidValue;
+  const bool quads = m % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0;
+  const PackedArgs a{static_cast<const char*>(Wp), static_cast<const char*>(Xp), Y, m, m,
+                     l.chunks, l.seg_pairs, true, quads, batch, row_tiles, batch_tiles, 1};
+  return launch_packed(a, choose_shape(row_tiles, batch, weight_kind == 1), weight_kind == 1,
+                       static_cast<hipStream_t>(stream));
+}
+
+extern "C" int pck_bgemm_product(int weight_kind, const void* Wp, const void* X, void* Xp, float* Y,
+                                 int64_t m, int64_t n, int64_t batch, void* stream) {
+  const bool plain = n >= 128 && n % 128 == 0 && m % 4 == 0;
+  const int err = plain ? pck_bgemm_pack(0, X, Xp, batch, n, stream)
+                        : pck_bgemm_pack_any(0, X, Xp, batch, n, stream);
+  if (err != hipSuccess) return err;
+  return plain ? pck_bgemm_packed(weight_kind, Wp, Xp, Y, m, n, batch, stream)
+               : pck_bgemm_packed_any(weight_kind, Wp, Xp, Y, m, n, batch, stream);
 }

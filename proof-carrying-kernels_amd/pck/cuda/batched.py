@@ -10,7 +10,8 @@ Two routes with the same bits:
 - `gemm_batched(W, X)` with a plain (m, n) weight tensor runs the element kernel (any shape);
 - `gemm_batched(pack_batched_weights(W), X)` runs the packed kernel: the weights are packed
   once, at load time, into 32-row tiles whose matrix-core operands are contiguous, and each call
-  packs X the same way into a workspace.  This is the decode path.
+  packs X the same way into a workspace.  This is the decode path.  Shapes with n % 128 != 0 or
+  m % 4 != 0 take the form of the layout that pads each K segment to whole step pairs.
 """
 
 from __future__ import annotations
@@ -20,7 +21,7 @@ from dataclasses import dataclass
 
 import torch
 
-from pck.cuda._lib import check, lib, stream_handle
+from pck.cuda._lib import check, lib, on_device, stream_handle
 
 STEP = 8
 WAVES = 8
@@ -40,14 +41,16 @@ def batched_height(n: int) -> int:
 
 @dataclass
 class BatchedWeights:
-    """Weights for `gemm_batched` in the packed 32-row tile layout (`packed` is None when the
-    shape has no packed route: n % 128 != 0 or m % 4 != 0; then `raw` is used)."""
+    """Weights for `gemm_batched` in the packed 32-row tile layout (`packed` is None when n % 128
+    != 0 or m % 4 != 0; `padded` then holds the tiles with each K segment padded to whole step
+    pairs and `raw` the weights as they were given)."""
 
     m: int
     n: int
     dtype: torch.dtype
     packed: torch.Tensor | None
     raw: torch.Tensor | None
+    padded: torch.Tensor | None = None
 
     @property
     def device(self) -> torch.device:
@@ -69,9 +72,21 @@ def _pack(src: torch.Tensor, kind: int) -> torch.Tensor:
     tiles = (rows + TILE - 1) // TILE
     elem = torch.uint8 if kind == 1 else torch.bfloat16
     dst = torch.empty(tiles * TILE * n, dtype=elem, device=src.device)
-    with torch.cuda.device(src.device):
+    with on_device(src.device):
         err = lib().pck_bgemm_pack(kind, src.data_ptr(), dst.data_ptr(), rows, n,
                                    stream_handle(src.device))  # fmt: skip
+    check(err, "batched pack launch")
+    return dst
+
+
+def _pack_any(src: torch.Tensor, kind: int) -> torch.Tensor:
+    rows, n = src.shape
+    columns = lib().pck_bgemm_any_columns(n)
+    elem = torch.uint8 if kind == 1 else torch.bfloat16
+    dst = torch.empty((rows + TILE - 1) // TILE * TILE * columns, dtype=elem, device=src.device)
+    with on_device(src.device):
+        err = lib().pck_bgemm_pack_any(kind, src.data_ptr(), dst.data_ptr(), rows, n,
+                                       stream_handle(src.device))  # fmt: skip
     check(err, "batched pack launch")
     return dst
 
@@ -89,11 +104,13 @@ def _validate_w(W: torch.Tensor) -> None:
 
 def pack_batched_weights(W: torch.Tensor) -> BatchedWeights:
     """Packs W (m, n) BF16 or float8_e4m3fn (raw codes) once for the packed kernel; enqueued on
-    the current stream.  Shapes without a packed route keep W as it is."""
+    the current stream.  Shapes with n % 128 != 0 or m % 4 != 0 also keep W as it is."""
     _validate_w(W)
     m, n = W.shape
-    if m == 0 or not _packable(m, n):
+    if m == 0 or n == 0:
         return BatchedWeights(m, n, W.dtype, None, W)
+    if not _packable(m, n):
+        return BatchedWeights(m, n, W.dtype, None, W, _pack_any(W, _kind(W.dtype)))
     return BatchedWeights(m, n, W.dtype, _pack(W, _kind(W.dtype)), None)
 
 
@@ -137,11 +154,13 @@ def gemm_batched(
     if n == 0:
         raise RuntimeError("n must be positive")
     kind = _kind(dtype)
-    with torch.cuda.device(device):
-        if packed and W.packed is not None:
-            Xp = _pack(X, 0)
-            err = lib().pck_bgemm_packed(kind, W.packed.data_ptr(), Xp.data_ptr(), Y.data_ptr(),
-                                         m, n, B, stream_handle(device))  # fmt: skip
+    tiles = (W.packed if W.packed is not None else W.padded) if packed else None
+    with on_device(device):
+        if tiles is not None:
+            columns = n if W.packed is not None else lib().pck_bgemm_any_columns(n)
+            Xp = torch.empty((B + TILE - 1) // TILE * TILE * columns, dtype=X.dtype, device=device)
+            err = lib().pck_bgemm_product(kind, tiles.data_ptr(), X.data_ptr(), Xp.data_ptr(),
+                                          Y.data_ptr(), m, n, B, stream_handle(device))  # fmt: skip
         else:
             raw = W.raw if packed else W
             assert raw is not None

@@ -346,3 +346,36 @@ def test_activation_pack_layout_aligned_and_8_byte_aligned(rows: int, n: int) ->
         got = dst.cpu().numpy().view(np.uint16)
         assert src.data_ptr() % 16 == (0 if src is flat else 8)
         assert np.array_equal(got, want)
+
+
+# (m, n, B): one chunk (seven empty segments), a partial chunk, segments of an odd number of
+# chunks (n = 60, 320, 1001, 3000), of 15 and 17 chunks (n = 960, 1088: the half pair ends a group
+# or begins one), rows past m, m % 4 != 0, several batch passes and workgroups looping over items.
+ANY_SHAPES = [(5, 7, 3), (1, 8, 1), (33, 128, 20), (32, 60, 20), (34, 320, 40), (64, 960, 33),
+              (64, 1088, 33), (101, 1001, 70), (36, 3000, 24), (66, 4100, 300), (19203, 520, 128)]  # fmt: skip
+
+
+@pytest.mark.parametrize(("m", "n", "B"), ANY_SHAPES, ids=str)
+@pytest.mark.parametrize("fam", ["real", "wide", "cancel", "tiny"])
+def test_padded_segments_give_the_element_kernels_bits(m: int, n: int, B: int, fam: str) -> None:
+    """BF16 and FP8 weights from unaligned views; the element kernel is itself bit-exact against
+    the model, which the smaller shapes are compared with as well."""
+    rng = np.random.default_rng(m + n + B)
+    W = _family(rng, (m, n), "real_w" if fam == "real" else fam)
+    X = _family(rng, (B, n), "real_x" if fam in ("real", "tiny") else fam)
+    Xt = _bf16_tensor(X)
+    Wt = torch.zeros(m * n + 1, dtype=torch.bfloat16, device=DEV)
+    Wt[1:] = _bf16_tensor(W).reshape(-1)
+    Wt = Wt[1:].view(m, n)
+    codes = rng.integers(0, 256, (m, n), dtype=np.uint8)
+    codes[(codes & 0x7F) == 0x7F] = 0  # no NaN codes
+    Q = torch.from_numpy(codes).view(torch.float8_e4m3fn).to(DEV)
+    for w in (Wt, Q):
+        bw = pack_batched_weights(w)
+        assert bw.padded is not None
+        got = gemm_batched(bw, Xt)
+        want = gemm_batched(w, Xt)
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+    if m * n * B < 10_000_000:
+        assert _same_bits(_run(W, X, packed=True), emulate_batched(W, X))
