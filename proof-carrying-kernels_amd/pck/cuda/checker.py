@@ -26,6 +26,7 @@ from pck.cuda._lib import (
     PckRowSumCheckDesc,
     check,
     lib,
+    on_device,
     stream_handle,
 )
 from pck.fp import U32, U64, ceil_div, gamma, next_up, sum_up_factor
@@ -287,7 +288,7 @@ def blocked_check(
     batch, outputs, device = build_batch(
         c, a, r, x, y, partial_cx, partial_s, counters, coef, geps, tau_floor
     )
-    with torch.cuda.device(device):
+    with on_device(device):
         err = lib().pck_blocked_check(batch, stream_handle(device))
     check(err, "checker kernel launch")
     return outputs
@@ -470,7 +471,7 @@ def rowsum_check_many(
     results: list[CheckResult] = []
     for i in range(0, len(items), MAX_BATCH):
         batch, res, device = rowsum_batch_for(items[i : i + MAX_BATCH])
-        with torch.cuda.device(device):
+        with on_device(device):
             err = lib().pck_rowsum_check(batch, stream_handle(device))
         check(err, "row-sum check launch")
         results.extend(res)
@@ -516,7 +517,7 @@ def _check_columns(ch: GpuBlockedChecker, X: torch.Tensor, Y: torch.Tensor) -> C
             [ch.c] * k, [ch.a] * k, [ch.r] * k, xs, ys, [ch._partial_cx] * k, [ch._partial_s] * k,
             [ch._counters] * k, [ch.coef] * k, [ch.geps] * k, [ch.tau_floor] * k,
         )  # fmt: skip
-        with torch.cuda.device(device):
+        with on_device(device):
             err = lib().pck_blocked_check(batch, stream_handle(device))
         check(err, "checker kernel launch")
         cols.extend(outputs)
@@ -589,7 +590,7 @@ def _check_batched_direct(
         check(lib().pck_batch_check_workspace(descs, len(chunk), ctypes.byref(need)),
               "batched checker plan")  # fmt: skip
         work = torch.empty(max(1, need.value // 8), dtype=torch.float64, device=device)
-        with torch.cuda.device(device):
+        with on_device(device):
             err = lib().pck_batch_check(descs, len(chunk), work.data_ptr(), need.value,
                                         stream_handle(device))  # fmt: skip
         check(err, "batched checker launch")
@@ -641,7 +642,7 @@ class SideStreamChecker:
         self.stream.wait_event(produced)
         for t in (x, y, result.passed, result.rho, result.tau):
             t.record_stream(self.stream)
-        with torch.cuda.device(device):
+        with on_device(device):
             err = lib().pck_blocked_check(batch, int(self.stream.cuda_stream))
         check(err, "checker kernel launch")
         done = torch.cuda.Event()

@@ -14,7 +14,7 @@ from typing import Any
 
 import torch
 
-from pck.cuda._lib import MAX_GROUP, PckGemv, check, lib, stream_handle
+from pck.cuda._lib import MAX_GROUP, PckGemv, check, lib, on_device, stream_handle
 
 INT32_MAX = 2**31 - 1
 _NAMES = {torch.bfloat16: "BFloat16", torch.float8_e4m3fn: "Float8_e4m3fn"}
@@ -55,7 +55,7 @@ def _launch(
         return y
     if W.size(1) == 0:
         raise RuntimeError("n must be positive")
-    with torch.cuda.device(W.device):
+    with on_device(W.device):
         err = getattr(handle, entry)(
             W.data_ptr(), x.data_ptr(), y.data_ptr(), W.size(0), W.size(1), threads,
             stream_handle(W.device),
@@ -145,7 +145,7 @@ def gemv_group_check(
         ride, results, check_device = batch_for(checks)
         if check_device != device:
             raise RuntimeError("the checks must be on the GEMVs' device")
-    with torch.cuda.device(device):
+    with on_device(device):
         err = lib().pck_gemv_group_check(
             kind, descs, len(pairs), threads, None if ride is None else ctypes.byref(ride),
             stream_handle(device),
@@ -189,7 +189,7 @@ def gemv_group_fp8_scaled(
         ride, results, check_device = batch_for(checks)
         if check_device != device:
             raise RuntimeError("the checks must be on the GEMVs' device")
-    with torch.cuda.device(device):
+    with on_device(device):
         err = lib().pck_gemv_group_fp8_scaled(
             descs, s_ptrs, y_ptrs, len(triples), threads,
             None if ride is None else ctypes.byref(ride), stream_handle(device),
@@ -218,7 +218,7 @@ def gemv_group(
     their weights (`harness/bench_decode_layer.py:48-53`).
     """
     descs, outs, kind, device = _group_descriptors(pairs, threads)
-    with torch.cuda.device(device):
+    with on_device(device):
         err = lib().pck_gemv_group(kind, descs, len(pairs), threads, stream_handle(device))
     check(err, "grouped gemv launch")
     return outs
@@ -248,7 +248,7 @@ def gemv_group_rowsums(
         ride, results, check_device = rowsum_batch_for(checks)
         if check_device != device:
             raise RuntimeError("the checks must be on the GEMVs' device")
-    with torch.cuda.device(device):
+    with on_device(device):
         err = lib().pck_gemv_group_rowsums(
             kind, descs, ptrs, len(pairs), threads, None if ride is None else ctypes.byref(ride),
             stream_handle(device),

@@ -11,12 +11,13 @@ trusted.
 
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass
 
 import torch
 
-from pck.cuda._lib import check, lib, stream_handle
+from pck.cuda._lib import check, compute_units, lib, on_device, stream_handle
 from pck.cuda.checker import _check_tensor
 from pck.fp import U32, U64, ceil_div, gamma
 
@@ -39,7 +40,7 @@ def default_segments(logits: torch.Tensor) -> int:
     """Split each row so that the grid has about ``BLOCKS_PER_SM`` workgroups per CU, with at
     least ``MIN_SEGMENT`` logits per segment (reference `cuda/sampling.py:43-47`)."""
     rows, vocab = logits.shape
-    cus = torch.cuda.get_device_properties(logits.device).multi_processor_count
+    cus = compute_units(logits.device.index)
     return max(1, min(ceil_div(BLOCKS_PER_SM * cus, rows), ceil_div(vocab, MIN_SEGMENT)))
 
 
@@ -90,7 +91,7 @@ def sampling_check(
     min_sel = buf[part + 16 * rows : part + 20 * rows].view(torch.float32)
     max_rej = buf[part + 20 * rows : part + 24 * rows].view(torch.float32)
     passed = buf[part + 24 * rows : part + 25 * rows].view(torch.bool)
-    with torch.cuda.device(device):
+    with on_device(device):
         err = handle.pck_sampling_check(
             logits.data_ptr(), selected.data_ptr(), None if lengths is None else lengths.data_ptr(),
             rows, vocab, max_len, k,
@@ -112,6 +113,7 @@ def check_topk_gpu(
     return SamplingCheck(*out)
 
 
+@functools.lru_cache(maxsize=256)
 def topp_slack(vocab: int, segments: int, tol: float) -> float:
     """The sampler's ``tol`` plus this checker's own rounding (reference
     `cuda/sampling.py:71-88`): each term is FP32 expf on a split argument (within 2 ulp, plus

@@ -23,7 +23,7 @@ import torch
 
 from pck.agent.column import ColumnConfig
 from pck.agent.config import GROUP, KernelConfig, template_flags
-from pck.cuda._lib import check, lib, stream_handle
+from pck.cuda._lib import check, lib, on_device, stream_handle
 from pck.cuda.gemv import INT32_MAX, _validate
 
 _p = ctypes.c_void_p
@@ -70,7 +70,7 @@ def _template(
         return y
     if W.size(1) == 0:
         raise RuntimeError("n must be positive")
-    with torch.cuda.device(W.device):
+    with on_device(W.device):
         err = _lib().pck_gemv_template(
             W.data_ptr(), x.data_ptr(), y.data_ptr(), W.size(0), W.size(1), threads,
             rows_per_block, vec, unroll, flags, stream_handle(W.device),
@@ -104,7 +104,7 @@ def _template_q8(
     y = torch.empty(m, dtype=torch.float32, device=x.device)
     if m == 0:
         return y
-    with torch.cuda.device(Wq.device):
+    with on_device(Wq.device):
         err = _lib().pck_gemv_template_q8(
             Wq.data_ptr(), S.data_ptr(), x.data_ptr(), y.data_ptr(), m, n, threads,
             rows_per_block, vec, unroll, stream_handle(Wq.device),
@@ -141,7 +141,7 @@ def _column_run(
             raise RuntimeError(
                 "tickets must be a zeroed int32 CUDA tensor with at least one entry per tile"
             )
-    with torch.cuda.device(WT.device):
+    with on_device(WT.device):
         err = _lib().pck_gemv_column(
             WT.data_ptr(), x.data_ptr(), y.data_ptr(), scratch.data_ptr(), None, m, n, threads,
             vec, splits, skip_below, stream_handle(WT.device),
@@ -197,7 +197,7 @@ def row_q8(
     m, n = Wd.shape
     Wq = torch.empty((m, n), dtype=torch.int8, device=Wd.device)
     S = torch.empty((m, -(-n // GROUP)), dtype=torch.float32, device=Wd.device)
-    with torch.cuda.device(Wd.device):
+    with on_device(Wd.device):
         err = _lib().pck_quantize_rows_q8(
             Wd.data_ptr(), 0 if Wd.dtype == torch.bfloat16 else 1, Wq.data_ptr(), S.data_ptr(),
             m, n, stream_handle(Wd.device),

@@ -19,6 +19,7 @@ error bounds the slack is built from (reference `src/pck/member.py:37-41,84-102`
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from dataclasses import dataclass
 from typing import Any
@@ -78,6 +79,7 @@ def check_member(
     return MemberVerdict(bool(r < next_up(top_p + slack)), above, r)
 
 
+@functools.lru_cache(maxsize=256)
 def member_eps32(vocab: int) -> float:
     """Error bound of r for FP32 split-argument terms summed in FP64 (reference
     `src/pck/member.py:84-102`): each term within 6 u32 relative plus 2^-124 absolute (a
@@ -92,7 +94,11 @@ def member_eps32(vocab: int) -> float:
 def _host_top_k(top_k: Any, top_k_host: Any, vocab: int) -> tuple[int, bool]:
     """(k_lim, all_k) from the host copy of top-k (reference `src/pck/member.py:152-157`):
     the largest top-k below the vocabulary and whether every row has one."""
-    host = top_k_host if top_k_host is not None else top_k.cpu().numpy()
+    host = np.asarray(top_k_host if top_k_host is not None else top_k.cpu().numpy())
+    if host.dtype.kind == "i" and host.size:
+        largest = int(host.max())
+        if largest < vocab:  # every row has a top-k
+            return max(largest, 1), True
     hk = np.clip(np.asarray(host).astype(np.int64), 1, vocab)
     lim = hk[hk < vocab]
     return (int(lim.max()), lim.size == hk.size) if lim.size else (0, False)
@@ -157,7 +163,7 @@ def launch_check(
     synchronises: top-k's host copy is ``top_k_host`` (or one copy of ``top_k``)."""
     import torch
 
-    from pck.cuda._lib import PckMemberArgs, check, lib, stream_handle
+    from pck.cuda._lib import PckMemberArgs, check, lib, on_device, stream_handle
 
     kinds = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
     if not logits.is_cuda:
@@ -176,7 +182,9 @@ def launch_check(
     def dev(x: Any, dtype: Any, name: str) -> int | None:
         if x is None:
             return None
-        t = x.to(device=device, dtype=dtype).reshape(rows).contiguous() if dtype else x
+        t = x
+        if not (x.dtype == dtype and x.device == device and x.dim() == 1 and x.is_contiguous()):
+            t = x.to(device=device, dtype=dtype).reshape(rows).contiguous()
         if t.numel() != rows:
             raise RuntimeError(f"{name} must have {rows} entries, got {t.numel()}")
         keep.append(t)
@@ -199,11 +207,9 @@ def launch_check(
         a.temperature_count = t.numel()
         a.temperature_index = dev(temperature_index, torch.long, "temperature_index")
     elif greedy is not None:  # a bool tensor is read as its bytes (0 or 1)
-        g = greedy.to(device=device, dtype=torch.bool).reshape(rows).contiguous().view(torch.uint8)
-        a.greedy = dev(g, None, "greedy")
+        a.greedy = dev(greedy, torch.bool, "greedy")
     if injected is not None:
-        inj = injected.to(device=device, dtype=torch.bool).reshape(rows).contiguous().view(torch.uint8)
-        a.injected = dev(inj, None, "injected")
+        a.injected = dev(injected, torch.bool, "injected")
     if totals is not None:
         if not (totals.is_cuda and totals.device == device and totals.dtype == torch.int64
                 and totals.numel() == 6 and totals.is_contiguous()):  # fmt: skip
@@ -211,12 +217,10 @@ def launch_check(
         a.totals = totals.data_ptr()
     out = None
     if outputs:
-        # the three outputs in one allocation: [mass_above | above | ok]
-        buf = torch.empty(17 * rows, dtype=torch.uint8, device=device)
         out = {
-            "ok": buf[16 * rows :].view(torch.bool),
-            "above": buf[8 * rows : 16 * rows].view(torch.int64),
-            "mass_above": buf[: 8 * rows].view(torch.float64),
+            "ok": torch.empty(rows, dtype=torch.bool, device=device),
+            "above": torch.empty(rows, dtype=torch.int64, device=device),
+            "mass_above": torch.empty(rows, dtype=torch.float64, device=device),
         }
         a.ok, a.above, a.mass_above = (
             out["ok"].data_ptr(), out["above"].data_ptr(), out["mass_above"].data_ptr()
@@ -227,7 +231,7 @@ def launch_check(
     handle = lib()
     need = ctypes.c_int64(0)
     check(handle.pck_check_members_workspace(a, kind, ctypes.byref(need)), "membership check plan")
-    with torch.cuda.device(device):
+    with on_device(device):
         if need.value:  # rows split over workgroups, read in the logits' own type
             work = torch.empty(need.value, dtype=torch.uint8, device=device)
             err = handle.pck_check_members_split(
