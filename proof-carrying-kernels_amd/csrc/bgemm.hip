@@ -78,12 +78,14 @@ struct BgemmArgs {
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
-// Two E4M3FN codes (bytes kHigh * 2, kHigh * 2 + 1 of w) as their BF16 bit patterns, packed
-// low / high.  Every E4M3 value is a BF16 value, so dropping the FP32 low half is exact.
+// Two E4M3FN codes (bytes kHigh * 2, kHigh * 2 + 1 of w) as BF16 values, packed low / high: one
+// conversion at scale 1, exact (every E4M3 value is a BF16 value; the bits equal the upper halves
+// of the FP32 conversion for all 256 codes).  One VALU instruction instead of a conversion, a
+// shift and an and-or: the products are bound by VALU issue, and the layer of 256 rows with its
+// checks takes 338.4 instead of 344.5 us.
 template <bool kHigh>
 __device__ __forceinline__ uint32_t fp8_pair_bf16(uint32_t w) {
-  auto f = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w), kHigh);
-  return (__float_as_uint(f[0]) >> 16) | (__float_as_uint(f[1]) & 0xFFFF0000u);
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, kHigh));
 }
 
 // Chunk c of row `row` (columns 8c .. 8c + 7) as 8 BF16 operands; zeros past n or past the
