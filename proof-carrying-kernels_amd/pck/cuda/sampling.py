@@ -116,12 +116,12 @@ def check_topk_gpu(
 @functools.lru_cache(maxsize=256)
 def topp_slack(vocab: int, segments: int, tol: float) -> float:
     """The sampler's ``tol`` plus this checker's own rounding (reference
-    `cuda/sampling.py:71-88`): each term is FP32 expf on a split argument (within 2 ulp, plus
-    under 2 u32 for the split and the FMA: 6 u32 relative) or below 2^-148 where dropped;
+    `cuda/sampling.py:71-88`): each term is an FP32 2^hi on a split argument (within 2 ulp, plus
+    under 2 u32 for the split and the FMA: 6 u32 relative) or below 2^-125 where dropped;
     each of the S segment partials is rescaled with one FP64 exp, multiply and add; the
-    largest term is exactly 1.  Each mass is then within 16 u32 + V 2^-146 +
+    largest term is exactly 1.  Each mass is then within 16 u32 + V 2^-124 +
     gamma_{V + 3S + 16}(u64), rounded up."""
-    own = 16 * U32 + math.ldexp(vocab, -146) + gamma(vocab + 3 * segments + 16, U64)
+    own = 16 * U32 + math.ldexp(vocab, -124) + gamma(vocab + 3 * segments + 16, U64)
     return math.nextafter(tol + own, math.inf)
 
 
