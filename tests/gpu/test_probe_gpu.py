@@ -5,6 +5,8 @@ libpck_probe.so, built with the library's flags), against exact host arithmetic.
   `src/pck/member.py:84-102`).  Every FP32 x in [-128, -2^-26] (276,824,065 values) is checked
   against the FP64 exponential, and a sample of (-2^-26, 0]; the error must be at most 2 ulp
   of the exact value's FP32 spacing (measured: below 1 ulp).
+- ``v_exp_f32``: the set checker's 2^hi, every FP32 in [-126, -2^-26]: at most 1 ulp; never above
+  2^-126 below that.
 - ``v_mfma_f64_16x16x4_f64``: the batched checker's c . x assumes every operation rounds to
   nearest.  Measured: each output is four IEEE FMAs in K order, each rounded once to nearest
   even, continued across chained steps.  Crafted cases separate this from one rounding of the
@@ -62,6 +64,25 @@ def test_expf_within_two_ulp_on_every_float_in_minus_128_to_0() -> None:
     assert worst <= 2.0
     tiny = -np.random.default_rng(0).uniform(0, 2.0**-26, 1 << 20).astype(np.float32)
     assert float(ulp_errors(np.append(tiny, np.float32(-0.0))).max()) <= 2.0
+
+
+def test_exp2_within_one_ulp_on_every_float_in_minus_126_to_0() -> None:
+    """The set checker's 2^hi: its bound takes 2 ulp for a normal result, and 0 below 2^-126."""
+    lo = int(np.float32(2.0**-26).view(np.uint32))
+    hi = int(np.float32(126.0).view(np.uint32))
+    worst = 0.0
+    for start in range(lo, hi + 1, 1 << 24):
+        bits = np.arange(start, min(start + (1 << 24), hi + 1), dtype=np.uint32) | np.uint32(1 << 31)
+        x = bits.view(np.float32)
+        y = probe.exp2(torch.from_numpy(x).cuda()).cpu().numpy().astype(np.float64)
+        e = np.exp2(x.astype(np.float64))
+        worst = max(worst, float((np.abs(y - e) / np.spacing(e.astype(np.float32))).max()))
+    print(f"exp2 over [-126, -2^-26]: max error {worst:.6f} ulp", flush=True)
+    assert worst <= 1.0
+    edges = torch.tensor([0.0, -0.0, -127.0, -128.0, -1000.0, float("-inf")], device="cuda")
+    got = probe.exp2(edges).cpu().numpy()
+    assert got[0] == got[1] == 1.0
+    assert (got[2:] >= 0.0).all() and (got[2:] <= 2.0**-126).all()
 
 
 # ---- FP64 matrix core ---------------------------------------------------------------------
