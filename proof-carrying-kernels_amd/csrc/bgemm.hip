@@ -335,7 +335,8 @@ __global__ void __launch_bounds__(kThreads) bgemm_packed_kernel(PackedArgs a) {
   const int64_t per = (chunks + kWaves - 1) / kWaves;
   const int64_t c_lo = wave * per < chunks ? wave * per : chunks;
   const int64_t c_hi = c_lo + per < chunks ? c_lo + per : chunks;
-  const int pairs = static_cast<int>(c_hi - c_lo + (kAny ? 1 : 0)) / 2;
+  // Without kAny every segment is seg_pairs whole pairs: no index arithmetic ahead of the loads.
+  const int pairs = kAny ? static_cast<int>(c_hi - c_lo + 1) / 2 : static_cast<int>(a.seg_pairs);
   const bool odd = kAny && (c_hi - c_lo) % 2 != 0;
   const int last = !kAny || pairs > 0 ? pairs - 1 : 0;
 
