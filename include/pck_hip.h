@@ -135,8 +135,9 @@ int pck_bgemm_packed(int weight_kind, const void* Wp, const void* Xp, float* Y, 
  * n.  A tile row then has pck_bgemm_any_columns(n) = 128 ceil(P / 2) elements (n itself when
  * n % 128 == 0, where the layout is pck_bgemm_pack's); dst holds ceil(rows / 32) * 32 times that,
  * 16-byte aligned.  pck_bgemm_packed_any takes operands packed by pck_bgemm_pack_any and gives
- * the bits of pck_bgemm.  pck_bgemm_any_columns returns -1 for n < 1 or n > 2^30.  No reference
- * counterpart. */
+ * the bits of pck_bgemm.  Tiles may have any size; rows may not: pck_bgemm_any_columns returns -1
+ * for n < 1 and for n > 2^23 - 128 (a batch tile's 32-bit offsets), and the other two refuse such
+ * an n.  No reference counterpart. */
 int64_t pck_bgemm_any_columns(int64_t n);
 int pck_bgemm_pack_any(int kind, const void* src, void* dst, int64_t rows, int64_t n, void* stream);
 int pck_bgemm_packed_any(int weight_kind, const void* Wp, const void* Xp, float* Y, int64_t m,

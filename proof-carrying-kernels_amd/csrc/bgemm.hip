@@ -683,11 +683,12 @@ template <bool kFp8>
 __global__ void __launch_bounds__(256) pack_any_kernel(const char* __restrict__ src,
                                                        char* __restrict__ dst, int64_t rows,
                                                        int64_t n, int64_t chunks, int64_t per,
-                                                       int64_t seg_pairs, int64_t pieces) {
+                                                       int64_t seg_pairs, int64_t pieces,
+                                                       int64_t first_piece) {
   constexpr int kBytes = kFp8 ? 1 : 2;
   typedef u32x2 u32x2_any __attribute__((aligned(2)));
   typedef uint32_t u32_any __attribute__((aligned(1)));
-  const int64_t p = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t p = first_piece + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (p >= pieces) return;
   const int64_t pairs = kWaves * seg_pairs;
   const int64_t L = p % 64;
@@ -807,8 +808,10 @@ hipError_t launch_rtf(PackedArgs a, hipStream_t stream) {
   int64_t resident = 0;
   const hipError_t err = resident_groups<R, T, kFp8, kAny>(&resident);
   if (err != hipSuccess) return err;
+  // A workgroup loops over items, so a grid at the dispatch limit takes any number of them.
+  constexpr int64_t kMaxGroups = 0x7FFFFFFF / kThreads;
+  if (resident > kMaxGroups) resident = kMaxGroups;
   const int64_t groups = items < resident ? items : resident;
-  if (groups > 0x7FFFFFFF / kThreads) return hipErrorInvalidValue;
   hipLaunchKernelGGL((bgemm_packed_kernel<R, T, kFp8, kAny>), dim3(static_cast<unsigned>(groups)),
                      dim3(kThreads), 0, stream, a);
   return hipGetLastError();
@@ -956,6 +959,8 @@ extern "C" int pck_bgemm_packed(int weight_kind, const void* Wp, const void* Xp,
 namespace pck {
 namespace {
 
+constexpr int64_t kMaxPackBlocks = int64_t{1} << 23;  // of 256 pieces: 32 GiB of BF16 a launch
+
 // Chunks per K segment and step pairs a segment takes in the layout, for any n.
 struct AnyLayout {
   int64_t chunks, per, seg_pairs;
@@ -967,46 +972,56 @@ AnyLayout any_layout(int64_t n) {
   return AnyLayout{chunks, per, (per + 1) / 2};
 }
 
+// Columns one buffer resource still covers: a weight tile and a pass's batch tiles have 32-bit
+// offsets.
+bool any_fits(int64_t n) {
+  return n >= 1 && n <= (int64_t{1} << 30) &&
+         any_layout(n).seg_pairs * kWaves * 2 * 32 * 16 * 4 <= 0x7FFFFFFFll;
+}
+
 }  // namespace
 }  // namespace pck
 
 extern "C" int64_t pck_bgemm_any_columns(int64_t n) {
-  if (n < 1 || n > (int64_t{1} << 30)) return -1;
+  if (!pck::any_fits(n)) return -1;
   return pck::any_layout(n).seg_pairs * pck::kWaves * 2 * pck::kStep;
 }
 
 extern "C" int pck_bgemm_pack_any(int kind, const void* src, void* dst, int64_t rows, int64_t n,
                                   void* stream) {
   using namespace pck;
-  if ((kind != 0 && kind != 1) || !src || !dst || rows < 1 || n < 1 || n > (int64_t{1} << 30) ||
+  if ((kind != 0 && kind != 1) || !src || !dst || rows < 1 || !any_fits(n) ||
       reinterpret_cast<uintptr_t>(dst) % 16 != 0 || (kind == 0 && reinterpret_cast<uintptr_t>(src) % 2 != 0))
     return hipErrorInvalidValue;
   const AnyLayout l = any_layout(n);
   const int64_t tiles = (rows + 31) / 32;
   const int64_t pieces = tiles * 64 * kWaves * l.seg_pairs;
-  if (pieces * (kind == 1 ? 8 : 16) > 0xFFFFFFFFll / 2) return hipErrorInvalidValue;
-  const dim3 grid(static_cast<unsigned>((pieces + 255) / 256));
+  // Tiles of any size: 64-bit indexes, and as many launches below the 32-bit dispatch as they need.
   auto s = static_cast<hipStream_t>(stream);
-  auto launch = [&](auto kernel) {
-    kernel<<<grid, dim3(256), 0, s>>>(static_cast<const char*>(src), static_cast<char*>(dst), rows,
-                                      n, l.chunks, l.per, l.seg_pairs, pieces);
-    return hipGetLastError();
-  };
-  return kind == 1 ? launch(pack_any_kernel<true>) : launch(pack_any_kernel<false>);
+  for (int64_t first = 0; first < pieces; first += kMaxPackBlocks * 256) {
+    const int64_t blocks = (pieces - first + 255) / 256;
+    const dim3 grid(static_cast<unsigned>(blocks < kMaxPackBlocks ? blocks : kMaxPackBlocks));
+    auto launch = [&](auto kernel) {
+      kernel<<<grid, dim3(256), 0, s>>>(static_cast<const char*>(src), static_cast<char*>(dst), rows,
+                                        n, l.chunks, l.per, l.seg_pairs, pieces, first);
+      return hipGetLastError();
+    };
+    const hipError_t err = kind == 1 ? launch(pack_any_kernel<true>) : launch(pack_any_kernel<false>);
+    if (err != hipSuccess) return err;
+  }
+  return hipSuccess;
 }
 
 extern "C" int pck_bgemm_packed_any(int weight_kind, const void* Wp, const void* Xp, float* Y,
                                     int64_t m, int64_t n, int64_t batch, void* stream) {
   using namespace pck;
-  if ((weight_kind != 0 && weight_kind != 1) || !Wp || !Xp || !Y || m < 1 || batch < 1 || n < 1 ||
-      n > (int64_t{1} << 30) || reinterpret_cast<uintptr_t>(Y) % 4 != 0 ||
+  if ((weight_kind != 0 && weight_kind != 1) || !Wp || !Xp || !Y || m < 1 || batch < 1 ||
+      !any_fits(n) || reinterpret_cast<uintptr_t>(Y) % 4 != 0 ||
       reinterpret_cast<uintptr_t>(Wp) % 16 != 0 || reinterpret_cast<uintptr_t>(Xp) % 16 != 0)
     return hipErrorInvalidValue;
   const AnyLayout l = any_layout(n);
   const int64_t row_tiles = (m + 31) / 32;
   const int64_t batch_tiles = (batch + 31) / 32;
-  // One buffer resource covers one weight tile and one pass's batch tiles (32-bit offsets).
-  if (l.seg_pairs * kWaves * 2 * 32 * 16 * 4 > 0x7FFFFFFFll) return hipErrorInvalidValue;
   const bool quads = m % 4 == 0 && reinterpret_cast<uintptr_t>(Y) % 16 == 0;
   const PackedArgs a{static_cast<const char*>(Wp), static_cast<const char*>(Xp), Y, m, m,
                      l.chunks, l.seg_pairs, true, quads, batch, row_tiles, batch_tiles, 1};

@@ -104,10 +104,11 @@ def _validate_w(W: torch.Tensor) -> None:
 
 def pack_batched_weights(W: torch.Tensor) -> BatchedWeights:
     """Packs W (m, n) BF16 or float8_e4m3fn (raw codes) once for the packed kernel; enqueued on
-    the current stream.  Shapes with n % 128 != 0 or m % 4 != 0 also keep W as it is."""
+    the current stream.  Shapes with n % 128 != 0 or m % 4 != 0 also keep W as it is, and rows
+    longer than the padded tiles take (`pck_bgemm_any_columns`) only that."""
     _validate_w(W)
     m, n = W.shape
-    if m == 0 or n == 0:
+    if m == 0 or n == 0 or not _packable(m, n) and lib().pck_bgemm_any_columns(n) < 0:
         return BatchedWeights(m, n, W.dtype, None, W)
     if not _packable(m, n):
         return BatchedWeights(m, n, W.dtype, None, W, _pack_any(W, _kind(W.dtype)))

@@ -379,3 +379,20 @@ def test_padded_segments_give_the_element_kernels_bits(m: int, n: int, B: int, f
         assert torch.equal(got.view(torch.int32), want.view(torch.int32))
     if m * n * B < 10_000_000:
         assert _same_bits(_run(W, X, packed=True), emulate_batched(W, X))
+
+
+def test_operands_of_more_than_two_gib_take_the_packed_route() -> None:
+    """Ragged weights, and activations, whose tiles exceed 2 GiB: the products equal those of the
+    row-major element kernel bit for bit (the last rows lie past the 32-bit byte range)."""
+    n, rows = 8200, 131112  # 2.15e9 bytes of BF16
+    g = torch.Generator(device=DEV)
+    g.manual_seed(11)
+    big = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV).normal_(generator=g)
+    few = torch.randn(5, n, generator=g, device=DEV).bfloat16()
+    assert big.numel() * 2 > 2**31
+    bw = pack_batched_weights(big)
+    assert bw.padded is not None
+    assert torch.equal(gemm_batched(bw, few).view(torch.int32), gemm_batched(big, few).view(torch.int32))
+    del bw
+    got = gemm_batched(pack_batched_weights(few), big)
+    assert torch.equal(got.view(torch.int32), gemm_batched(few, big).view(torch.int32))

@@ -177,3 +177,14 @@ def test_batch_check_plan_rejects_what_32_bit_offsets_cannot_address() -> None:
     assert _workspace(_check_descs([(8, 4, 1 << 14, 1, 1 << 14)]))[0] != 0
     # X must be 16-byte aligned
     assert _workspace(_check_descs([(4096, 128, 32, 1, 128)], x_offset=8))[0] != 0
+
+
+def test_any_columns_names_every_row_length_the_padded_tiles_take() -> None:
+    """The query that packing decides by: -1 exactly where a batch tile's offsets leave 32 bits,
+    so such rows keep the row-major weights instead of failing in the product."""
+    columns = _lib.lib().pck_bgemm_any_columns
+    for n in (1, 7, 8, 128, 1000, 8192, 2**20 + 1):
+        assert columns(n) >= n and columns(n) % 128 == 0
+    assert columns(2**23 - 128) > 0
+    for n in (-1, 0, 2**23 - 127, 2**23, 2**30, 2**40):
+        assert columns(n) == -1
