@@ -11,7 +11,8 @@ Two routes with the same bits:
 - `gemm_batched(pack_batched_weights(W), X)` runs the packed kernel: the weights are packed
   once, at load time, into 32-row tiles whose matrix-core operands are contiguous, and each call
   packs X the same way into a workspace.  This is the decode path.  Shapes with n % 128 != 0 or
-  m % 4 != 0 take the form of the layout that pads each K segment to whole step pairs.
+  m % 4 != 0 take the form of the layout that pads each K segment to whole step pairs, except for
+  the short products that the element kernel finishes sooner (`_element_is_faster`).
 """
 
 from __future__ import annotations
@@ -43,7 +44,9 @@ def batched_height(n: int) -> int:
 class BatchedWeights:
     """Weights for `gemm_batched` in the packed 32-row tile layout (`packed` is None when n % 128
     != 0 or m % 4 != 0; `padded` then holds the tiles with each K segment padded to whole step
-    pairs and `raw` the weights as they were given)."""
+    pairs, and `raw` row-major weights where the element kernel is the faster one for some batch:
+    a copy, so that both routes compute with the weights as they were when packed).  Rows that the
+    padded tiles do not take have only `raw`, the weights themselves."""
 
     m: int
     n: int
@@ -54,7 +57,7 @@ class BatchedWeights:
 
     @property
     def device(self) -> torch.device:
-        t = self.packed if self.packed is not None else self.raw
+        t = next((t for t in (self.packed, self.padded) if t is not None), self.raw)
         assert t is not None
         return t.device
 
@@ -91,6 +94,22 @@ def _pack_any(src: torch.Tensor, kind: int) -> torch.Tensor:
     return dst
 
 
+def _element_is_faster(kind: int, m: int, n: int, B: int, vectors: bool = True) -> bool:
+    """Whether the element kernel's one launch beats the padded tiles' two (a pack of X, 2.5 us,
+    and the product).  Both times in ns beyond a launch of 2.6 us, fitted to 1,260 graph-replayed
+    products of m = 1 .. 14338, n = 7 .. 4100, B = 1 .. 256: per round of 256 workgroups the element
+    kernel reduces its outputs (B rows of up to 32) and walks n columns for each 32 rows of X, in
+    16-byte loads (``vectors``, n % 8 == 0) or element by element.  512 x 520, B = 3: 5.0 against
+    6.8 us; 4096 x 130, B = 1: 5.7 / 6.4, B = 32: 9.1 / 6.4; 512 x 1001, B = 3: 23.7 / 7.5.  By
+    this rule 5 of the 1,260 take more than 4% longer than the element kernel, 7% at most."""
+    if B > 128 or n > 1536:
+        return False
+    column = (5.0 if kind == 1 else 3.5) if vectors and n % 8 == 0 else 21.0
+    column = 0.75 * column if m < 8 else column
+    element = -(-m // 8192) * (B * (8 + 3.2 * min(m, 32)) + n * column * -(-B // 32))
+    return element < 3100 + 1.7 * n + 12 * B
+
+
 def _validate_w(W: torch.Tensor) -> None:
     if not W.is_cuda:
         raise RuntimeError("W must be a CUDA tensor")
@@ -104,14 +123,15 @@ def _validate_w(W: torch.Tensor) -> None:
 
 def pack_batched_weights(W: torch.Tensor) -> BatchedWeights:
     """Packs W (m, n) BF16 or float8_e4m3fn (raw codes) once for the packed kernel; enqueued on
-    the current stream.  Shapes with n % 128 != 0 or m % 4 != 0 also keep W as it is, and rows
-    longer than the padded tiles take (`pck_bgemm_any_columns`) only that."""
+    the current stream.  Later writes to W are not seen, except for rows longer than the padded
+    tiles take (n % 128 != 0 or m % 4 != 0, `pck_bgemm_any_columns`), which keep W as it is."""
     _validate_w(W)
     m, n = W.shape
     if m == 0 or n == 0 or not _packable(m, n) and lib().pck_bgemm_any_columns(n) < 0:
         return BatchedWeights(m, n, W.dtype, None, W)
     if not _packable(m, n):
-        return BatchedWeights(m, n, W.dtype, None, W, _pack_any(W, _kind(W.dtype)))
+        raw = W.detach().clone() if _element_is_faster(_kind(W.dtype), m, n, 1) else None
+        return BatchedWeights(m, n, W.dtype, None, raw, _pack_any(W, _kind(W.dtype)))
     return BatchedWeights(m, n, W.dtype, _pack(W, _kind(W.dtype)), None)
 
 
@@ -156,6 +176,8 @@ def gemm_batched(
         raise RuntimeError("n must be positive")
     kind = _kind(dtype)
     tiles = (W.packed if W.packed is not None else W.padded) if packed else None
+    if packed and W.raw is not None and _element_is_faster(kind, m, n, B, X.data_ptr() % 16 == 0):
+        tiles = None
     with on_device(device):
         if tiles is not None:
             columns = n if W.packed is not None else lib().pck_bgemm_any_columns(n)

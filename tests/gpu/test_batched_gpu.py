@@ -3,6 +3,7 @@ kernel's order, within the proven bound of the exact product, and the wrapper's 
 
 from __future__ import annotations
 
+from dataclasses import replace
 from fractions import Fraction
 
 import numpy as np
@@ -373,6 +374,7 @@ def test_padded_segments_give_the_element_kernels_bits(m: int, n: int, B: int, f
     for w in (Wt, Q):
         bw = pack_batched_weights(w)
         assert bw.padded is not None
+        bw = replace(bw, raw=None)  # the padded tiles also where the element kernel is faster
         got = gemm_batched(bw, Xt)
         want = gemm_batched(w, Xt)
         torch.cuda.synchronize()
@@ -396,3 +398,22 @@ def test_operands_of_more_than_two_gib_take_the_packed_route() -> None:
     del bw
     got = gemm_batched(pack_batched_weights(few), big)
     assert torch.equal(got.view(torch.int32), gemm_batched(few, big).view(torch.int32))
+
+
+@pytest.mark.parametrize(("m", "n"), [(1, 8), (7, 130), (34, 320), (300, 1001), (36, 1544), (66, 3000)])
+def test_ragged_weights_keep_rows_only_where_the_element_kernel_is_faster(m: int, n: int) -> None:
+    """Long rows hold one copy of the weights; short ones give the same bits by either route (the
+    batches lie on both sides of the rule), from the weights as they were when packed."""
+    rng = np.random.default_rng(m + n)
+    W = _bf16_tensor(_family(rng, (m, n), "real_w"))
+    bw = pack_batched_weights(W)
+    assert bw.padded is not None and bw.device == W.device
+    assert (bw.raw is not None) == (n <= 130 or n == 320)
+    for B in (1, 3, 32, 64, 129):
+        X = _bf16_tensor(_family(rng, (B, n), "real_x"))
+        want = gemm_batched(W, X)
+        kept = W.clone()
+        W.zero_()
+        got = gemm_batched(bw, X)
+        W.copy_(kept)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))
