@@ -21,8 +21,8 @@ extern "C" {
 /* y[i] = expf(x[i]) for i < n, compiled as the membership kernels compile it. */
 int pck_probe_expf(const float* x, float* y, int64_t n, void* stream);
 
-/* y[i] = 2^x[i] by v_exp_f32 for i < n, as the set checker issues it. */
-int pck_probe_exp2(const float* x, float* y, int64_t n, void* stream);
+/* y[i] = 2^(hi[i] + lo[i]) for i < n, as the set checker forms it; lo may be null (zeros). */
+int pck_probe_exp2(const float* hi, const float* lo, float* y, int64_t n, void* stream);
 
 /* Chains of v_mfma_f64_16x16x4_f64: a, b (tiles * steps * 64) doubles, c, d (tiles * 64 * 4). */
 int pck_probe_mfma_f64(const double* a, const double* b, const double* c, double* d,

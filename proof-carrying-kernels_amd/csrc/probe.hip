@@ -4,7 +4,7 @@
 //
 //   pck_probe_expf            y = expf(x), the FP32 exponential the membership kernels call (same
 //                             header, same flags, same code);
-//   pck_probe_exp2            v_exp_f32, the set checker's 2^hi;
+//   pck_probe_exp2            2^(hi + lo), the set checker's exponential (same header);
 //   pck_probe_mfma_f64        v_mfma_f64_16x16x4_f64 chains, as the batched checker runs c . x;
 //   pck_probe_mfma_bf16       v_mfma_f32_32x32x16_bf16 chains;
 //   pck_probe_mfma_bf16_k8    v_mfma_f32_32x32x8_bf16 chains (the batched product's step: one
@@ -24,6 +24,7 @@
 
 #include <cstdint>
 
+#include "exp2_term.h"
 #include "pck_probe.h"
 #include "rounding.h"
 
@@ -43,10 +44,11 @@ __global__ void __launch_bounds__(256) expf_kernel(const float* x, float* y, int
     y[i] = expf(x[i]);
 }
 
-__global__ void __launch_bounds__(256) exp2_kernel(const float* x, float* y, int64_t n) {
+__global__ void __launch_bounds__(256) exp2_kernel(const float* hi, const float* lo, float* y,
+                                                   int64_t n) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride)
-    y[i] = __builtin_amdgcn_exp2f(x[i]);
+    y[i] = pck::exp2_pair(hi[i], lo != nullptr ? lo[i] : 0.0f);
 }
 
 __global__ void __launch_bounds__(kWave) mfma_f64_kernel(const double* a, const double* b,
@@ -149,12 +151,12 @@ extern "C" int pck_probe_expf(const float* x, float* y, int64_t n, void* stream)
   return hipGetLastError();
 }
 
-extern "C" int pck_probe_exp2(const float* x, float* y, int64_t n, void* stream) {
-  if (n < 0 || (n > 0 && (x == nullptr || y == nullptr))) return hipErrorInvalidValue;
+extern "C" int pck_probe_exp2(const float* hi, const float* lo, float* y, int64_t n, void* stream) {
+  if (n < 0 || (n > 0 && (hi == nullptr || y == nullptr))) return hipErrorInvalidValue;
   if (n == 0) return hipSuccess;
   const int64_t blocks = (n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096;
   exp2_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                static_cast<hipStream_t>(stream)>>>(x, y, n);
+                static_cast<hipStream_t>(stream)>>>(hi, lo, y, n);
   return hipGetLastError();
 }
 

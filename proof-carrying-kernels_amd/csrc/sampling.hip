@@ -11,9 +11,9 @@
 //     logit, e = exp((l - M) / T), M the row maximum.  `slack` comes from the host: the
 //     sampler's declared error plus the bound below for this kernel's own rounding.
 // min(selected) and max(rejected) are exact (FP32 comparisons).  Each e is an FP32
-// 2^d on the split argument d = (l - m) log2(e) / T = hi + lo in two floats:
-// e = 2^hi (1 + lo ln 2), within a few FP32 ulps for every |d| (an FP32 argument alone would
-// lose |d| ulps), 0 for e < 2^-126 (masked -inf logits among them); the sums are FP64.
+// 2^d on the split argument d = (l - m) log2(e) / T = hi + lo in two floats, within 0.8 FP32 ulps
+// for every |d| (an FP32 argument alone would lose |d| ulps), 0 for e < 2^-150 (masked -inf logits
+// among them); the sums are FP64.
 //
 // Launches on the caller's stream; nothing depends on scheduling:
 //   mark:    (selections longer than kLdsSelect only) one lane per selected entry sets its bit
@@ -41,6 +41,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "exp2_term.h"
 #include "pck_hip.h"
 
 namespace pck {
@@ -168,12 +169,9 @@ __device__ __forceinline__ bool float_quotient(double temperature) {
   return temperature >= 0x1p-40 && temperature <= 0x1p40;
 }
 
-// e^((l - m) / T) = 2^d, d = hi + lo: the exponential unit's 2^hi (1 ulp for a normal result, 0
-// below 2^-126), corrected by lo (2^(hi + lo) = 2^hi (1 + lo ln 2 + ...), |lo| <= 2^-24 |hi|).
-// l - m is exact (Knuth's TwoSum) and the product with log2(e) / T within 2^-44 relative, so d is
-// within 2^-37 at |d| = 128 against the 2^-24 of the FP32 terms.  log2(e) rides in the constant,
-// so no term pays expf's own reduction: check_topp_gpu of 64 x 151,936 logits 20.9 us against 22.8
-// with expf of a base-e split, error of the masses against 64 bits unchanged (3e-10).
+// e^((l - m) / T) = 2^d, d = hi + lo (exp2_term.h).  l - m is exact (Knuth's TwoSum) and the product
+// with log2(e) / T within 2^-44 relative, so d is within 2^-36 at |d| = 150 against the 2^-24 of the
+// FP32 terms.  log2(e) rides in the constant, so no term pays a reduction of its own base.
 template <bool kFloats>
 __device__ __forceinline__ double term(float l, float m, const InvT& inv, double temperature) {
   float hi, lo;
@@ -186,16 +184,12 @@ __device__ __forceinline__ double term(float l, float m, const InvT& inv, double
     const float s = l + nm;
     const float bv = s - l;
     const float err = (l - (s - bv)) + (nm - bv);
-    const float p = s * inv.hi;
-    float e = __builtin_fmaf(s, inv.hi, -p);
-    e = __builtin_fmaf(s, inv.lo, e);
-    e = __builtin_fmaf(err, inv.hi, e);
-    hi = p + e;
-    lo = e - (hi - p);
+    hi = s * inv.hi;
+    lo = __builtin_fmaf(s, inv.hi, -hi);
+    lo = __builtin_fmaf(s, inv.lo, lo);
+    lo = __builtin_fmaf(err, inv.hi, lo);
   }
-  const float eh = __builtin_amdgcn_exp2f(hi);
-  // 2^hi is 0 there (and hi is -inf or NaN for -inf logits): 0; a NaN logit is flagged elsewhere
-  return hi >= -128.0f ? __builtin_fmaf(eh, lo * 0x1.62e430p-1f, eh) : 0.0f;
+  return exp2_pair(hi, lo);  // 0 for -inf logits; a NaN logit is flagged elsewhere
 }
 
 __device__ __forceinline__ float wave_min(float v) {

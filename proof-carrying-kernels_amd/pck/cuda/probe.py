@@ -23,7 +23,7 @@ LIBRARY = Path(__file__).resolve().parents[1] / "libpck_probe.so"
 _p, _i64, _int = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
 SIGNATURES = {
     "pck_probe_expf": [_p, _p, _i64, _p],
-    "pck_probe_exp2": [_p, _p, _i64, _p],
+    "pck_probe_exp2": [_p, _p, _p, _i64, _p],
     "pck_probe_mfma_f64": [_p, _p, _p, _p, _i64, _int, _p],
     "pck_probe_mfma_bf16": [_p, _p, _p, _p, _i64, _int, _p],
     "pck_probe_mfma_bf16_16x16": [_p, _p, _p, _p, _i64, _int, _p],
@@ -66,13 +66,16 @@ def expf(x: torch.Tensor) -> torch.Tensor:
     return y
 
 
-def exp2(x: torch.Tensor) -> torch.Tensor:
-    """``v_exp_f32`` (2^x) of every element of the FP32 CUDA tensor ``x``."""
+def exp2(x: torch.Tensor, lo: torch.Tensor | None = None) -> torch.Tensor:
+    """The set checker's 2^(x + lo) of every element of the FP32 CUDA tensors (``lo`` of x's
+    shape, or zeros)."""
     x = _cuda(x, torch.float32, tuple(x.shape), "x")
+    if lo is not None:
+        lo = _cuda(lo, torch.float32, tuple(x.shape), "lo")
     y = torch.empty_like(x)
     with torch.cuda.device(x.device):
-        check(lib().pck_probe_exp2(x.data_ptr(), y.data_ptr(), x.numel(), stream_handle(x.device)),
-              "exp2 probe")  # fmt: skip
+        check(lib().pck_probe_exp2(x.data_ptr(), None if lo is None else lo.data_ptr(), y.data_ptr(),
+                                   x.numel(), stream_handle(x.device)), "exp2 probe")  # fmt: skip
     return y
 
 

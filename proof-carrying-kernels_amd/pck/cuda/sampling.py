@@ -116,12 +116,12 @@ def check_topk_gpu(
 @functools.lru_cache(maxsize=256)
 def topp_slack(vocab: int, segments: int, tol: float) -> float:
     """The sampler's ``tol`` plus this checker's own rounding (reference
-    `cuda/sampling.py:71-88`): each term is an FP32 2^hi on a split argument (within 2 ulp, plus
-    under 2 u32 for the split and the FMA: 6 u32 relative) or below 2^-125 where dropped;
-    each of the S segment partials is rescaled with one FP64 exp, multiply and add; the
-    largest term is exactly 1.  Each mass is then within 16 u32 + V 2^-124 +
-    gamma_{V + 3S + 16}(u64), rounded up."""
-    own = 16 * U32 + math.ldexp(vocab, -124) + gamma(vocab + 3 * segments + 16, U64)
+    `cuda/sampling.py:71-88`): each term is an FP32 2^(hi + lo) within 0.8 ulp (6 u32 relative taken)
+    or below 2^-148 where subnormal or dropped; a term passes fewer than V + 3S FP64 additions and
+    roundings (at most V / 256 + 32 additions, V / 5120 + 1 rescalings to its wave's and segment's
+    maximum and one per segment to the row's, of three roundings each); the largest term is exactly
+    1.  Each mass is then within 16 u32 + V 2^-146 + gamma_{V + 3S + 16}(u64), rounded up."""
+    own = 16 * U32 + math.ldexp(vocab, -146) + gamma(vocab + 3 * segments + 16, U64)
     return math.nextafter(tol + own, math.inf)
 
 
