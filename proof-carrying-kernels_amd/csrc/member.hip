@@ -590,11 +590,15 @@ __global__ void __launch_bounds__(kThreads) member_kernel(const MemberArgs A) {
 //            their count, so ties, such as the -inf of masked logits, take no slots).  A row
 //            without a top-k adds the segments' sums scaled by exp(m_s - max) in FP64.
 // Orders are fixed (lane, wave, segment), nothing depends on scheduling.  A segment with more
-// than kSegSlots logits above its low, or more than kCap of them above G, sends the row to an
-// exact radix select over the row by the finish workgroup, as in the one-workgroup kernel.
+// logits above its low than slots, or more than kCap of them above G, sends the row to an exact
+// radix select over the row by the finish workgroup (130 us at 50,257 logits), so both are kept
+// rare.  A segment has a slot for each logit of one load of the workgroup (16 bytes a lane): finite
+// logits in a run no longer than that fit whatever their low is (-inf where a wave holds none of
+// them), a longer run reaches every lane, and in a row sorted by token id the logits above low lie
+// within one load.  The logits of a row's last, partial segment are dealt to the lanes one by one,
+// so 256 of them are enough for a low above -inf.
 constexpr int kSegThreads = 256;
 constexpr int kSegWaves = kSegThreads / kWave;
-constexpr int kSegSlots = 1024;
 constexpr int kFinishThreads = 256;
 constexpr int kFinishWaves = kFinishThreads / kWave;
 constexpr int64_t kSplitMaxK = 128;  // top-k values the lane maxima of a segment can bound
@@ -617,15 +621,17 @@ __device__ __forceinline__ float wave_bound(float v, int want) {
 enum class Logits { kF32, kBf16, kF16 };
 
 template <Logits kType>
-struct LogitType;
+struct LogitType;  // slots: one 16-byte load of the workgroup
 template <>
 struct LogitType<Logits::kF32> {
   typedef float type;
+  static constexpr int kSlots = kSegThreads * 4;
   static __device__ __forceinline__ float widen(float v) { return v; }
 };
 template <>
 struct LogitType<Logits::kBf16> {
   typedef uint16_t type;
+  static constexpr int kSlots = kSegThreads * 8;
   static __device__ __forceinline__ float widen(uint16_t v) {
     return __uint_as_float(static_cast<uint32_t>(v) << 16);
   }
@@ -633,13 +639,14 @@ struct LogitType<Logits::kBf16> {
 template <>
 struct LogitType<Logits::kF16> {
   typedef _Float16 type;
+  static constexpr int kSlots = kSegThreads * 8;
   static __device__ __forceinline__ float widen(_Float16 v) { return static_cast<float>(v); }
 };
 
 struct alignas(16) SegmentHeader {
   float max, low;
   uint32_t above, ties;  // logits above the token's; logits equal to low
-  uint32_t count;        // logits above low (the first kSegSlots are in the slots)
+  uint32_t count;        // logits above low (the first kSlots are in the slots)
   int flags;             // bit 0: a NaN
   double z, a;           // kept mass and mass above the token, relative to max (no top-k)
   uint64_t unused;
@@ -649,7 +656,7 @@ static_assert(sizeof(SegmentHeader) == 48, "three 16-byte words");
 struct SplitArgs {
   MemberArgs m;
   SegmentHeader* headers;  // (rows, segments)
-  float* slots;            // (rows, segments, kSegSlots), when any row has a top-k
+  float* slots;            // (rows, segments, kSlots), when any row has a top-k
   int64_t segments;
   int64_t length;  // logits per segment
 };
@@ -695,7 +702,7 @@ __global__ void __launch_bounds__(kSegThreads) member_segment_kernel(const Split
   } else {
 #pragma unroll
     for (int i = 0; i < kElems; ++i) {
-      const int64_t j = j0 + (i / kVec * kSegThreads + t) * kVec + i % kVec;
+      const int64_t j = j0 + i * kSegThreads + t;
       const float v = L::widen(row[j < vocab ? j : vocab - 1]);
       x[i] = j < vocab ? v : -inf;
     }
@@ -748,12 +755,12 @@ __global__ void __launch_bounds__(kSegThreads) member_segment_kernel(const Split
     __syncthreads();
     uint32_t at = incl - mine;
     for (int w = 0; w < wave; ++w) at += s.count[w];
-    float* slots = S.slots + static_cast<int64_t>(item) * kSegSlots;
+    float* slots = S.slots + static_cast<int64_t>(item) * L::kSlots;
     if (mine != 0) {
 #pragma unroll
       for (int i = 0; i < kElems; ++i) {
         if (x[i] > low) {
-          if (at < kSegSlots) slots[at] = x[i];
+          if (at < L::kSlots) slots[at] = x[i];
           ++at;
         }
       }
@@ -808,7 +815,7 @@ __global__ void __launch_bounds__(kFinishThreads) member_finish_kernel(const Spl
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(wave_id());
   const int64_t n = S.segments;
   const SegmentHeader* hs = S.headers + r * n;
-  const float* slots = S.slots + r * n * kSegSlots;
+  const float* slots = S.slots + r * n * L::kSlots;
   const float inf = __builtin_inff();
   // Lane i of wave w holds the header of segment w + 4 i; the first slots of the wave's first
   // segments are requested with the headers (what they hold past a segment's count is not used).
@@ -824,7 +831,7 @@ __global__ void __launch_bounds__(kFinishThreads) member_finish_kernel(const Spl
       const int64_t seg = wave + static_cast<int64_t>(i) * kFinishWaves;
 #pragma unroll
       for (int d = 0; d < kDeep; ++d)
-        early[i][d] = slots[(seg < n ? seg : 0) * kSegSlots + d * kWave + lane];
+        early[i][d] = slots[(seg < n ? seg : 0) * L::kSlots + d * kWave + lane];
     }
   }
   const RowRequest q = row_request(A, r);
@@ -843,7 +850,7 @@ __global__ void __launch_bounds__(kFinishThreads) member_finish_kernel(const Spl
   float m = -inf, low = -inf;
   headers([&](const SegmentHeader& h) {
     above32 += h.above;
-    flags |= h.flags | (h.count > kSegSlots ? 2 : 0) | (h.count > kDeep * kWave ? 4 : 0);
+    flags |= h.flags | (h.count > L::kSlots ? 2 : 0) | (h.count > kDeep * kWave ? 4 : 0);
     m = fmaxf(m, h.max);
     low = fmaxf(low, h.low);
   });
@@ -919,7 +926,7 @@ __global__ void __launch_bounds__(kFinishThreads) member_finish_kernel(const Spl
             const int count = static_cast<int>(
                 i < kWave ? read_lane(mine_h.count, static_cast<int>(i)) : hs[seg].count);
             for (int j = i < kEarly ? kDeep * kWave : 0; j < count; j += kWave) {
-              const float v = slots[seg * kSegSlots + (j + lane < count ? j + lane : count - 1)];
+              const float v = slots[seg * L::kSlots + (j + lane < count ? j + lane : count - 1)];
               f(j + lane < count ? v : -inf);
             }
           }
@@ -1109,9 +1116,11 @@ SplitPlan split_plan(const PckMemberArgs& a, int kind) {
   if (a.rows * segments > 0x7FFFFFFF / kSegThreads) return p;
   p.length = length;
   p.segments = segments;
+  const int64_t slots =
+      kind == 0 ? LogitType<Logits::kF32>::kSlots : LogitType<Logits::kBf16>::kSlots;
   p.header_bytes = a.rows * segments * static_cast<int64_t>(sizeof(SegmentHeader));
   p.bytes = p.header_bytes +
-            (cut ? a.rows * segments * kSegSlots * static_cast<int64_t>(sizeof(float)) : 0);
+            (cut ? a.rows * segments * slots * static_cast<int64_t>(sizeof(float)) : 0);
   return p;
 }
 

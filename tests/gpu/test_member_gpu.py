@@ -7,11 +7,14 @@ tokens replaced by out-of-set tokens that must all be flagged, with no false ala
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle.member import check_member, check_members_ref
+from pck.cuda._lib import PckMemberArgs, lib
 from pck.member import check_members, member_eps32
 
 pytestmark = [
@@ -261,7 +264,7 @@ def test_request_index_outside_the_temperature_array_rejects_the_row() -> None:
     assert int(totals[0]) == rows and int(totals[1]) == 2
 
 
-SPLIT_CASES = ["plain", "ties", "masked", "all_masked", "nan", "sorted", "overflow", "mixed"]
+SPLIT_CASES = ["plain", "ties", "masked", "all_masked", "nan", "sorted", "overflow", "overflow16", "mixed"]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
@@ -288,8 +291,10 @@ def test_rows_split_over_workgroups_match_the_oracle(case: str, vocab: int, dtyp
         logits[::2, vocab - 1] = np.nan
     elif case == "sorted":
         logits[:] = 5.0 - (np.arange(vocab) % 8192) * 2.0**-9 + np.arange(rows)[:, None]
-    elif case == "overflow":
+    elif case == "overflow":  # the fourth wave's FP32 logits
         logits[:, np.arange(vocab) % 1024 >= 768] = -50.0
+    elif case == "overflow16":  # its 16-bit ones
+        logits[:, np.arange(vocab) % 2048 >= 1536] = -50.0
     t = torch.from_numpy(logits).to(dtype)
     host = t.float().numpy()
     order = np.argsort(-np.nan_to_num(host, nan=-1e30), axis=1, kind="stable")
@@ -307,3 +312,41 @@ def test_rows_split_over_workgroups_match_the_oracle(case: str, vocab: int, dtyp
             finite = np.isfinite(want["mass_above"]) & ~np.isnan(host).any(axis=1)
             err = np.abs(got["mass_above"] - want["mass_above"])[finite]
             assert np.all(err <= 2 * member_eps32(vocab))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("tail", [1, 255, 257, 1105, 1600, 8191])
+@pytest.mark.parametrize("case", ["plain", "sorted", "run"])
+def test_candidates_of_ordinary_rows_fit_their_slots(case: str, tail: int, dtype: torch.dtype) -> None:
+    """Rows whose last segment holds ``tail`` logits; logits sorted by token id; finite logits only
+    in runs of 1,105.  No segment may have more logits above its bound than slots (the row would be
+    selected again from memory, ten times slower), read from the headers of a workspace that the
+    test holds: 48 bytes a segment, the count at byte 16, then the FP32 slots."""
+    rows, vocab, k = 3, 12 * 8192 + tail, 50
+    g = torch.Generator(device="cuda")
+    g.manual_seed(tail)
+    logits = torch.randn((rows, vocab), generator=g, device="cuda") * 3
+    if case == "sorted":
+        logits = logits.sort(dim=1, descending=True).values
+    elif case == "run":
+        logits[:, torch.arange(vocab, device="cuda") % 8192 >= 1105] = -torch.inf
+    logits = logits.to(dtype).contiguous()
+    tokens = logits.float().argmax(1)
+    top_k = torch.full((rows,), k, device="cuda")
+    top_p = torch.full((rows,), 0.9, dtype=torch.float64, device="cuda")
+    ok = torch.empty(rows, dtype=torch.bool, device="cuda")
+    args = PckMemberArgs(logits=logits.data_ptr(), rows=rows, vocab=vocab, tokens=tokens.data_ptr(),
+                         top_k=top_k.data_ptr(), k_lim=k, all_k=1, top_p=top_p.data_ptr(),
+                         slack=1e-4, ok=ok.data_ptr())  # fmt: skip
+    kind = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype]
+    need = ctypes.c_int64(0)
+    assert lib().pck_check_members_workspace(args, kind, ctypes.byref(need)) == 0 and need.value > 0
+    work = torch.zeros(need.value, dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib().pck_check_members_split(args, kind, work.data_ptr(), need.value, stream) == 0
+    torch.cuda.synchronize()
+    assert bool(ok.all())
+    segments = rows * 13
+    slots = (need.value - 48 * segments) // (4 * segments)
+    counts = work[: 48 * segments].view(torch.int32).view(segments, 12)[:, 4]
+    assert int(counts.max()) <= slots, (slots, counts.tolist())
