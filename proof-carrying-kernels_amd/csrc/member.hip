@@ -354,10 +354,15 @@ struct RowRequest {
   int64_t k_eff;
 };
 
-__device__ __forceinline__ RowRequest row_request(const MemberArgs& A, int64_t r) {
+// The token first, for the kernel that reads its logit ahead of the rest of the request.
+__device__ __forceinline__ RowRequest row_token(const MemberArgs& A, int64_t r) {
   RowRequest q;
   q.token = A.tokens[r];
   q.in_range = q.token >= 0 && q.token < A.vocab;
+  return q;
+}
+
+__device__ __forceinline__ RowRequest row_request(const MemberArgs& A, int64_t r, RowRequest q) {
   const int64_t k_req = A.top_k ? A.top_k[r] : A.vocab;
   q.k_row = k_req < 1 ? 1 : (k_req > A.vocab ? A.vocab : k_req);
   // Greedy rows: the caller's flags, or temperature 0 of the row's request (vLLM's sampling
@@ -415,8 +420,9 @@ __global__ void __launch_bounds__(kThreads) member_kernel(const MemberArgs A) {
   const int64_t vocab = A.vocab;
   const float* __restrict__ row = A.logits + r * vocab;
 
-  const RowRequest q = row_request(A, r);
-  const float lt = row[q.in_range ? q.token : (q.token < 0 ? 0 : vocab - 1)];
+  const RowRequest asked = row_token(A, r);
+  const float lt = row[asked.in_range ? asked.token : (asked.token < 0 ? 0 : vocab - 1)];
+  const RowRequest q = row_request(A, r, asked);
   const bool want_mass = q.want_mass, use_kth = q.use_kth;
   const int64_t k_eff = q.k_eff;
   const bool fused = want_mass && use_kth && k_eff <= kThreads;
@@ -707,7 +713,7 @@ __global__ void __launch_bounds__(kSegThreads) member_segment_kernel(const Split
       x[i] = j < vocab ? v : -inf;
     }
   }
-  const RowRequest q = row_request(A, r);
+  const RowRequest q = row_request(A, r, row_token(A, r));
   const float lt = L::widen(row[q.in_range ? q.token : (q.token < 0 ? 0 : vocab - 1)]);
 
   uint32_t above = 0;
@@ -834,7 +840,7 @@ __global__ void __launch_bounds__(kFinishThreads) member_finish_kernel(const Spl
         early[i][d] = slots[(seg < n ? seg : 0) * L::kSlots + d * kWave + lane];
     }
   }
-  const RowRequest q = row_request(A, r);
+  const RowRequest q = row_request(A, r, row_token(A, r));
   const int64_t vocab = A.vocab;
   const T* __restrict__ row = reinterpret_cast<const T*>(A.logits) + r * vocab;
   const float lt = L::widen(row[q.in_range ? q.token : (q.token < 0 ? 0 : vocab - 1)]);
@@ -1086,28 +1092,55 @@ hipError_t validate(const PckMemberArgs* args) {
 }
 
 // The split of a batch: logits per segment, segments per row and the workspace (0 bytes: the
-// one-workgroup kernel).  FP32 rows split where that is faster; 16-bit logits always do, since
-// the one-workgroup kernel would need them converted first.  Measured on 151,936 logits a row,
-// one workgroup against split (us; top-k 50 + top-p / top-p only / top-k only):
-//   1 row     21.5 / 10.7    38.8 / 6.2     11.2 / 5.0
-//   64 rows   25.8 / 17.3    44.4 / 17.6    15.7 / 11.6
-//   128 rows  29.3 / 23.9    48.0 / 25.8    18.5 / 17.2
-//   256 rows  34.0 / 36.4    62.2 / 46.1    28.4 / 28.8
-// A row that keeps everything is read once instead of twice at any batch size; the others gain
-// while the rows leave compute units idle.  Short rows (16,384 logits: 9.8 / 10.6, 7.7 / 6.7 us)
-// lose to the second launch first where a k-th logit is selected.
+// one-workgroup kernel).  Each line of splits() is where the split stops being the faster one, by
+// both routes timed at 24 vocabularies from 100 to 262,144 and 1 to 384 rows.  Time of the split
+// relative to one workgroup per row, FP32 rows at 16-byte addresses:
+//                     4 rows   64 rows   128 rows   256 rows
+//   top-k alone
+//     32,000          1.08      1.11      1.18       1.13
+//     65,536          0.88      1.01      1.12       1.07
+//     151,936         0.58      0.75      0.96       1.02
+//   top-k and top-p
+//     24,576          1.00      1.04      1.09       1.06
+//     32,000          0.97      0.98      1.04       1.05
+//     151,936         0.54      0.67      0.91       1.11
+//   top-p alone
+//     12,000          0.91      0.96      1.01       1.11
+//     16,384          0.89      0.94      1.06       1.09
+//     24,576          0.69      0.82      0.85       0.94
+//   top-p, a top-k in some rows
+//     24,576          1.03      1.09      1.14       1.15
+//     32,000          0.95      1.00      1.01       1.09
+//     40,000          0.82      0.86      0.94       0.99
+// Rows at other addresses make the one-workgroup kernel two to four times slower from 20,000
+// logits, the segments hardly at all (20,001: 0.75 to 1.05, 151,937: 0.18 to 0.40).  16-bit logits
+// cost that kernel a conversion first; the split is faster but for cut rows too short to fill a
+// segment, up to a workgroup per compute unit (1,000 logits 1.10, 4,096 0.98).
 // Segments are 8,192 logits (their candidates are what the finish reads), shorter ones only
 // where no row is cut and the batch would not fill the GPU.
 struct SplitPlan {
   int64_t length = 0, segments = 0, header_bytes = 0, bytes = 0;
 };
 
+bool splits(const PckMemberArgs& a, int kind, bool cut, bool keeps_all) {
+  if (kind != 0) return !cut || a.vocab >= 4096 || a.rows > 256;
+  if (reinterpret_cast<uintptr_t>(a.logits) % 16 != 0 || (a.vocab % 4 != 0 && a.rows > 1)) {
+    if (keeps_all) return a.vocab >= (cut ? 20000 : 16384);
+    return a.vocab >= 20000 && a.rows < 192;
+  }
+  if (keeps_all)
+    return cut ? a.vocab >= 40000 || (a.vocab >= 32000 && a.rows <= 96)
+               : a.vocab >= 24576 || (a.vocab >= 16384 && a.rows <= 96);
+  if (cut) return a.vocab >= 32000 && a.rows <= 160 && a.rows <= a.vocab / 512;
+  return a.vocab >= 65536 && a.rows <= 128 && a.rows <= (a.vocab - 32768) / 1024;
+}
+
 SplitPlan split_plan(const PckMemberArgs& a, int kind) {
   SplitPlan p;
   if (a.rows < 1) return p;
   const bool cut = a.top_p != nullptr && a.k_lim > 0;     // a row may be cut at its k-th logit
   const bool keeps_all = a.top_p != nullptr && !a.all_k;  // a row may keep every logit
-  if (kind == 0 && !(keeps_all ? a.vocab >= 16384 : a.vocab >= 24576 && a.rows < 192)) return p;
+  if (!splits(a, kind, cut, keeps_all)) return p;
   int64_t length = 8192;
   while (!cut && length > 2048 && a.rows * ((a.vocab + length - 1) / length) < 1024) length /= 2;
   const int64_t segments = (a.vocab + length - 1) / length;

@@ -188,3 +188,30 @@ def test_any_columns_names_every_row_length_the_padded_tiles_take() -> None:
     assert columns(2**23 - 128) > 0
     for n in (-1, 0, 2**23 - 127, 2**23, 2**30, 2**40):
         assert columns(n) == -1
+
+
+def test_membership_plan_splits_rows_only_where_that_is_faster() -> None:
+    """Both sides of each line of the plan: FP32 rows at 16-byte and at other addresses, top-k alone
+    ("k"), with a top-p ("kp"), in some rows ("mix"), top-p alone ("p"); 16-bit rows.  Pure host code:
+    the pointers are never read."""
+
+    def split(rows: int, vocab: int, opt: str, kind: int = 0, address: int = 4096) -> bool:
+        a = _lib.PckMemberArgs(logits=address, rows=rows, vocab=vocab, tokens=8, slack=1e-4)
+        if opt != "p":
+            a.top_k, a.k_lim, a.all_k = 8, 50, int(opt != "mix")
+        if opt != "k":
+            a.top_p = 8
+        need = ctypes.c_int64(-1)
+        assert _lib.lib().pck_check_members_workspace(a, kind, ctypes.byref(need)) == 0
+        return need.value > 0
+
+    one = [(128, 24576, "k"), (191, 32000, "k"), (64, 50256, "k"), (64, 65536, "k"), (160, 151936, "k"),
+           (16, 24576, "kp"), (128, 32000, "kp"), (161, 151936, "kp"), (64, 24576, "mix"), (128, 32000, "mix"),
+           (192, 16384, "p"), (4, 12000, "p"), (1, 32001, "k"), (64, 16385, "k"), (192, 151937, "k")]  # fmt: skip
+    two = [(4, 65536, "k"), (64, 151936, "k"), (62, 32000, "kp"), (128, 151936, "kp"), (96, 32000, "mix"),
+           (256, 40000, "mix"), (96, 16384, "p"), (512, 24576, "p"), (64, 20001, "k"), (191, 151937, "kp"),
+           (256, 20001, "mix"), (256, 16385, "p")]  # fmt: skip
+    assert [c for c in one if split(*c)] == [] and [c for c in two if not split(*c)] == []
+    assert split(64, 24576, "kp", address=4100) and not split(64, 24576, "kp")
+    assert split(64, 1000, "k", kind=1) and split(64, 1000, "p", kind=2) and split(257, 1000, "kp", kind=1)
+    assert split(64, 4096, "kp", kind=1) and not split(64, 4095, "kp", kind=1)
