@@ -27,9 +27,9 @@ extern "C" {
 
 /* ---------------------------------------------------------------------------------------------
  * GEMV y = W x: W (m, n) row-major, x (n,) BF16, y (m,) FP32.  1 <= threads <= 1024, a power of
- * two (>= 32 for the coalesced kernels).  The coalesced kernels use 16-byte loads for every n of
- * at least one vector, at any address (no byte outside W and x is read); shorter rows, and the
- * naive kernel's rows that are not whole aligned vectors, use element loads with identical bits.
+ * two (>= 32 for the coalesced kernels).  All use 16-byte loads for every n of at least one vector,
+ * at any address (no byte outside W and x is read); shorter rows, and the naive kernel's chunks of
+ * under four columns, use element loads with identical bits.
  * -------------------------------------------------------------------------------------------*/
 
 /* BF16 weights, naive tree (contiguous chunk per lane, then neighbour pairs).

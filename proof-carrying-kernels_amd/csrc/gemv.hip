@@ -515,7 +515,8 @@ __global__ void __launch_bounds__(kGroupThreads)
 // (16) or a read of lane 32 (32); the lanes that matter at a level read only lanes that
 // mattered at the level before, so lane 0 ends with the wave's subtree.  The levels of stride 64
 // and up combine the T / 64 wave sums, which meet in LDS behind one barrier, in the same pair
-// order.  kLoad: kAligned, 16-byte loads of chunks that are whole aligned vectors; kUnaligned, the
+// order.  kLoad: kAligned, 16-byte loads of chunks that are whole aligned vectors, none past n (the
+// chain's arithmetic bounds short rows, so a vector carries no bounds of its own); kUnaligned, the
 // same at any 2-byte address (n >= 8), where a chunk's columns past its last whole vector, and
 // vectors that cross n, are read as 16 bytes inside the row and moved into place, so no lane takes
 // element loads; kElement, element loads, for chunks of fewer than four columns (a wave's lanes
@@ -532,13 +533,35 @@ __global__ void __launch_bounds__(1024)
   const uint16_t* rows[R];
 #pragma unroll
   for (int r = 0; r < R; ++r)  // rows past m compute on row m - 1 and are not stored
-    rows[r] = W + (row0 + r < m ? row0 + r : m - 1) * n;
+    rows[r] = W + (R == 1 || row0 + r < m ? row0 + r : m - 1) * n;
 
   float acc[R];  // -0.0 + p0 is p0: the chain starts from its first product
 #pragma unroll
   for (int r = 0; r < R; ++r) acc[r] = -0.0f;
-  if constexpr (kLoad != Load::kElement) {
-    constexpr bool kAny = kLoad == Load::kUnaligned;
+  auto add8 = [&](float& sum, const uint4& w, const uint4& xv) {
+    const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+    const uint32_t xd[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      sum = sum + bf16_lo(wd[k]) * bf16_lo(xd[k]);
+      sum = sum + bf16_hi(wd[k]) * bf16_hi(xd[k]);
+    }
+  };
+  if constexpr (kLoad == Load::kAligned) {
+    for (int64_t v = 0; v < chunk; v += 8) {
+      const int64_t col = first + v;
+      uint4 wv[R], xv = make_uint4(0, 0, 0, 0);  // past n: +0 products
+#pragma unroll
+      for (int r = 0; r < R; ++r) wv[r] = make_uint4(0, 0, 0, 0);
+      if (col < n) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) wv[r] = load16<false, false>(rows[r] + col);
+        xv = load16<false, false>(x + col);
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) add8(acc[r], wv[r], xv);
+    }
+  } else if constexpr (kLoad == Load::kUnaligned) {
     // columns col .. col + 7 of x and of the rows (+0 past n)
     struct Vectors {
       uint4 x, w[R];
@@ -546,9 +569,9 @@ __global__ void __launch_bounds__(1024)
     auto load = [&](int64_t col) {
       const int64_t at = col < n - 8 ? col : n - 8;
       Vectors v;
-      v.x = load16<false, kAny>(x + at);
+      v.x = load16<false, true>(x + at);
 #pragma unroll
-      for (int r = 0; r < R; ++r) v.w[r] = load16<false, kAny>(rows[r] + at);
+      for (int r = 0; r < R; ++r) v.w[r] = load16<false, true>(rows[r] + at);
       return v;
     };
     auto add = [&](Vectors& v, int64_t col, int count) {  // the first `count` columns
@@ -581,14 +604,12 @@ __global__ void __launch_bounds__(1024)
       else add(a, first + c, static_cast<int>(chunk - c));
     }
   } else {
+    static_assert(R == 1);
     for (int64_t j = first; j < first + chunk; ++j) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float p = 0.0f;
-        if (j < n) p = __uint_as_float(static_cast<uint32_t>(rows[r][j]) << 16) *
-                       __uint_as_float(static_cast<uint32_t>(x[j]) << 16);
-        acc[r] = acc[r] + p;
-      }
+      float p = 0.0f;
+      if (j < n) p = __uint_as_float(static_cast<uint32_t>(rows[0][j]) << 16) *
+                     __uint_as_float(static_cast<uint32_t>(x[j]) << 16);
+      acc[0] = j == first ? p : acc[0] + p;
     }
   }
 
@@ -1023,14 +1044,17 @@ int pck_gemv_bf16_naive(const void* W, const void* x, float* y, int64_t m, int64
   const bool aligned = chunk % 8 == 0 && n % 8 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(x) % 16 == 0;
   const Load load = n < 8 || chunk < 4 ? Load::kElement : aligned ? Load::kAligned : Load::kUnaligned;
-  // Four rows per workgroup for many short aligned chunks (14336 x 4096 at T = 256: 24.3 against
-  // 25.7 us with one; longer chunks of several rows push each other out of the L1: 4096 x 14336
-  // 84 against 58) and for ragged ones (14536 x 3647 at T = 512: 23 against 100 us with element
-  // loads; 7182 x 8960, T = 256: 55 against 212).
-  const bool four = load == Load::kUnaligned ? m >= 2048
-                                             : load == Load::kAligned && chunk <= 16 && m >= 8192 &&
-                                                   threads >= 256;
-  const int rows = four ? 4 : 1;
+  // Rows per workgroup, from 8192 rows on (fewer leave too few workgroups).  Aligned chunks of one
+  // vector: four (14336 x 4096, T = 512: 22.4 against 25.1 us with one; 8192 x 2048, T = 256, from
+  // the caches: 5.5 / 6.3); of two: two, since four rows' loads push each other out of the L1 (14336 x
+  // 4096, T = 256, from HBM 26.1 / 26.8 with two, from the caches 20.1 with four, 19.0 with two, 18.7
+  // with one); longer ones: one (4096 x 14336: 84 us with four, 58 with one).  Ragged chunks: four
+  // (7182 x 8960, T = 256: 55 against 212 us with element loads), with fewer rows only where those are
+  // long enough to be bound by their loads (3000 x 512, T = 128: equal; 2048 x 512: 3.9 / 3.1).
+  const bool many = load == Load::kUnaligned
+                        ? m >= 8192 || (m >= 2048 && m * n >= 1500000)
+                        : load == Load::kAligned && chunk <= 16 && m >= 8192 && threads >= 256;
+  const int rows = !many ? 1 : load == Load::kAligned && chunk > 8 ? 2 : 4;
   const dim3 grid(static_cast<unsigned>((m + rows - 1) / rows)), group(static_cast<unsigned>(lanes));
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const auto* w16 = static_cast<const uint16_t*>(W);
@@ -1041,9 +1065,10 @@ int pck_gemv_bf16_naive(const void* W, const void* x, float* y, int64_t m, int64
   };
   if (load == Load::kElement) return launch(pck::gemv_naive_kernel<Load::kElement, 1>);
   if (load == Load::kAligned)
-    return four ? launch(pck::gemv_naive_kernel<Load::kAligned, 4>)
-                : launch(pck::gemv_naive_kernel<Load::kAligned, 1>);
-  return four ? launch(pck::gemv_naive_kernel<Load::kUnaligned, 4>)
+    return rows == 4   ? launch(pck::gemv_naive_kernel<Load::kAligned, 4>)
+           : rows == 2 ? launch(pck::gemv_naive_kernel<Load::kAligned, 2>)
+                       : launch(pck::gemv_naive_kernel<Load::kAligned, 1>);
+  return many ? launch(pck::gemv_naive_kernel<Load::kUnaligned, 4>)
               : launch(pck::gemv_naive_kernel<Load::kUnaligned, 1>);
 }
 

@@ -104,10 +104,10 @@ def test_naive_vector_and_element_paths(m: int, n: int, threads: int) -> None:
     assert_bits(run(KERNELS[0], W, x, threads), emulate_gemv(W, x, threads))
 
 
-# (m, n, threads): four rows per workgroup with a last partial one (ragged and aligned chunks),
-# chunks of 3 (element loads), 4, 17 and 8 k + 1 columns, lanes wholly past n, one vector per row.
+# (m, n, threads): four rows per workgroup with a last partial one (ragged and aligned chunks), two
+# (8195 x 4096), chunks of 3 (element loads), 4, 17 and 8 k + 1 columns, lanes wholly past n, one vector per row.
 @pytest.mark.parametrize(("m", "n", "threads"), [(2051, 1003, 64), (2050, 4100, 256), (8195, 4096, 256),
-                                                 (7, 3072, 1024), (7, 4099, 1024), (5, 9, 1), (6, 8, 2),
+                                                 (8195, 2048, 256), (7, 3072, 1024), (7, 4099, 1024), (5, 9, 1), (6, 8, 2),
                                                  (5, 2049, 32)])  # fmt: skip
 def test_naive_rows_of_any_length_and_address(m: int, n: int, threads: int) -> None:
     """Against the C model; W and x start one and three elements into NaN-filled buffers, so a
