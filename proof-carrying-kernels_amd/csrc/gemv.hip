@@ -278,13 +278,21 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
   while (g + 1 < batch.count && group >= batch.first_group[g + 1]) ++g;
   const GemvItem& it = batch.item[g];
   const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
-  const int64_t wave =
-      (group - batch.first_group[g]) * kWavesPerGroup + (static_cast<int>(threadIdx.x) >> 6);
-  const int slot = lane / kLanesPerRow;
-  const int chain0 = lane % kLanesPerRow;
+  const int64_t first_group = batch.first_group[g];
+  const int64_t m = it.m;
   const int64_t n = it.n;
   const int64_t P = it.per_lane;
+  const void* W = it.W;
   const uint16_t* __restrict__ x = it.x;
+  // BF16: everything ahead of the first load in one round trip to the scalar cache, not the three
+  // that the scheduler forms (512 x 1024, T = 64: 2.69 against 2.95 us; the FP8 kernels, whose loads
+  // it orders well, would lose 3%).
+  if constexpr (!kFp8)
+    __asm__ volatile("" ::"s"(first_group), "s"(m), "s"(n), "s"(P), "s"(W), "s"(x));
+  const int64_t wave =
+      (group - first_group) * kWavesPerGroup + (static_cast<int>(threadIdx.x) >> 6);
+  const int slot = lane / kLanesPerRow;
+  const int chain0 = lane % kLanesPerRow;
 
   // Rows past m compute on row m - 1 (a valid address) and are not stored.
   const unsigned char* w_rows[R];
@@ -292,9 +300,8 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int64_t row = (wave * kSlots + slot) * R + r;
-    live[r] = row < it.m;
-    w_rows[r] =
-        static_cast<const unsigned char*>(it.W) + (live[r] ? row : it.m - 1) * n * kElemBytes;
+    live[r] = row < m;
+    w_rows[r] = static_cast<const unsigned char*>(W) + (live[r] ? row : m - 1) * n * kElemBytes;
   }
 
   // Row scales of a scaled FP8 item, loaded ahead of the weight stream so that their latency
@@ -303,7 +310,7 @@ __device__ __forceinline__ void gemv_rows(const GemvBatch& batch, int64_t group)
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int64_t row = (wave * kSlots + slot) * R + r;
-    scale[r] = (kFp8 && it.y_scaled != nullptr) ? it.scale[live[r] ? row : it.m - 1] : 1.0f;
+    scale[r] = (kFp8 && it.y_scaled != nullptr) ? it.scale[live[r] ? row : m - 1] : 1.0f;
   }
 
   float acc[R][kLive];
@@ -659,8 +666,8 @@ __global__ void __launch_bounds__(1024)
 
 // Launch shape of the coalesced kernel: rows per wave slot, vector positions loaded ahead and
 // non-temporal weight loads.  T = 256 with aligned rows (the reference's default tree) has every
-// combination instantiated for tuning; every other route has the one or two shapes it uses, with
-// non-temporal weight loads.
+// combination instantiated for tuning; every other route has only the shapes it uses (aligned rows
+// of T != 256 with non-temporal or plain weight loads, kCachedBytes; the others non-temporal).
 struct TreeShape {
   int rows;
   int unroll;
@@ -680,22 +687,29 @@ TreeShape g_shape_override = {0, 0, 0};
 //     with two rows, 3573 x 13824: 20.2 against 19.2; 1024 x 14336: 8.5 against 11.4).
 //   FP8 rows are half as long, so two rows per wave keep as many bytes in flight as one BF16 row;
 //     one row per wave below 2048 rows (1024 x 14336: 6.8 against 8.6 us), for rows of one
-//     position up to 4096 rows (o: 4.9 against 5.4 us) and of two up to 3072.
+//     position up to 4096 rows (o: 4.9 against 5.4 us) and of two up to 3072, these with both
+//     positions ahead below 1536 rows (256 x 8192: 4.1 against 4.35).
 TreeShape choose_shape(int64_t per_lane, int64_t rows, bool fp8) {
   if (g_shape_override.rows > 0) return g_shape_override;
   if (!fp8) {
     if (per_lane <= 2 || rows < 1536) return TreeShape{1, 2, 1};
     return rows <= 3072 ? TreeShape{1, 1, 1} : TreeShape{2, 1, 1};
   }
-  if (per_lane == 1 && rows <= 4096) return TreeShape{1, 2, 1};
+  if ((per_lane == 1 && rows <= 4096) || (per_lane == 2 && rows < 1536)) return TreeShape{1, 2, 1};
   if (rows < 2048 || (per_lane == 2 && rows <= 3072)) return TreeShape{1, 1, 1};
   return TreeShape{2, 1, 1};
 }
 
-// Trees of T != 256 lanes read aligned weights with plain loads where a launch's weights may
-// still be in the 256 MB Infinity Cache at the next call on them (below a third of it, as when one matrix
-// is evaluated again and again: 2653 x 11376, T = 512, three copies in turn, 14.0 against 15.8
-// us), and with non-temporal ones above (14336 x 4096, T = 512, from HBM: 20.0 against 21.8).
+// Trees of T != 256 lanes read aligned weights with plain loads below this size and with
+// non-temporal ones (and more rows or positions per wave) from it on.  A launch cannot see whether
+// its weights still lie in the 256 MB Infinity Cache, only what its own size allows: a pass that
+// uses three or more such matrices in turn (a decode layer's launches are four) cannot keep them
+// from a third of the cache on.  Below it either may be true, and there a wrong non-temporal load
+// costs more than a wrong plain one.  Aligned launches of 64 .. 14336 rows and 512 .. 14336 columns
+// at T = 32, 64 and 128, non-temporal against plain loads, time streamed from HBM / of one matrix
+// again and again (geometric mean, range over launches):
+//   below 85 MiB   0.95 (0.73 .. 1.37) / 1.14 (0.91 .. 1.63)
+//   from 85 MiB    0.89 (0.77 .. 0.98) / 1.05 (0.98 .. 1.19)
 // T = 256 is the decode path, which streams its weights: non-temporal.
 constexpr int64_t kCachedBytes = int64_t{85} << 20;
 
@@ -715,7 +729,7 @@ struct GroupPlan {
   GemvBatch batch{};
   Load load = Load::kAligned;
   bool pad = false;
-  bool dead_slot = false;  // some chain slot of a last position lies wholly past its row
+  int64_t dead_slots = 0;  // most chain slots of a last position that lie wholly past its row
   int64_t max_vectors = 1;
   int64_t max_per_lane = 1;
   int64_t rows = 0;
@@ -779,11 +793,13 @@ hipError_t launch_default(GemvBatch& batch, TreeShape shape, const PckRowSumBatc
   }
 }
 
-// Aligned rows in a tree of T != 256 lanes.  The shapes keep 8 to 16 vectors in flight per lane
-// (chains x R x U), fewer chains per lane leaving room for more rows or positions; the best of
-// R in {1, 2, 4}, U in {1 .. 4, 8} streamed from HBM, against R = 1, U = 2 with plain loads
-// (14336 x 4096 BF16: T = 64 / 128 / 512 19.6 / 19.9 / 20.0 against 23.5 / 22.4 / 21.8 us;
-// 4096 x 14336 FP8: T = 64 / 128 / 512 12.0 / 12.1 / 16.1 against 14.0 / 15.2 / 18.2 us).
+// Aligned rows in a tree of T != 256 lanes.  With non-temporal loads the shapes keep 8 to 16 vectors
+// in flight per lane (chains x R x U), fewer chains per lane leaving room for more rows or positions;
+// the best of R in {1, 2, 4}, U in {1 .. 4, 8} streamed from HBM.  Against R = 1, U = 2 with plain
+// loads, which is what smaller launches take: BF16 14336 x 4096 T = 64 / 128 / 512 20.0 / 19.6 / 19.5
+// against 23.2 / 21.9 / 21.5 us; FP8 14336 x 8192 23.0 / 23.0 / 23.0 against 24.9 / 24.7 / 32.2.
+// T = 32 holds two rows side by side in a wave already: one such pair for BF16 (8192 x 8192 25.5
+// against 30.6 us with two and 27.7 before).
 template <int T, bool kFp8, Pad kPad, bool kNt, bool kSums>
 hipError_t launch_other(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
   constexpr Load L = Load::kAligned;
@@ -801,7 +817,10 @@ hipError_t launch_other(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s
       // one row per wave for BF16 rows of at most 4096 columns and for few rows
       if ((!kFp8 && plan.max_vectors <= 512) || plan.rows < 4096)
         return launch_tree<T, 1, 4, kFp8, L, kPad, kNt, kSums>(b, rs, s);
-      return launch_tree<T, 2, T >= 128 ? 2 : 4, kFp8, L, kPad, kNt, kSums>(b, rs, s);
+      if constexpr (T == 32 && !kFp8)
+        return launch_tree<T, 1, 4, kFp8, L, kPad, kNt, kSums>(b, rs, s);
+      else
+        return launch_tree<T, 2, T >= 128 ? 2 : 4, kFp8, L, kPad, kNt, kSums>(b, rs, s);
     }
   }
 }
@@ -818,8 +837,8 @@ hipError_t launch_aligned(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t
 }
 
 // Rows read at any byte address.  Two rows per wave slot: the best shape of the same sweep for
-// nearly every T and length.  Against element loads, at T = 256: BF16 14336 x 4100 22.3 against
-// 122 us, 14337 x 4099 29.7 against 120; FP8 28672 x 4104 27.1 against 325 us, 28673 x 4099
+// nearly every T and length.  Against element loads, at T = 256: BF16 14336 x 4100 20.6 against
+// 118 us, 14337 x 4099 29.7 against 120; FP8 28672 x 4104 26.3 against 326 us, 28673 x 4099
 // (addresses of any byte) 51 against 326.
 template <int T, bool kFp8, bool kSums>
 hipError_t launch_unaligned(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s) {
@@ -842,8 +861,12 @@ hipError_t launch_live(GroupPlan& plan, const PckRowSumBatch* rs, hipStream_t s)
 
 // The route of a launch: element loads for rows shorter than a vector; else the fewest live
 // chain slots that hold the longest row (T = 1024, 14336 x 4096: BF16 8 slots of 16 20.3 against
-// 36.6 us with all and 62 before, FP8 4 slots 19.9 against 69.5 and 139 us); else all slots.
-// pck_gemv_set_shape picks the shape of aligned T = 256 launches, which then keep all slots.
+// 36.6 us with all and 62 before, FP8 4 slots 19.9 against 69.5 and 139 us); else all slots, dead
+// ones skipped where that pays for its branches: at T = 1024 for more than a quarter of the slots and
+// from 2048 rows on (BF16 11264 columns, ten dead slots: 4096 rows 21.5 against 24.7 us zeroed; 14336
+// columns, four: 512 rows 8.9 against 8.1), at T = 256 and 512 always (FP8 11264 columns at T = 512,
+// five: 512 rows 5.6 against 6.2 us, 8192 rows 22.4 against 25.4).  pck_gemv_set_shape picks the shape
+// of aligned T = 256 launches, which then keep all slots.
 template <int T, bool kFp8, bool kSums = false>
 hipError_t launch_for_threads(GroupPlan& plan, hipStream_t s, const PckRowSumBatch* rs = nullptr) {
   if (plan.load == Load::kElement)
@@ -861,8 +884,11 @@ hipError_t launch_for_threads(GroupPlan& plan, hipStream_t s, const PckRowSumBat
   }
   if (plan.load == Load::kUnaligned) return launch_unaligned<T, kFp8, kSums>(plan, rs, s);
   if (!plan.pad) return launch_aligned<T, kFp8, Pad::kNone, kSums>(plan, rs, s);
-  if constexpr (T >= 256) {
-    if (plan.dead_slot && !all) return launch_aligned<T, kFp8, Pad::kSkipped, kSums>(plan, rs, s);
+  if constexpr (T >= 1024) {
+    if (plan.dead_slots > 4 && plan.rows >= 2048)
+      return launch_aligned<T, kFp8, Pad::kSkipped, kSums>(plan, rs, s);
+  } else if constexpr (T >= 256) {
+    if (plan.dead_slots > 0 && !all) return launch_aligned<T, kFp8, Pad::kSkipped, kSums>(plan, rs, s);
   }
   return launch_aligned<T, kFp8, Pad::kZeroed, kSums>(plan, rs, s);
 }
@@ -892,7 +918,7 @@ hipError_t launch_ride_pad(GroupPlan& plan, const PckCheckBatch& ride, hipStream
 template <bool kFp8>
 hipError_t launch_ride(GroupPlan& plan, const PckCheckBatch& ride, hipStream_t stream) {
   if (!plan.pad) return launch_ride_pad<kFp8, Pad::kNone>(plan, ride, stream);
-  return plan.dead_slot ? launch_ride_pad<kFp8, Pad::kSkipped>(plan, ride, stream)
+  return plan.dead_slots > 0 ? launch_ride_pad<kFp8, Pad::kSkipped>(plan, ride, stream)
                         : launch_ride_pad<kFp8, Pad::kZeroed>(plan, ride, stream);
 }
 
@@ -933,8 +959,11 @@ hipError_t plan_group(const PckGemv* gemvs, double* const* sums, int count, int 
       plan.max_vectors = vectors > plan.max_vectors ? vectors : plan.max_vectors;
       plan.max_per_lane = per_lane > plan.max_per_lane ? per_lane : plan.max_per_lane;
       plan.pad = plan.pad || n % (static_cast<int64_t>(threads) * V) != 0;
-      plan.dead_slot =
-          plan.dead_slot || (threads > kWave && (vectors + kWave - 1) / kWave % (threads / kWave) != 0);
+      if (threads > kWave) {
+        const int64_t slots = threads / kWave;
+        const int64_t dead = (slots - (vectors + kWave - 1) / kWave % slots) % slots;
+        plan.dead_slots = dead > plan.dead_slots ? dead : plan.dead_slots;
+      }
     }
   }
   return hipSuccess;
