@@ -555,18 +555,27 @@ __global__ void __launch_bounds__(1024)
     }
   };
   if constexpr (kLoad == Load::kAligned) {
-    for (int64_t v = 0; v < chunk; v += 8) {
-      const int64_t col = first + v;
-      uint4 wv[R], xv = make_uint4(0, 0, 0, 0);  // past n: +0 products
+    constexpr int A = R == 2 ? 2 : 1;  // vectors loaded ahead: a whole chunk of two
+    for (int64_t v = 0; v < chunk; v += 8 * A) {
+      uint4 wv[A][R], xv[A];
 #pragma unroll
-      for (int r = 0; r < R; ++r) wv[r] = make_uint4(0, 0, 0, 0);
-      if (col < n) {
+      for (int a = 0; a < A; ++a) {
+        const int64_t col = first + v + 8 * a;
+        xv[a] = make_uint4(0, 0, 0, 0);  // past n: +0 products
 #pragma unroll
-        for (int r = 0; r < R; ++r) wv[r] = load16<false, false>(rows[r] + col);
-        xv = load16<false, false>(x + col);
+        for (int r = 0; r < R; ++r) wv[a][r] = make_uint4(0, 0, 0, 0);
+        if (col < n && (a == 0 || v + 8 < chunk)) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) wv[a][r] = load16<false, false>(rows[r] + col);
+          xv[a] = load16<false, false>(x + col);
+        }
       }
 #pragma unroll
-      for (int r = 0; r < R; ++r) add8(acc[r], wv[r], xv);
+      for (int a = 0; a < A; ++a) {
+        if (a == 1 && v + 8 >= chunk) break;  // uniform
+#pragma unroll
+        for (int r = 0; r < R; ++r) add8(acc[r], wv[a][r], xv[a]);
+      }
     }
   } else if constexpr (kLoad == Load::kUnaligned) {
     // columns col .. col + 7 of x and of the rows (+0 past n)
@@ -1074,12 +1083,13 @@ int pck_gemv_bf16_naive(const void* W, const void* x, float* y, int64_t m, int64
                        reinterpret_cast<uintptr_t>(x) % 16 == 0;
   const Load load = n < 8 || chunk < 4 ? Load::kElement : aligned ? Load::kAligned : Load::kUnaligned;
   // Rows per workgroup, from 8192 rows on (fewer leave too few workgroups).  Aligned chunks of one
-  // vector: four (14336 x 4096, T = 512: 22.4 against 25.1 us with one; 8192 x 2048, T = 256, from
-  // the caches: 5.5 / 6.3); of two: two, since four rows' loads push each other out of the L1 (14336 x
-  // 4096, T = 256, from HBM 26.1 / 26.8 with two, from the caches 20.1 with four, 19.0 with two, 18.7
-  // with one); longer ones: one (4096 x 14336: 84 us with four, 58 with one).  Ragged chunks: four
-  // (7182 x 8960, T = 256: 55 against 212 us with element loads), with fewer rows only where those are
-  // long enough to be bound by their loads (3000 x 512, T = 128: equal; 2048 x 512: 3.9 / 3.1).
+  // vector: four (14336 x 4096, T = 512: 22.4 against 25.3 us with one; 8192 x 2048, T = 256, from
+  // the caches: 5.5 / 6.3).  Of two: two, both vectors ahead (14336 x 4096, T = 256, from HBM 25.1
+  // us, one row 26.7, four 25.0; from the caches 18.6 / 18.8 / 19.3, as four rows' loads push each
+  // other out of the L1).  Longer ones: one (4096 x 14336: 84 us with four, 58 with one).  Ragged
+  // chunks: four (7182 x 8960, T = 256: 55 against 212 us with element loads), in fewer rows only
+  // where those are long enough to be bound by their loads (3000 x 512, T = 128: equal; 2048 x 512:
+  // 3.9 / 3.1).
   const bool many = load == Load::kUnaligned
                         ? m >= 8192 || (m >= 2048 && m * n >= 1500000)
                         : load == Load::kAligned && chunk <= 16 && m >= 8192 && threads >= 256;
