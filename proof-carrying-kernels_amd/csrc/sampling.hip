@@ -251,17 +251,20 @@ __device__ __forceinline__ float uniform_max(float v) {
 // 4-byte address), the next chunk's loads in flight while one is used: its extremes, then, for
 // top-p, its terms relative to the wave's largest logit so far (a wave's sums are rescaled in
 // FP64 when a chunk raises that).  Top-k is bound by the loads, top-p by the terms' arithmetic
-// (about 31 instructions a logit), so a wave without a selected logit in its chunk (nearly all)
+// (about 28 instructions a logit), so a wave without a selected logit in its chunk (nearly all)
 // skips what the selection needs.  The selection's entries are requested ahead of the logits and
 // every load is unconditional: loads return in order, and a branch around one makes all later
 // uses wait for everything in flight.  Both launches at 151,936 logits a row, against two passes
-// over memory with an FP64 division and an LDS read per logit: top-p 64 rows 25.7 against 33.8
-// us, 256 rows 66 against 110; top-k 50 256 rows 30.9 against 49.6 us (5.1 TB/s).
-constexpr int kQuads = 5;                      // 16-byte loads per lane and chunk
-constexpr int kChunk = kQuads * 4 * kThreads;  // logits per chunk
+// over memory with an FP64 division and an LDS read per logit: top-p 64 rows 22.1 against 33.3
+// us, 256 rows 49.4 against 108; top-k 50 256 rows 30.1 against 47.4 us (5.2 TB/s).
+//
+// kQuads: 16-byte loads per lane and chunk.  kOne: every segment is at most one chunk, so there is no
+// next one to request; launch_segments has the forms.
+constexpr int kLongQuads = 5;  // of segments of several chunks
 
-template <bool kLds>
+template <bool kLds, int kQuads, bool kOne>
 __global__ void __launch_bounds__(kThreads) segment_kernel(const Args a) {
+  constexpr int kChunk = kQuads * 4 * kThreads;  // logits per chunk
   extern __shared__ uint32_t lds_bits[];  // kLds: the segment's bitmap
   __shared__ float fred[3][kWaves];
   __shared__ double dred[2][kWaves];
@@ -299,9 +302,9 @@ __global__ void __launch_bounds__(kThreads) segment_kernel(const Args a) {
   int64_t first_sel[kAhead];
   if constexpr (kLds) request_selection(a.sel + row * a.max_len, a.max_len, first_sel);
   __builtin_amdgcn_sched_barrier(0);
-  f32x4 xa[kQuads], xb[kQuads];
+  f32x4 xa[kQuads], xb[kQuads];  // xb: the next chunk (not kOne)
   load(xa, 0);
-  load(xb, kChunk);
+  if constexpr (!kOne) load(xb, kChunk);
   if (no_quad) {  // at most three logits, in lane 0's first quad
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -392,11 +395,15 @@ __global__ void __launch_bounds__(kThreads) segment_kernel(const Args a) {
     else
       terms(std::false_type{});
   };
-  for (int64_t c0 = 0; c0 < count; c0 += 2 * kChunk) {
-    use(xa, c0);
-    load(xa, c0 + 2 * kChunk);
-    if (c0 + kChunk < count) use(xb, c0 + kChunk);
-    load(xb, c0 + 3 * kChunk);
+  if constexpr (kOne) {
+    if (count > 0) use(xa, 0);
+  } else {
+    for (int64_t c0 = 0; c0 < count; c0 += 2 * kChunk) {
+      use(xa, c0);
+      load(xa, c0 + 2 * kChunk);
+      if (c0 + kChunk < count) use(xb, c0 + kChunk);
+      load(xb, c0 + 3 * kChunk);
+    }
   }
   mn = -uniform_max(-mn);
   mx_rej = uniform_max(mx_rej);
@@ -487,6 +494,24 @@ __global__ void __launch_bounds__(kThreads) finish_kernel(const Args a, int lds_
   a.without[row] = without;
 }
 
+// The segment launch.  Segments of at most 4,096 logits (the default for rows that already fill the
+// GPU, or are short) are one chunk: without the next chunk's registers seven waves fit a SIMD instead
+// of three, so all of 1,024 workgroups run at once, and nothing is requested past the segment.
+// Against the form of several chunks, which has the shortest rows wait for ten loads a lane: top-k 50
+// of 128 x 32,000 logits 9.8 against 12.8 us, top-p 14.3 / 17.5; of 512 x 1,000 (one load a lane) top-p
+// 9.8 / 12.9.
+template <bool kLds>
+hipError_t launch_segments(const Args& a, size_t lds, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(a.segments), static_cast<unsigned>(a.rows));
+  if (a.seg_len <= 4 * kThreads)
+    segment_kernel<kLds, 1, true><<<grid, dim3(kThreads), lds, s>>>(a);
+  else if (a.seg_len <= 16 * kThreads)
+    segment_kernel<kLds, 4, true><<<grid, dim3(kThreads), lds, s>>>(a);
+  else
+    segment_kernel<kLds, kLongQuads, false><<<grid, dim3(kThreads), lds, s>>>(a);
+  return hipGetLastError();
+}
+
 }  // namespace
 }  // namespace pck
 
@@ -546,20 +571,17 @@ extern "C" int pck_sampling_check(const float* logits, const int64_t* selected,
   a.mass = mass;
   a.without = mass_without_smallest;
   auto s = static_cast<hipStream_t>(stream);
-  const dim3 seg_grid(static_cast<unsigned>(segments), static_cast<unsigned>(rows));
   hipError_t err;
   if (lds_select) {
-    const size_t lds = static_cast<size_t>((seg_len + 31) / 32) * sizeof(uint32_t);
-    segment_kernel<true><<<seg_grid, dim3(kThreads), lds, s>>>(a);
+    err = launch_segments<true>(a, static_cast<size_t>((seg_len + 31) / 32) * sizeof(uint32_t), s);
   } else {
     const dim3 mark_grid(static_cast<unsigned>((max_len + kThreads - 1) / kThreads),
                          static_cast<unsigned>(rows));
     mark_kernel<<<mark_grid, dim3(kThreads), 0, s>>>(a);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
-    segment_kernel<false><<<seg_grid, dim3(kThreads), 0, s>>>(a);
+    err = launch_segments<false>(a, 0, s);
   }
-  err = hipGetLastError();
   if (err != hipSuccess) return err;
   finish_kernel<<<dim3(static_cast<unsigned>((rows + kWaves - 1) / kWaves)), dim3(kThreads), 0,
                   s>>>(a, lds_select ? 1 : 0);

@@ -235,11 +235,11 @@ def test_native_entry_takes_the_pybind_sampling_arguments() -> None:
     assert torch.equal(out[2], ref.max_rejected)
 
 
-@pytest.mark.parametrize("vocab", [2, 4, 5, 5119, 5121, 10_243, 25_601])
+@pytest.mark.parametrize("vocab", [2, 4, 5, 1024, 1025, 4096, 4097, 5119, 5121, 10_243, 25_601])
 @pytest.mark.parametrize("segments", [1, 2, 3])
 @pytest.mark.parametrize("temp", [1.0, 0.7, 1e-42, 1e30])
 def test_chunks_of_a_segment_match_cpu(vocab: int, segments: int, temp: float) -> None:
-    """Segments around the 5,120 logits of one chunk, with a partial last quad, one to five
+    """Segments around the 1,024 and 4,096 logits of a single chunk and the 5,120 of one of several, with a partial last quad, one to five
     chunks, rows at any 4-byte address, maxima that rise from chunk to chunk, and temperatures
     of each way the quotient is formed (T = 1, two floats, FP64)."""
     segments = min(segments, vocab)
