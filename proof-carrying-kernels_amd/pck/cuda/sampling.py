@@ -114,6 +114,10 @@ def check_topk_gpu(
 
 
 @functools.lru_cache(maxsize=256)
+def _own_rounding(vocab: int, segments: int) -> float:
+    return 16 * U32 + math.ldexp(vocab, -146) + gamma(vocab + 3 * segments + 16, U64)
+
+
 def topp_slack(vocab: int, segments: int, tol: float) -> float:
     """The sampler's ``tol`` plus this checker's own rounding (reference
     `cuda/sampling.py:71-88`): each term is an FP32 2^(hi + lo) within 0.8 ulp (6 u32 relative taken)
@@ -121,8 +125,7 @@ def topp_slack(vocab: int, segments: int, tol: float) -> float:
     roundings (at most V / 256 + 32 additions, V / 5120 + 1 rescalings to its wave's and segment's
     maximum and one per segment to the row's, of three roundings each); the largest term is exactly
     1.  Each mass is then within 16 u32 + V 2^-146 + gamma_{V + 3S + 16}(u64), rounded up."""
-    own = 16 * U32 + math.ldexp(vocab, -146) + gamma(vocab + 3 * segments + 16, U64)
-    return math.nextafter(tol + own, math.inf)
+    return math.nextafter(tol + _own_rounding(int(vocab), int(segments)), math.inf)
 
 
 def check_topp_gpu(

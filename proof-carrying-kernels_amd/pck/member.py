@@ -79,13 +79,17 @@ def check_member(
     return MemberVerdict(bool(r < next_up(top_p + slack)), above, r)
 
 
-@functools.lru_cache(maxsize=256)
 def member_eps32(vocab: int) -> float:
     """Error bound of r for FP32 split-argument terms summed in FP64 (reference
     `src/pck/member.py:84-102`): each term within 6 u32 relative plus 2^-124 absolute (a
     2-ulp ``expf``, two roundings, terms below e^-128 dropped), both sums within
     gamma_{V+2}(u64), so E = 6 u32 + V 2^-124 + gamma_{V+2}(u64) (1 + 6 u32 + V 2^-124) and
     the quotient is within 2E / (1 - E) + u64."""
+    return _eps32(int(vocab))
+
+
+@functools.lru_cache(maxsize=256)
+def _eps32(vocab: int) -> float:
     tiny = math.ldexp(vocab, -124)
     e = 6 * U32 + tiny + gamma(vocab + 2, U64) * (1 + 6 * U32 + tiny)
     return 2 * e / (1 - e) + U64

@@ -160,3 +160,21 @@ def test_check_member_equals_the_oracle() -> None:
         got = pmember.check_member(row, token, top_k, top_p, greedy=greedy, tol=1e-4)
         want = omember.check_member(row, token, top_k, top_p, greedy=greedy, tol=1e-4)
         assert (got.ok, got.above) == (want.ok, want.above) and same(got.mass_above, want.mass_above)
+
+
+def test_error_bounds_follow_the_values_of_their_arguments() -> None:
+    """The bounds remember host arithmetic by value only: a tolerance or a size in a tensor or array
+    that changes in place gives the bound of what it holds now, and unhashable numbers are taken."""
+    import torch
+
+    from pck.cuda.sampling import topp_slack
+
+    tol = torch.tensor(1e-6, dtype=torch.float64)
+    vocab = torch.tensor(1000)
+    first = topp_slack(1000, 4, tol), pmember.member_eps32(vocab)
+    assert first == (topp_slack(1000, 4, 1e-6), pmember.member_eps32(1000))
+    tol.fill_(1e-2)
+    vocab.fill_(151936)
+    assert topp_slack(1000, 4, tol) == topp_slack(1000, 4, 1e-2) > first[0]
+    assert pmember.member_eps32(vocab) == pmember.member_eps32(151936) > first[1]
+    assert topp_slack(1000, 4, np.array(1e-6)) == first[0]
