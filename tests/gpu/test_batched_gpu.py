@@ -351,9 +351,11 @@ def test_activation_pack_layout_aligned_and_8_byte_aligned(rows: int, n: int) ->
 
 # (m, n, B): one chunk (seven empty segments), a partial chunk, segments of an odd number of
 # chunks (n = 60, 320, 1001, 3000), of 15 and 17 chunks (n = 960, 1088: the half pair ends a group
-# or begins one), rows past m, m % 4 != 0, several batch passes and workgroups looping over items.
+# or begins one), rows past m, m % 4 != 0, several batch passes and workgroups looping over items;
+# three row tiles an item with a partial last one (130 tiles, 128 rows of X), two batch tiles an item.
 ANY_SHAPES = [(5, 7, 3), (1, 8, 1), (33, 128, 20), (32, 60, 20), (34, 320, 40), (64, 960, 33),
-              (64, 1088, 33), (101, 1001, 70), (36, 3000, 24), (66, 4100, 300), (19203, 520, 128)]  # fmt: skip
+              (64, 1088, 33), (101, 1001, 70), (36, 3000, 24), (66, 4100, 300), (19203, 520, 128), (4131, 520, 128),
+              (101, 1001, 128)]  # fmt: skip
 
 
 @pytest.mark.parametrize(("m", "n", "B"), ANY_SHAPES, ids=str)

@@ -111,16 +111,18 @@ def test_batched_layer_graph_replays_match_eager() -> None:
             assert torch.equal(a.rho, b.rho) and torch.equal(a.tau, b.tau), replay
 
 
-def test_membership_graph_replays_match_eager() -> None:
+@pytest.mark.parametrize("most", [200, 60])
+def test_membership_graph_replays_match_eager(most: int) -> None:
     """The membership check under capture (B = 64, V = 151936, top-k and top-p rows, greedy
     rows, one planted out-of-set token), given the host copy of top-k as vLLM passes it: every
-    replay equals the eager run, with eager work between replays."""
+    replay equals the eager run, with eager work between replays.  Top-k below 200: one workgroup per
+    row; below 60: rows split over workgroups, with a workspace from the capture's pool."""
     from pck.member import check_members
 
     gen = torch.Generator().manual_seed(13)
     B, V = 64, 151936
     logits = (torch.randn(B, V, generator=gen) * 3).cuda()
-    top_k = torch.randint(1, 200, (B,), generator=gen).cuda()
+    top_k = torch.randint(1, most, (B,), generator=gen).cuda()
     top_p = (torch.rand(B, generator=gen) * 0.5 + 0.5).cuda()
     greedy = torch.zeros(B, dtype=torch.bool)
     greedy[::9] = True

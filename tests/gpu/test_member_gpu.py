@@ -350,3 +350,38 @@ def test_candidates_of_ordinary_rows_fit_their_slots(case: str, tail: int, dtype
     slots = (need.value - 48 * segments) // (4 * segments)
     counts = work[: 48 * segments].view(torch.int32).view(segments, 12)[:, 4]
     assert int(counts.max()) <= slots, (slots, counts.tolist())
+
+
+# (vocab, first hot id, top-k): the finish launch reads the first slots of 20 segments of 8,192 logits
+# ahead and walks the others, and holds the headers of 256 in registers; ties at the k-th logit.
+MANY_SEGMENTS = [(163_841, 163_840, [1, 50, 100, 7]), (262_144, 20 * 8192, [1, 50, 80, 7]),
+                 (2_100_000, 256 * 8192, [1, 9, 5, 9])]  # fmt: skip
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize(("vocab", "hot", "ks"), MANY_SEGMENTS, ids=str)
+def test_rows_of_many_segments_match_the_oracle(vocab: int, hot: int, ks: list[int], dtype: torch.dtype) -> None:
+    """The largest logits, the k-th among them with its ties, lie in segments past those held ahead
+    (row 3: before them); top-p with top-k, and top-p alone."""
+    rng = np.random.default_rng(vocab)
+    logits = np.clip(rng.standard_normal((4, vocab)) * 2, -9, 7)
+    for r, k in enumerate(ks):
+        start, end = (0, hot) if r == 3 else (hot, vocab)
+        at = rng.permutation(end - start)[: 2 * k] + start
+        logits[r, at] = 8 + np.arange(at.size)[::-1] / 16  # descending: at[k - 1] is the k-th
+        if at.size > k > 1:
+            logits[r, at[k:]] = logits[r, at[k - 1]]
+    t = torch.from_numpy(logits).to(dtype)
+    host = t.float().numpy()
+    order = np.argsort(-host, axis=1, kind="stable")
+    top_k = np.array(ks)
+    tokens = order[np.arange(4), [0, 1, top_k[2] - 1, 3]]
+    top_p = np.array([0.9, 0.9, 1 - 1e-9, 0.5])
+    for k in (top_k, None):
+        dev = None if k is None else torch.from_numpy(k).cuda()
+        out = check_members(t.cuda(), torch.from_numpy(tokens).cuda(), dev, torch.from_numpy(top_p).cuda(), top_k_host=k)
+        want = check_members_ref(host, tokens, k, top_p, None, top_k_host=k)
+        np.testing.assert_array_equal(out["ok"].cpu().numpy(), want["ok"])
+        np.testing.assert_array_equal(out["above"].cpu().numpy(), want["above"])
+        err = np.abs(out["mass_above"].cpu().numpy() - want["mass_above"])
+        assert np.all(err <= 2 * member_eps32(vocab))
