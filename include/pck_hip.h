@@ -145,7 +145,8 @@ int pck_bgemm_packed_any(int weight_kind, const void* Wp, const void* Xp, float*
 
 /* Both launches of a batched product from row-major X in one call: packs X (batch, n) into the
  * caller's Xp (as pck_bgemm_pack's dst, or pck_bgemm_pack_any's), then the product.  Wp is packed
- * by pck_bgemm_pack when n % 128 == 0 and m % 4 == 0, else by pck_bgemm_pack_any. */
+ * by pck_bgemm_pack when n % 128 == 0 and m % 4 == 0 (X then at an 8-byte, Y at a 16-byte address),
+ * else by pck_bgemm_pack_any. */
 int pck_bgemm_product(int weight_kind, const void* Wp, const void* X, void* Xp, float* Y, int64_t m,
                       int64_t n, int64_t batch, void* stream);
 

@@ -804,8 +804,7 @@ struct FinishScratch : Scratch {
 };
 
 // 256 lanes: the exchanges between waves are short chains of LDS reads, and a row of 152 K logits
-// has 19 segments, one round of early slots.  Against 1024 lanes and a radix select for every
-// row: see the figures at split_plan.
+// has 19 segments, one round of early slots (64 rows with a top-k and a top-p: 5.8 us).
 template <Logits kType>
 __global__ void __launch_bounds__(kFinishThreads) member_finish_kernel(const SplitArgs S) {
   using L = LogitType<kType>;
