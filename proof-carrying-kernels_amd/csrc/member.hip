@@ -210,7 +210,9 @@ __device__ __forceinline__ void for_each4(const float* __restrict__ row, int64_t
     const f32x4* quads = reinterpret_cast<const f32x4*>(row);
     const int64_t q1 = end / 4;
     int64_t q = begin / 4 + t;
-    const bool first = q + 3 * kThreads < q1;
+    // four quads ahead where the wave's last lane has them all, so a wave's lanes go the same way
+    const int64_t ahead = 3 * kThreads + (kWave - 1 - lane_id());
+    const bool first = q + ahead < q1;
     f32x4 a, b, c, d;
     if (first) {
       a = load_quad<kNt>(quads + q);
@@ -223,7 +225,7 @@ __device__ __forceinline__ void for_each4(const float* __restrict__ row, int64_t
       f4(a), f4(b), f4(c), f4(d);
       q += 4 * kThreads;
     }
-    for (; q + 3 * kThreads < q1; q += 4 * kThreads) {
+    for (; q + ahead < q1; q += 4 * kThreads) {
       a = load_quad<kNt>(quads + q);
       b = load_quad<kNt>(quads + q + kThreads);
       c = load_quad<kNt>(quads + q + 2 * kThreads);
@@ -464,9 +466,9 @@ __global__ void __launch_bounds__(kThreads) member_kernel(const MemberArgs A) {
   };
   // Compacts every logit >= low into the wave's LDS segment.  The wave's count follows the
   // ballots, so no atomic is needed.  Lanes may diverge at the end of a range: the lanes that
-  // run a step are then always a prefix of the wave from its lane 0 (a lane's trip count never
-  // exceeds that of a lower lane), so lane 0 runs every step and holds the wave's count, and
-  // each step takes the count from the first active lane.
+  // run a step are then always a prefix of the wave from its lane 0 (for_each4 unrolls by whole
+  // waves, and a lane's trip count never exceeds that of a lower lane), so lane 0 runs every step
+  // and holds the wave's count, and each step takes the count from the first active lane.
   float* const seg = s.cand + wave_id() * kSeg;
   int wcount = 0;
   auto compact = [&](float l) {

@@ -385,3 +385,28 @@ def test_rows_of_many_segments_match_the_oracle(vocab: int, hot: int, ks: list[i
         np.testing.assert_array_equal(out["above"].cpu().numpy(), want["above"])
         err = np.abs(out["mass_above"].cpu().numpy() - want["mass_above"])
         assert np.all(err <= 2 * member_eps32(vocab))
+
+
+@pytest.mark.parametrize("vocab", [12_548, 14_532, 16_320, 31_004, 47_408, 64_900])
+@pytest.mark.parametrize("k", [5, 60, 200])
+def test_candidates_at_the_end_of_the_unrolled_loads_are_all_kept(vocab: int, k: int) -> None:
+    """FP32 rows whose last unrolled step of four 16-byte loads ends inside a wave: the lanes past that
+    point take their last loads one at a time.  The kept logits lie in that wave's last loads, on both
+    sides of the point, so one lost or written over changes the k-th logit, the masses or the verdict."""
+    base = 0 if vocab < 16_384 else 4096  # quads before the streamed part
+    n = vocab // 4 - base
+    edge = n % 4096 - 3072  # the first lane whose last unrolled step is not whole
+    assert 0 < edge < 1024 and edge % 64 != 0
+    t = np.arange(edge // 64 * 64, edge // 64 * 64 + 64)
+    quads = (base + n // 4096 * 4096 + t[:, None] + 1024 * np.arange(4)).reshape(-1)
+    places = (4 * quads[quads < vocab // 4][:, None] + np.arange(4)).reshape(-1)
+    rng = np.random.default_rng(vocab + k)
+    rows = 170  # one workgroup per row at every vocabulary here
+    logits = np.clip(rng.standard_normal((rows, vocab)) * 2, -9, 7).astype(np.float32)
+    for r in range(rows):
+        at = rng.permutation(places)[: k + 20]
+        logits[r, at] = 8 + np.arange(at.size, dtype=np.float32)[::-1] / 64
+    order = np.argsort(-logits, axis=1, kind="stable")
+    tokens = order[np.arange(rows), rng.integers(0, k, rows)]
+    top_k, top_p = np.full(rows, k), np.full(rows, 0.7)
+    assert_matches_oracle(logits, tokens, top_k, top_p, top_k_host=top_k)
