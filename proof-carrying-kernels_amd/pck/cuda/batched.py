@@ -17,6 +17,7 @@ Two routes with the same bits:
 
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass
 
@@ -57,7 +58,7 @@ class BatchedWeights:
 
     @property
     def device(self) -> torch.device:
-        t = next((t for t in (self.packed, self.padded) if t is not None), self.raw)
+        t = self.packed if self.packed is not None else self.padded if self.padded is not None else self.raw
         assert t is not None
         return t.device
 
@@ -84,7 +85,7 @@ def _pack(src: torch.Tensor, kind: int) -> torch.Tensor:
 
 def _pack_any(src: torch.Tensor, kind: int) -> torch.Tensor:
     rows, n = src.shape
-    columns = lib().pck_bgemm_any_columns(n)
+    columns = _any_columns(n)
     elem = torch.uint8 if kind == 1 else torch.bfloat16
     dst = torch.empty((rows + TILE - 1) // TILE * TILE * columns, dtype=elem, device=src.device)
     with on_device(src.device):
@@ -92,6 +93,12 @@ def _pack_any(src: torch.Tensor, kind: int) -> torch.Tensor:
                                        stream_handle(src.device))  # fmt: skip
     check(err, "batched pack launch")
     return dst
+
+
+@functools.lru_cache(maxsize=256)
+def _any_columns(n: int) -> int:
+    """Columns of a padded tile row for rows of n, -1 where the tiles do not take them."""
+    return int(lib().pck_bgemm_any_columns(n))
 
 
 def _element_is_faster(kind: int, m: int, n: int, B: int, vectors: bool = True) -> bool:
@@ -127,7 +134,7 @@ def pack_batched_weights(W: torch.Tensor) -> BatchedWeights:
     tiles take (n % 128 != 0 or m % 4 != 0, `pck_bgemm_any_columns`), which keep W as it is."""
     _validate_w(W)
     m, n = W.shape
-    if m == 0 or n == 0 or not _packable(m, n) and lib().pck_bgemm_any_columns(n) < 0:
+    if m == 0 or n == 0 or not _packable(m, n) and _any_columns(n) < 0:
         return BatchedWeights(m, n, W.dtype, None, W)
     if not _packable(m, n):
         raw = W.detach().clone() if _element_is_faster(_kind(W.dtype), m, n, 1) else None
@@ -180,7 +187,7 @@ def gemm_batched(
         tiles = None
     with on_device(device):
         if tiles is not None:
-            columns = n if W.packed is not None else lib().pck_bgemm_any_columns(n)
+            columns = n if W.packed is not None else _any_columns(n)
             Xp = torch.empty((B + TILE - 1) // TILE * TILE * columns, dtype=X.dtype, device=device)
             err = lib().pck_bgemm_product(kind, tiles.data_ptr(), X.data_ptr(), Xp.data_ptr(),
                                           Y.data_ptr(), m, n, B, stream_handle(device))  # fmt: skip
